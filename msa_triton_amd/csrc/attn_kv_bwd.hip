@@ -358,66 +358,57 @@ __device__ __forceinline__ float4 main_row_record(double lse2, double mass, doub
                      static_cast<float>(w));
 }
 
-// mass = sum_s A_s, delta = sum_s B_s / mass over the row's valid slots (FP64);
-// 32 lanes per (token, head), slots lane-parallel then a fixed shuffle tree. Rows
-// outside the pass (flat rows, unless all_rows) keep the forward's mass. The mass
-// keeps the sign of the forward's mark, so a repeated backward selects the same rows.
-// Every row of the chunk then gets the main pass's fp32 record in rowf. A 32-lane
-// segment owns rps consecutive rows (32 when only the forward's peaked rows take the
-// pass, 1 when all do): each lane settles its own row if it is outside the pass, then
-// the segment takes its rows in the pass one after the other.
+// mass = sum_s A_s, delta = sum_s B_s / mass over the row's valid slots (FP64, slot
+// order), one lane per (token, head): a row's records are contiguous, so the slots' loads
+// of a wave walk whole cache lines. Rows outside the pass (flat rows, unless all_rows) keep
+// the forward's mass. The mass keeps the sign of the forward's mark, so a repeated backward
+// selects the same rows. Every row of the chunk then gets the main pass's fp32 record in
+// rowf. (32 lanes per row, a segment's peaked rows one after the other, took 41 us for the
+// 10 240 rows of two sequences of 512 and 768 tokens and 8 heads, where most rows are
+// peaked: a serial chain of loads per row.)
 __global__ __launch_bounds__(256) void kv_bwd_stats_combine(const int32_t* __restrict__ indices,
                                                             const int32_t* __restrict__ cu, int nseq, int64_t t0,
                                                             int64_t t1, int Hq, int G, int K, int B, int all_rows,
-                                                            int rps, const float2* __restrict__ spart,
+                                                            const float2* __restrict__ spart,
                                                             double* __restrict__ row_state,
                                                             float4* __restrict__ rowf) {
-  const int sub = threadIdx.x & 31;
-  const int64_t base = t0 * Hq + (static_cast<int64_t>(blockIdx.x) * 8 + (threadIdx.x >> 5)) * rps;
-  const int64_t end = t1 * Hq;
-  bool in_pass = false;
-  if (sub < rps && base + sub < end) {
-    const int64_t th = base + sub;
-    const double4 rs = *reinterpret_cast<const double4*>(row_state + th * 4);
-    in_pass = all_rows || !(rs.y > 0.0);
-    if (!in_pass) rowf[th] = main_row_record(rs.x, rs.y, rs.z, rs.w);
-  }
-  // this segment's rows in the pass (bits of its half of the wave)
-  uint32_t todo = static_cast<uint32_t>(__ballot(in_pass) >> (threadIdx.x & 32));
-  while (todo) {
-    const int j = __builtin_ctz(todo);
-    todo &= todo - 1;
-    const int64_t th = base + j;
-    const double mark = row_state[th * 4 + 1];
-    const int64_t t = th / Hq;
-    const int h = static_cast<int>(th % Hq);
-    const int g = h / (Hq / G);
-    const int s = find_seq(cu, nseq, t);
-    const int64_t qb = (t - cu[s]) / B;
-    const int32_t* sel = indices + (t * G + g) * K;
-    const int64_t rec0 = ((t - t0) * Hq + h) * static_cast<int64_t>(K);
+  constexpr int kBatch = 8;
+  const uint32_t lr = blockIdx.x * 256 + threadIdx.x;  // chunk-local row
+  if (lr >= static_cast<uint32_t>(t1 - t0) * Hq) return;
+  const int64_t th = t0 * Hq + lr;
+  double4 rs = *reinterpret_cast<const double4*>(row_state + th * 4);
+  if (all_rows || !(rs.y > 0.0)) {
+    const int32_t tl = lr / static_cast<uint32_t>(Hq), t = static_cast<int32_t>(t0) + tl;
+    const int g = static_cast<int>(lr - tl * Hq) / (Hq / G);
+    const int32_t qb = (t - cu[find_seq_near(cu, nseq, t)]) / B;
+    const int32_t* sel = indices + (static_cast<int64_t>(t) * G + g) * K;
+    const float2* rec = spart + static_cast<int64_t>(lr) * K;
     double a = 0.0, b = 0.0;
-    for (int slot = sub; slot < K; slot += 32) {
-      const int id = sel[slot];
-      if (id >= 0 && id <= qb) {
-        const float2 ab = spart[rec0 + slot];
-        a += static_cast<double>(ab.x);
-        b += static_cast<double>(ab.y);
+    for (int s0 = 0; s0 < K; s0 += kBatch) {
+      bool ok[kBatch];
+      float2 ab[kBatch];
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) {
+        const int slot = s0 + u < K ? s0 + u : K - 1;
+        const int id = sel[slot];
+        ok[u] = s0 + u < K && id >= 0 && id <= qb;
+        ab[u] = rec[slot];  // in bounds for every slot, used only where valid
+      }
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) {
+        if (ok[u]) {
+          a += static_cast<double>(ab[u].x);
+          b += static_cast<double>(ab[u].y);
+        }
       }
     }
-#pragma unroll
-    for (int o = 16; o > 0; o >>= 1) {
-      a += __shfl_xor(a, o, 32);
-      b += __shfl_xor(b, o, 32);
-    }
-    if (sub == 0) {
-      const bool has = a > 0.0;
-      const double mass = copysign(has ? a : 1.0, mark), delta = has ? b / a : 0.0;
-      row_state[th * 4 + 1] = mass;
-      row_state[th * 4 + 3] = delta;
-      rowf[th] = main_row_record(row_state[th * 4], mass, row_state[th * 4 + 2], delta);
-    }
+    const bool has = a > 0.0;
+    rs.y = copysign(has ? a : 1.0, rs.y);
+    rs.w = has ? b / a : 0.0;
+    row_state[th * 4 + 1] = rs.y;
+    row_state[th * 4 + 3] = rs.w;
   }
+  rowf[th] = main_row_record(rs.x, rs.y, rs.z, rs.w);
 }
 
 // One workgroup (8 waves) per work item: a key block row and <= kMainEdges of its
@@ -930,43 +921,58 @@ __global__ __launch_bounds__(32 * kDqCombineRows) void kv_bwd_dq_combine(const i
                                                          uint16_t* __restrict__ dq) {
   constexpr int kBatch = 8;
   const int sub = threadIdx.x & 31;
-  const int64_t th = t0 * Hq + static_cast<int64_t>(blockIdx.x) * kDqCombineRows + (threadIdx.x >> 5);
-  if (th >= t1 * Hq) return;
-  const int64_t t = th / Hq;
-  const int h = static_cast<int>(th % Hq);
-  const int g = h / (Hq / G);
-  const int s = find_seq(cu, nseq, t);
-  const int64_t qb = (t - cu[s]) / B;
-  const int32_t* sel = indices + (t * G + g) * K;
-  const int64_t rec0 = ((t - t0) * Hq + h) * static_cast<int64_t>(K);
+  const uint32_t lr = blockIdx.x * kDqCombineRows + (threadIdx.x >> 5);  // chunk-local row
+  if (lr >= static_cast<uint32_t>(t1 - t0) * Hq) return;
+  const int32_t tl = lr / static_cast<uint32_t>(Hq), t = static_cast<int32_t>(t0) + tl;
+  const int64_t th = t0 * Hq + lr;
+  const int g = static_cast<int>(lr - tl * Hq) / (Hq / G);
+  const int32_t qb = (t - cu[find_seq_near(cu, nseq, t)]) / B;
+  const int32_t* sel = indices + (static_cast<int64_t>(t) * G + g) * K;
+  const int64_t rec0 = static_cast<int64_t>(lr) * K;
+  // Only the slots that one of the wave's two rows has are read (see attn_fwd_combine).
+  double acc[DC][4];
+  int dcol[DC];
 #pragma unroll
-  for (int hc = 0; hc < DC; ++hc) {  // 128-dim halves of the row (4 dims per lane in each)
-  const int dc = 128 * hc + 4 * sub;
-  if (dc >= D) return;
-  double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
-  for (int s0 = 0; s0 < K; s0 += kBatch) {
-    float4 x[kBatch];
-    bool ok[kBatch];
+  for (int hc = 0; hc < DC; ++hc) {
+    acc[hc][0] = acc[hc][1] = acc[hc][2] = acc[hc][3] = 0.0;
+    dcol[hc] = 128 * hc + 4 * sub < D ? 128 * hc + 4 * sub : 0;  // lanes without dims read (and ignore) dims 0..3
+  }
+  const int half = threadIdx.x & 32;
+  for (int s0 = 0; s0 < K; s0 += 32) {
+    const int id = s0 + sub < K ? sel[s0 + sub] : -1;
+    const uint64_t bal = __ballot(id >= 0 && id <= qb);
+    const uint32_t own = static_cast<uint32_t>(bal >> half);  // this row's slots
+    uint32_t slots = static_cast<uint32_t>(bal) | static_cast<uint32_t>(bal >> 32);
+    while (slots) {
+      int j[kBatch];
+      f32x4 x[kBatch][DC];
 #pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      const int slot = s0 + u < K ? s0 + u : K - 1;
-      const int id = sel[slot];
-      ok[u] = s0 + u < K && id >= 0 && id <= qb;
-      const f32x4 y = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(dqpart + (rec0 + slot) * D + dc));
-      x[u] = make_float4(y[0], y[1], y[2], y[3]);
-    }
+      for (int u = 0; u < kBatch; ++u) {
+        j[u] = slots ? __builtin_ctz(slots) : -1;  // past the last slot: no load
+        slots &= slots - 1;
+        if (j[u] >= 0) {
 #pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      if (ok[u]) {
-        a0 += static_cast<double>(x[u].x);
-        a1 += static_cast<double>(x[u].y);
-        a2 += static_cast<double>(x[u].z);
-        a3 += static_cast<double>(x[u].w);
+          for (int hc = 0; hc < DC; ++hc)
+            x[u][hc] = __builtin_nontemporal_load(
+                reinterpret_cast<const f32x4*>(dqpart + (rec0 + s0 + j[u]) * D + dcol[hc]));
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) {
+        if (j[u] >= 0 && ((own >> j[u]) & 1)) {
+#pragma unroll
+          for (int hc = 0; hc < DC; ++hc)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[hc][i] += static_cast<double>(x[u][hc][i]);
+        }
       }
     }
   }
-  *reinterpret_cast<uint2*>(dq + th * D + dc) = pack4_from_f64<DT>(a0 * scale, a1 * scale, a2 * scale, a3 * scale);
-  }
+#pragma unroll
+  for (int hc = 0; hc < DC; ++hc)
+    if (128 * hc + 4 * sub < D)
+      *reinterpret_cast<uint2*>(dq + th * D + dcol[hc]) =
+          pack4_from_f64<DT>(acc[hc][0] * scale, acc[hc][1] * scale, acc[hc][2] * scale, acc[hc][3] * scale);
 }
 
 static int nk_of_dim(int D) { return D <= 32 ? 1 : (D <= 64 ? 2 : (D <= 128 ? 4 : 8)); }
@@ -1077,9 +1083,8 @@ int attn_bwd_kv(int dt, const void* q, const void* k, const void* v, const void*
     }
     {
       ProfScope ps(kProfBwdStatsCombine, st);
-      const int rps = all_rows ? 1 : 32;  // rows per 32-lane segment
-      hipLaunchKernelGGL(kv_bwd_stats_combine, dim3(grid_1d((t1 - t0) * Hq, 8 * rps)), dim3(256), 0, st, indices, cu,
-                         nseq, t0, t1, Hq, G, K, B, all_rows, rps, spart, rs, rowf);
+      hipLaunchKernelGGL(kv_bwd_stats_combine, dim3(grid_1d((t1 - t0) * Hq, 256)), dim3(256), 0, st, indices, cu,
+                         nseq, t0, t1, Hq, G, K, B, all_rows, spart, rs, rowf);
     }
     if (rows > 0) {
       const int32_t* hi = kv_plan_hi(mp, mbase, c);

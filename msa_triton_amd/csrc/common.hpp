@@ -105,6 +105,15 @@ __device__ __forceinline__ int find_seq(const int32_t* __restrict__ cu, int nseq
   return lo;
 }
 
+// find_seq for the lanes of a wave whose tokens are close together: the search runs once,
+// for the first active lane's token (scalar loads), and the other lanes step on from there
+// (tokens must not decrease with the lane).
+__device__ __forceinline__ int find_seq_near(const int32_t* __restrict__ cu, int nseq, int32_t t) {
+  int s = find_seq(cu, nseq, __builtin_amdgcn_readfirstlane(t));
+  while (s + 1 < nseq && cu[s + 1] <= t) ++s;
+  return s;
+}
+
 // Largest index i in [0, n) with a[i] <= x, for nondecreasing a with a[0] <= x.
 __device__ __forceinline__ int upper_index(const int32_t* __restrict__ a, int n, int64_t x) {
   int lo = 0, hi = n;

@@ -45,16 +45,18 @@ def _sub_block_view(q, k, indices, meta, block_size, seqs):
     return _k2q.sub_block_selection(indices, meta, block_size, seqs, fits)
 
 
-def _attn_forward(q, k, v, indices, cu, meta, block_size, scale, seqs, public_csr=False, save_f32=False):
-    """Forward launch on contiguous inputs: (out, lse, row_state, out_f32 or None,
+def _attn_forward(q, k, v, indices, cu, meta, block_size, scale, seqs, public_csr=False, save_f32=False,
+                  save_state=True):
+    """Forward launch on contiguous inputs: (out, lse, row_state or None, out_f32 or None,
     csr or None). With ``public_csr`` the KV-major path builds its CSR through the
-    public builder; with ``save_f32`` it also returns the fp32 output for the backward."""
+    public builder; with ``save_f32`` it also returns the fp32 output for the backward,
+    without ``save_state`` it leaves out the backward's row state."""
     total, heads, dim = q.shape
     groups = k.shape[1]
     out = torch.empty_like(q)
     lse = torch.empty((total, heads), device=q.device, dtype=torch.float32)
     # Private fp64 per-row state shared by forward and backward: lse, mass, center, delta.
-    row_state = torch.empty((total, heads, 4), device=q.device, dtype=torch.float64)
+    row_state = torch.empty((total, heads, 4), device=q.device, dtype=torch.float64) if save_state else None
     out_f32 = torch.empty((total, heads, dim), device=q.device, dtype=torch.float32) if save_f32 else None
     csr = None
     if total:
@@ -80,7 +82,7 @@ def _attn_forward(q, k, v, indices, cu, meta, block_size, scale, seqs, public_cs
                 _lib.ptr(None if csr is None else csr.row_ptr),
                 _lib.ptr(None if csr is None else csr.query_indices),
                 _lib.ptr(None if csr is None else csr.slot_indices), _lib.ptr(workspace), ws_bytes,
-                out.data_ptr(), lse.data_ptr(), row_state.data_ptr(), _lib.ptr(out_f32), _lib.stream_of(q.device),
+                out.data_ptr(), lse.data_ptr(), _lib.ptr(row_state), _lib.ptr(out_f32), _lib.stream_of(q.device),
             )
         _lib.check(status, "msa_attn_fwd")
     return out, lse, row_state, out_f32, csr
@@ -146,7 +148,8 @@ class _SparseAttention(torch.autograd.Function):
         need_kv = ctx.needs_input_grad[1] or ctx.needs_input_grad[2]
         need_any = need_kv or ctx.needs_input_grad[0]
         out, lse, row_state, out_f32, csr = _attn_forward(q, k, v, indices, cu, meta, block_size, scale, seqs,
-                                                          public_csr=need_kv, save_f32=need_any)
+                                                          public_csr=need_kv, save_f32=need_any,
+                                                          save_state=need_any)
         ctx.save_for_backward(q, k, v, indices, cu, out, row_state, out_f32)
         ctx.csr = csr
         ctx.meta = meta
