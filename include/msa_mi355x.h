@@ -80,7 +80,7 @@ int msa_k2q_build_noalloc(const int32_t* indices, const int32_t* cu_seqlens, con
                           int32_t* slot_indices, void* stream);
 
 /* Stage 1 forward workspace in bytes: the squared norm of every index key (fp32 [T])
- * and one bit per (token, group, block) marking the pairs whose winner the bf16 MFMA
+ * and one bit per (token, group, block) marking the pairs whose winner the MFMA
  * pass could not certify. 0 for invalid sizes. */
 int64_t msa_score_fwd_workspace_bytes(int64_t total_tokens, int64_t groups, int64_t num_blocks);
 

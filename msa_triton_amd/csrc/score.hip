@@ -735,8 +735,11 @@ int score_fwd_launch(const void* iq, const void* ik, const int32_t* cu, int nseq
   // inside the MFMA kernel's tiles, from the scores just written, was measured slower
   // at c4 (2.43-2.81 ms vs 2.27 ms for the two launches): the score kernel runs two
   // workgroups per CU and the selection's registers cost its main loop.
-  if (DT == kBF16 && score_mfma_supported(Di, B, scale)) {
-    const int rc = score_fwd_mfma_launch(iq, ik, cu, nseq, rows, G, Di, NB, B, scale, scores, tie, ws, st);
+  // The MFMA pass reads 16 bytes at a time; fp16 and fp32 rows that do not start on 16-byte
+  // boundaries (or a caller without a workspace) keep the exact kernel.
+  const bool aligned = ((reinterpret_cast<uintptr_t>(iq) | reinterpret_cast<uintptr_t>(ik)) & 15) == 0;
+  if ((DT == kBF16 || (aligned && ws)) && score_mfma_supported(Di, B, scale)) {
+    const int rc = score_fwd_mfma_launch(DT, iq, ik, cu, nseq, rows, G, Di, NB, B, scale, scores, tie, ws, st);
     if (rc != kOk || !sel) return rc;
     return topk_launch(scores, cu, nseq, rows, G, NB, B, K, L, sel, st);
   }

@@ -1,5 +1,8 @@
-// Stage 1 on MFMA (bf16 inputs): block maxima of the indexer logits with a
-// certified exact winner.
+// Stage 1 on MFMA: block maxima of the indexer logits with a certified exact winner,
+// for bf16 and fp16 inputs (score_fwd_mfma_kernel) and fp32 inputs (score_fwd_f32_kernel).
+// Measured against the FP64 kernel that fp16 and fp32 used before (score_fwd_exact, one
+// wave per row and block): 8192 tokens x 4 groups of 128 dims in fp16 85.8 -> 0.13 ms with
+// the top-k, 2048 tokens x 2 groups in fp32 1.05 -> 0.12 ms.
 //
 // Work unit: a tile of 128 consecutive (t, g) rows of the flattened [T*G] row
 // space, 4 waves x 32 rows. A wave keeps its rows' query fragments in
@@ -11,10 +14,9 @@
 // the blocks go from memory straight to LDS (global_load_lds_dwordx4: 16 bytes
 // per lane, no staging registers) into unpadded rows whose 16-byte chunks are
 // XOR-swizzled by row, so the fragment reads stay bank-conflict free. Tiles are
-// issued heaviest first (the last rows of a sequence see the most blocks).
-// Squared key norms (for the error bound below) are computed once per key by a
-// pre-pass (score_key_norms), and each key block's largest norm and safety once per
-// block by a second (score_block_norms), instead of per tile.
+// issued heaviest first (the last rows of a sequence see the most blocks), each as one
+// or more workgroups (tile_parts). Each key block's largest norm and safety (for the error
+// bound below) come from a pre-pass (score_block_norms) instead of being formed per tile.
 //
 // Exactness (the public score is the reference's FP32 form of the exact winning dot,
 // public_score, and the winner set must be the exact one, index_score.py:121-136): with
@@ -34,12 +36,13 @@
 // half masked to zero: exact in fp32 when every nonzero element of the query row and
 // the key block lies in [2^-60, 2^55) ("safe": products then are normal fp32 numbers,
 // and no MFMA sum can overflow), and adding that exact product in FP64 gives the bits
-// of exact_dot's fused multiply-add. Pairs of an unsafe row or block go to the resolve
-// kernel below.
+// of exact_dot's fused multiply-add. (fp16 products are exact in fp32 whatever the finite
+// values; v_fma_mix_f32 forms them. fp32 elements are converted and fused in FP64.) Pairs of
+// an unsafe row or block go to the resolve kernel below.
 // Otherwise the (row, block) pair is marked in a bitmap that a second
-// kernel (score_fwd_resolve) settles after the main pass: one wave re-evaluates
-// every visible key of the block in FP64 (same order) and takes max / tie count /
-// first winner exactly. Deferring keeps the rare ambiguous rows (a few per
+// kernel (score_fwd_resolve) settles after the main pass: the keys within the bound of the
+// row's maximum are evaluated in FP64 (same order) for the maximum, tie count and first
+// winner. Deferring keeps the rare ambiguous rows (a few per
 // thousand on random data) from holding the other waves of a workgroup at the
 // next block barrier.
 // A negative scale flips the query signs once (exact), so every comparison is
@@ -62,7 +65,7 @@ constexpr int kThreads = 256;
 // block's first key), then the ambiguous-pair bitmap, block-major: bit
 // block * rows_pad + row of 32-bit words, rows_pad = rows rounded up to a whole number
 // of resolve chunks.
-constexpr int kResolveRows = 8192;  // rows per resolve workgroup
+constexpr int kResolveRows = 4096;  // rows per resolve wave: 64 bits for each of its lanes
 int64_t align256(int64_t x) { return (x + 255) & ~int64_t{255}; }
 int64_t ws_bnorm_offset(int64_t T) { return align256(4 * (T > 0 ? T : 1)); }
 int64_t ws_bitmap_offset(int64_t T) { return 2 * ws_bnorm_offset(T); }
@@ -126,9 +129,6 @@ __device__ __forceinline__ LanePair pair_xor16(uint32_t x) {
   return LanePair{r[0], r[1]};
 }
 
-__device__ __forceinline__ float bf16_lo(uint32_t w) { return __uint_as_float(w << 16); }
-__device__ __forceinline__ float bf16_hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
-
 // Both bf16 of a word zero or of magnitude in [2^-60, 2^55) (biased exponent 67 .. 181):
 // the product of two such values is zero or a normal fp32 number below 2^110, and a
 // sum of up to 128 of them stays below 2^117.
@@ -136,16 +136,149 @@ __device__ __forceinline__ bool bf16_safe(uint32_t x16) {
   const uint32_t e = (x16 >> 7) & 0xffu;
   return (x16 & 0x7fffu) == 0u || (e >= 67u && e <= 181u);
 }
-__device__ __forceinline__ bool word_safe(uint32_t w) { return bf16_safe(w & 0xffffu) && bf16_safe(w >> 16); }
-
-// fp32 product of the low (lo) or high bf16 of a and of b, exact when both are safe.
-__device__ __forceinline__ float prod_lo(uint32_t a, uint32_t b) {
-  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, a), __builtin_bit_cast(bf16x2_t, b & 0xffffu),
-                                         0.0f, false);
+// fp16: every product of two finite values is exact in fp32 (22 significant bits, from 2^-48
+// to 2^32, and sums of 128 stay finite), so only infinities and NaN are unsafe.
+template <int DT>
+__device__ __forceinline__ bool word_safe(uint32_t w) {
+  if constexpr (DT == kF16) return (w & 0x7c00u) != 0x7c00u && (w & 0x7c000000u) != 0x7c000000u;
+  else return bf16_safe(w & 0xffffu) && bf16_safe(w >> 16);
 }
+
+// fp32: zero or of magnitude in [2^-40, 2^55), so that the products of the bf16 terms (each
+// no smaller than 2^-63) are normal and their sums stay finite.
+__device__ __forceinline__ bool f32_safe(uint32_t w) {
+  const uint32_t e = (w >> 23) & 0xffu;
+  return (w & 0x7fffffffu) == 0u || (e >= 87u && e <= 181u);
+}
+
+// Eight consecutive elements as loaded.
+template <int DT>
+struct Words8 {
+  static constexpr int N = DT == kF32 ? 8 : 4;
+  uint32_t w[N];
+};
+template <int DT>
+__device__ __forceinline__ Words8<DT> load_words(const void* __restrict__ base, int64_t i) {
+  Words8<DT> r;
+  const uint4* p = reinterpret_cast<const uint4*>(static_cast<const char*>(base) + i * (DT == kF32 ? 4 : 2));
+#pragma unroll
+  for (int u = 0; u < Words8<DT>::N / 4; ++u) {
+    const uint4 x = p[u];
+    r.w[4 * u] = x.x, r.w[4 * u + 1] = x.y, r.w[4 * u + 2] = x.z, r.w[4 * u + 3] = x.w;
+  }
+  return r;
+}
+// n2 += the square(s) of the word's element(s); safe cleared if one is not safe.
+template <int DT>
+__device__ __forceinline__ void add_square(uint32_t w, float& n2, bool& safe) {
+  if constexpr (DT == kF32) {
+    n2 = fmaf(__uint_as_float(w), __uint_as_float(w), n2);
+    safe = safe && f32_safe(w);
+  } else {
+    n2 = fmaf(lo16_f32<DT>(w), lo16_f32<DT>(w), n2);
+    n2 = fmaf(hi16_f32<DT>(w), hi16_f32<DT>(w), n2);
+    safe = safe && word_safe<DT>(w);
+  }
+}
+// An MFMA operand of eight fp32 elements as two bf16 terms, x ~ hi + mid (to 2^-18 |x|).
+struct SplitFrag {
+  bf16x8 hi, mid;
+};
+__device__ __forceinline__ SplitFrag split_frag(const uint32_t (&w)[8]) {
+  uint32_t h[4], m[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const float x0 = __uint_as_float(w[2 * u]), x1 = __uint_as_float(w[2 * u + 1]);
+    h[u] = cvt_pk_bf16(x0, x1);
+    m[u] = cvt_pk_bf16(sub_lo_half(h[u], x0), sub_hi_half(h[u], x1));
+  }
+  return SplitFrag{__builtin_bit_cast(bf16x8, make_uint4(h[0], h[1], h[2], h[3])),
+                   __builtin_bit_cast(bf16x8, make_uint4(m[0], m[1], m[2], m[3]))};
+}
+// acc += a . b with both operands as two bf16 terms (the smaller products first).
+__device__ __forceinline__ f32x4 mfma_split(const SplitFrag& a, const SplitFrag& b, f32x4 acc) {
+  acc = mfma(a.mid, b.hi, acc);
+  acc = mfma(a.hi, b.mid, acc);
+  return mfma(a.hi, b.hi, acc);
+}
+
+// fp32 product of the low (lo) or high element of a and of b, exact when both are safe.
+template <int DT>
+__device__ __forceinline__ float prod_lo(uint32_t a, uint32_t b) {
+  if constexpr (DT == kF16)
+    return __builtin_fmaf(lo16_f32<DT>(a), lo16_f32<DT>(b), 0.f);  // v_fma_mix_f32
+  else
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, a),
+                                           __builtin_bit_cast(bf16x2_t, b & 0xffffu), 0.0f, false);
+}
+template <int DT>
 __device__ __forceinline__ float prod_hi(uint32_t a, uint32_t b) {
-  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, a),
-                                         __builtin_bit_cast(bf16x2_t, b & 0xffff0000u), 0.0f, false);
+  if constexpr (DT == kF16)
+    return __builtin_fmaf(hi16_f32<DT>(a), hi16_f32<DT>(b), 0.f);
+  else
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, a),
+                                           __builtin_bit_cast(bf16x2_t, b & 0xffff0000u), 0.0f, false);
+}
+
+// Two logits x, y (keys at positions pos, pos + 1) into a running top 2 (m1 the maximum,
+// m2 the largest other value, m1 >= m2 throughout): the second largest of {m1, m2, x, y}
+// is max(m2, med3(m1, x, y)). med3(a, b, +inf) is max(a, b); unlike fmaxf it needs no
+// canonicalised inputs. pinf is +inf in a register the optimiser cannot see through, or it
+// would turn the med3 back into a maximum with canonicalisations.
+__device__ __forceinline__ void fold_pair(float x, float y, uint32_t pos, float pinf, float& m1, float& m2) {
+  x = pack_key(x, pos);
+  y = pack_key(y, pos + 1);
+  const float t = __builtin_amdgcn_fmed3f(m1, x, y);
+  m2 = __builtin_amdgcn_fmed3f(m2, t, pinf);
+  m1 = max3(m1, x, y);
+}
+
+// A row's top 2 over its four key quarters (lanes c, c + 16, c + 32, c + 48): a1 the
+// maximum, a2 the largest other value, and the key index of the maximum (unique whenever
+// the row is certified).
+struct RowTop {
+  float a1, a2;
+  int key;
+};
+__device__ __forceinline__ RowTop merge_quarters(float m1, float m2, int q4) {
+  RowTop r{m1, m2, 0};
+#pragma unroll
+  for (int o = 16; o <= 32; o <<= 1) {  // with the quarter of lane ^ o
+    const LanePair p1 = o == 16 ? pair_xor16(__float_as_uint(r.a1)) : pair_xor32(__float_as_uint(r.a1));
+    const LanePair p2 = o == 16 ? pair_xor16(__float_as_uint(r.a2)) : pair_xor32(__float_as_uint(r.a2));
+    const float u = __uint_as_float(p1.a), v = __uint_as_float(p1.b);
+    r.a2 = max3(__uint_as_float(p2.a), __uint_as_float(p2.b), min2(u, v));
+    r.a1 = max3(u, v, v);
+  }
+  int wq = m1 == r.a1 ? q4 : 4;  // the quarter holding the maximum
+  const LanePair w16 = pair_xor16(static_cast<uint32_t>(wq));
+  wq = min(static_cast<int>(w16.a), static_cast<int>(w16.b));
+  const LanePair w32 = pair_xor32(static_cast<uint32_t>(wq));
+  wq = min(static_cast<int>(w32.a), static_cast<int>(w32.b));
+  const int pos = static_cast<int>(__float_as_uint(r.a1) & 0x7fu);  // 4 kt + i
+  r.key = 16 * (pos >> 2) + 4 * wq + (pos & 3);
+  return r;
+}
+
+// The sum of the two halves of a row's dot, held by lanes l and l ^ 32 (half 0 first; the
+// value is that of the lane pair whatever the lane).
+__device__ __forceinline__ double add_halves(double half) {
+  const uint64_t hbits = static_cast<uint64_t>(__double_as_longlong(half));
+  const LanePair hlo = pair_xor32(static_cast<uint32_t>(hbits));
+  const LanePair hhi = pair_xor32(static_cast<uint32_t>(hbits >> 32));
+  const double h0 = __longlong_as_double(static_cast<long long>((static_cast<uint64_t>(hhi.a) << 32) | hlo.a));
+  const double h1 = __longlong_as_double(static_cast<long long>((static_cast<uint64_t>(hhi.b) << 32) | hlo.b));
+  return h0 + h1;
+}
+
+// The logits' error bound per ||q|| max ||k||: half the distance below the approximate
+// maximum from which a key is certainly beaten. 16-bit inputs: DP exact products summed in
+// fp32. fp32 inputs enter as two bf16 terms each (s = qh kh + qh km + qm kh): the terms left
+// out are below 3 x 2^-18 |q| |k| in all, and 3 DP products are summed.
+template <int DT, int DP>
+constexpr float logit_error() {
+  return DT == kF32 ? 3.1f * 0x1p-18f + static_cast<float>(3 * DP + 8) * 0x1p-22f
+                    : static_cast<float>(DP + 8) * 0x1p-22f;
 }
 
 // Iteration space of a tile: (sequence, block) pairs for every sequence overlapping
@@ -178,40 +311,128 @@ __device__ __forceinline__ BlockCursor next_block(const int32_t* __restrict__ cu
   return BlockCursor{nseq, 0, -1};
 }
 
+// Part `part` of `parts` equal runs of the tile's (sequence, block) pairs: its first pair and
+// their number.
+__device__ __forceinline__ BlockCursor tile_share(const int32_t* __restrict__ cu, int nseq, int64_t r0, int nr, int G,
+                                                  int B, int part, int parts, int& todo) {
+  const int64_t t_last = (r0 + nr - 1) / G;
+  const int s0 = find_seq(cu, nseq, r0 / G);
+  int pairs = 0;
+  for (int s = s0; s < nseq && cu[s] <= t_last; ++s)
+    if (cu[s + 1] > cu[s]) pairs += last_block_of(cu, s, r0, nr, G, B) + 1;
+  int skip = static_cast<int>(static_cast<int64_t>(pairs) * part / parts);
+  todo = static_cast<int>(static_cast<int64_t>(pairs) * (part + 1) / parts) - skip;
+  if (todo <= 0) return BlockCursor{nseq, 0, -1};
+  for (int s = s0; s < nseq && cu[s] <= t_last; ++s) {
+    if (cu[s + 1] <= cu[s]) continue;
+    const int last = last_block_of(cu, s, r0, nr, G, B);
+    if (skip <= last) return BlockCursor{s, skip, last};
+    skip -= last + 1;
+  }
+  return BlockCursor{nseq, 0, -1};
+}
+
+// Blocks without a causal key: score -inf, tie code 0, for up to 32 rows from `row0` (those
+// of one wave); the tile's parts (blockIdx.y) share the rows.
+__device__ __forceinline__ void fill_future(const int32_t* __restrict__ cu, int nseq, int64_t row0, int nr, int G,
+                                            int NB, int B, float* __restrict__ scores, int32_t* __restrict__ tie) {
+  const int lane = threadIdx.x & 63, j0 = lane & 31;
+  int own = NB;
+  if (j0 < nr) {
+    const int64_t t = (row0 + j0) / G;
+    own = static_cast<int>((t - cu[find_seq(cu, nseq, t)]) / B);
+  }
+  for (int j = blockIdx.y; j < 32 && j < nr; j += gridDim.y) {
+    const int64_t base = (row0 + j) * NB;
+    for (int b = __shfl(own, j, kWave) + 1 + lane; b < NB; b += kWave) {
+      scores[base + b] = -__builtin_inff();
+      if (tie) tie[base + b] = 0;
+    }
+  }
+}
+
 }  // namespace
 
-// Squared norm of every index key, rounded up by 1.0001 (bounds the fp32 rounding of
-// the sum): the max over a key block enters the MFMA logits' error bound. The sign bit
-// is set for a key that is not safe (a nonzero element outside [2^-60, 2^55)).
-// Also clears the ambiguous-pair bitmap the main pass marks.
-__global__ __launch_bounds__(256) void score_key_norms(const uint16_t* __restrict__ ik, int64_t T, int Di,
+// The squared norm of `n` elements from element i, rounded up by 1.0001 (bounds the fp32
+// rounding of the sum), with the sign bit set when one of them is not safe.
+template <int DT>
+__device__ __forceinline__ float signed_norm2(const void* __restrict__ ik, int64_t i, int n) {
+  float n2 = 0.f;
+  bool safe = true;
+#pragma unroll 8  // a row's loads in flight together
+  for (int d = 0; d < n; d += 8) {
+    const Words8<DT> w = load_words<DT>(ik, i + d);
+#pragma unroll
+    for (int u = 0; u < Words8<DT>::N; ++u) add_square<DT>(w.w[u], n2, safe);
+  }
+  return safe ? n2 * 1.0001f : -(fabsf(n2) * 1.0001f) - 1.0f;
+}
+
+// The key norms that enter the error bound, and the ambiguous-pair bitmap cleared. Per key
+// block, stored at the block's first key: the largest key norm, sqrt(max ||k||^2), negated
+// when a key of the block is not safe (or not a number). Safety is read from the sign bit:
+// a block whose only unsafe key is NaN (fmaxf skips its NaN entry) and whose other keys are
+// zero stores -0. One workgroup per 64 tokens; for each block that starts among them (one or
+// two when 64 <= B <= 128, this kernel's range) two threads take each key, half a row each.
+// Bound by the latency of its few loads (8.4 us at 2048 keys of 512 bytes; with one lane
+// per whole row in one wave per block 14.7 us, with the lanes side by side along a row 39.8 us:
+// the shuffles).
+template <int DT>
+__global__ __launch_bounds__(256) void score_block_norms(const void* __restrict__ ik, const int32_t* __restrict__ cu,
+                                                         int nseq, int64_t T, int Di, int B, float* __restrict__ bnorm,
+                                                         uint32_t* __restrict__ amb, int64_t amb_words) {
+  __shared__ float part[256];
+  __shared__ float wmax[2];
+  const int64_t a = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (a < amb_words) amb[a] = 0u;
+  const int tid = threadIdx.x, lane = tid & 63, key = tid & 127, hf = tid >> 7;
+  const int64_t base = static_cast<int64_t>(blockIdx.x) * 64;
+  if (base >= T) return;  // whole workgroup
+  int32_t end = 0;
+  bool starts = false;
+  if (base + lane < T) {  // every wave looks at the same 64 tokens
+    const int32_t t = static_cast<int32_t>(base) + lane;
+    const int s = find_seq_near(cu, nseq, t);
+    end = cu[s + 1];
+    starts = (t - cu[s]) % B == 0;
+  }
+  for (uint64_t m = __ballot(starts); m; m &= m - 1) {
+    const int l = __builtin_ctzll(m);
+    const int64_t t0 = base + l;
+    const int64_t e0 = __shfl(end, l, kWave);
+    const int nk = static_cast<int>(t0 + B < e0 ? B : e0 - t0);
+    const int n1 = Di / 16 * 8;  // the first half's elements, a multiple of 8
+    part[tid] = key < nk ? signed_norm2<DT>(ik, (t0 + key) * Di + (hf ? n1 : 0), hf ? Di - n1 : n1) : 0.f;
+    __syncthreads();
+    if (tid < 128) {
+      const float x = part[tid], y = part[tid + 128];
+      const float r = sqrtf(fmaxf(wave_max_f32(fabsf(x) + fabsf(y)), 0.f));  // (maxima skip NaN)
+      const bool ok = __ballot(!(x >= 0.f && y >= 0.f)) == 0;
+      if (lane == 0) wmax[tid >> 6] = ok ? r : -r;
+    }
+    __syncthreads();
+    if (tid == 0) {
+      const float x = wmax[0], y = wmax[1], r = fmaxf(fabsf(x), fabsf(y));
+      bnorm[t0] = __builtin_signbit(x) == 0 && __builtin_signbit(y) == 0 ? r : -r;
+    }
+    __syncthreads();  // part is rewritten for the next block
+  }
+}
+
+// The same for blocks of fewer than 64 keys, in two passes: the norms of all keys (and the
+// bitmap), then one thread per block.
+template <int DT>
+__global__ __launch_bounds__(256) void score_key_norms(const void* __restrict__ ik, int64_t T, int Di,
                                                        float* __restrict__ knorm2, uint32_t* __restrict__ amb,
                                                        int64_t amb_words) {
   const int64_t j = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
   if (j < amb_words) amb[j] = 0u;
-  if (j >= T) return;
-  float n2 = 0.f;
-  bool safe = true;
-  for (int d = 0; d < Di; d += 8) {
-    const uint4 w = *reinterpret_cast<const uint4*>(ik + j * Di + d);
-    const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      n2 = fmaf(bf16_lo(ws[u]), bf16_lo(ws[u]), n2);
-      n2 = fmaf(bf16_hi(ws[u]), bf16_hi(ws[u]), n2);
-      safe = safe && word_safe(ws[u]);
-    }
-  }
-  knorm2[j] = safe ? n2 * 1.0001f : -(n2 * 1.0001f) - 1.0f;  // unsafe: negative
+  if (j < T) knorm2[j] = signed_norm2<DT>(ik, j * Di, Di);
 }
 
-// Per key block, stored at the block's first key: the largest key norm of the block,
-// sqrt(max |knorm2|), negated when a key of the block is not safe (or not a number).
-// Safety is read from the sign bit: a block whose only unsafe key is NaN (fmaxf skips
-// its NaN entry) and whose other keys are zero stores -0.
-__global__ __launch_bounds__(256) void score_block_norms(const float* __restrict__ knorm2,
-                                                         const int32_t* __restrict__ cu, int nseq, int64_t T, int B,
-                                                         float* __restrict__ bnorm) {
+__global__ __launch_bounds__(256) void score_small_block_norms(const float* __restrict__ knorm2,
+                                                               const int32_t* __restrict__ cu, int nseq, int64_t T,
+                                                               int B, float* __restrict__ bnorm) {
   const int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
   if (t >= T) return;
   const int s = find_seq(cu, nseq, t);
@@ -231,7 +452,7 @@ __global__ __launch_bounds__(256) void score_block_norms(const float* __restrict
 
 // Two workgroups per CU; one for the widest partial-width variant (index dim 72..120),
 // whose register staging of the next block does not fit beside two.
-template <int NK, bool FULLD>
+template <int DT, int NK, bool FULLD>
 __global__ __launch_bounds__(kThreads, NK == 4 && !FULLD ? 1 : 2) void score_fwd_mfma_kernel(const uint16_t* __restrict__ iq,
                                                                      const uint16_t* __restrict__ ik,
                                                                      const int32_t* __restrict__ cu, int nseq,
@@ -252,7 +473,7 @@ __global__ __launch_bounds__(kThreads, NK == 4 && !FULLD ? 1 : 2) void score_fwd
   const bool neg = scale < 0.0;
   const float fscale = static_cast<float>(fabs(scale));  // the reference's FP32 |scale|
   const uint32_t flip = neg ? 0x80008000u : 0u;
-  const float cerr = static_cast<float>(DP + 8) * 0x1p-22f;
+  constexpr float cerr = logit_error<DT, DP>();
   // exact_dot's split point (Di % 8 == 0, so h % 4 == 0); compile-time for Di == DP
   const int h = FULLD ? DP / 2 : Di / 2;
 
@@ -294,11 +515,11 @@ __global__ __launch_bounds__(kThreads, NK == 4 && !FULLD ? 1 : 2) void score_fwd
     x.y ^= flip;
     qh[2 * w4] = x.x;
     qh[2 * w4 + 1] = x.y;
-    pn2 = fmaf(bf16_lo(x.x), bf16_lo(x.x), pn2);
-    pn2 = fmaf(bf16_hi(x.x), bf16_hi(x.x), pn2);
-    pn2 = fmaf(bf16_lo(x.y), bf16_lo(x.y), pn2);
-    pn2 = fmaf(bf16_hi(x.y), bf16_hi(x.y), pn2);
-    psafe = psafe && word_safe(x.x) && word_safe(x.y);
+    pn2 = fmaf(lo16_f32<DT>(x.x), lo16_f32<DT>(x.x), pn2);
+    pn2 = fmaf(hi16_f32<DT>(x.x), hi16_f32<DT>(x.x), pn2);
+    pn2 = fmaf(lo16_f32<DT>(x.y), lo16_f32<DT>(x.y), pn2);
+    pn2 = fmaf(hi16_f32<DT>(x.y), hi16_f32<DT>(x.y), pn2);
+    psafe = psafe && word_safe<DT>(x.x) && word_safe<DT>(x.y);
   }
   pn2 += __shfl_xor(pn2, 32, kWave);
   psafe = psafe && __shfl_xor(static_cast<int>(psafe), 32, kWave) != 0;  // both halves of the row
@@ -374,13 +595,8 @@ __global__ __launch_bounds__(kThreads, NK == 4 && !FULLD ? 1 : 2) void score_fwd
     return bc.s < nseq ? bnorm[cu[bc.s] + static_cast<int64_t>(bc.b) * B] : 0.f;
   };
 
-  // first (sequence, block) of the tile
-  BlockCursor cur{nseq, 0, -1};
-  {
-    const int64_t t_first = r0 / G;
-    const int s0 = find_seq(cu, nseq, t_first);
-    cur = BlockCursor{s0, 0, last_block_of(cu, s0, r0, nr, G, B)};
-  }
+  int todo;
+  BlockCursor cur = tile_share(cu, nseq, r0, nr, G, B, blockIdx.y, gridDim.y, todo);
   const float cn = block_norm(cur);
   fetch(cur, ik, sm.k[0]);
   commit(0);
@@ -390,7 +606,8 @@ __global__ __launch_bounds__(kThreads, NK == 4 && !FULLD ? 1 : 2) void score_fwd
   bool bsafe = !__builtin_signbit(cn);  // -0 marks an unsafe block too
   int buf = 0;
   while (cur.s < nseq) {
-    const BlockCursor nxt = next_block(cu, nseq, cur, r0, nr, G, B);
+    BlockCursor nxt = next_block(cu, nseq, cur, r0, nr, G, B);
+    if (--todo <= 0) nxt.s = nseq;
     const float nn = block_norm(nxt);
     // The next block's fetch and this block's LDS reads go through the restrict-qualified
     // pointers of one inlined call, so the compiler's wait insertion can tell the fetch's
@@ -412,12 +629,8 @@ __global__ __launch_bounds__(kThreads, NK == 4 && !FULLD ? 1 : 2) void score_fwd
     }
     const bool wave_on = __ballot(lim[0] > 0 || lim[1] > 0) != 0;  // wave-uniform
     // approximate logits, 16 keys at a time, key position packed into their low bits,
-    // folded into a per-row running top 2: m1 the maximum, m2 the largest other value
-    // (med3(m1, v, m2) is the new second largest)
+    // folded into a per-row running top 2
     float m1[2] = {kMaskedLogit, kMaskedLogit}, m2[2] = {kMaskedLogit, kMaskedLogit};
-    // med3(m1, v, +inf) is the maximum; unlike fmaxf it needs no canonicalised inputs. The
-    // +inf sits in a register the optimiser cannot see through, or it would turn the med3
-    // back into a maximum with canonicalisations.
     float pinf = __builtin_inff();
     asm volatile("" : "+v"(pinf));
     auto scan = [&](auto masked) {
@@ -430,19 +643,15 @@ __global__ __launch_bounds__(kThreads, NK == 4 && !FULLD ? 1 : 2) void score_fwd
         for (int rt = 0; rt < 2; ++rt) {
           f32x4 a = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int kk = 0; kk < NK; ++kk) a = mfma(kf[kk], qf[rt][kk], a);
+          for (int kk = 0; kk < NK; ++kk) a = mfma_t<DT>(kf[kk], qf[rt][kk], a);
 #pragma unroll
-          for (int i = 0; i < 4; i += 2) {  // two logits x, y at a time (m1 >= m2 throughout):
-            float x = a[i], y = a[i + 1];     // second largest of {m1, m2, x, y} = max(m2, med3(m1, x, y))
+          for (int i = 0; i < 4; i += 2) {
+            float x = a[i], y = a[i + 1];
             if constexpr (decltype(masked)::value) {
               x = 16 * kt + 4 * q4 + i < lim[rt] ? x : kMaskedLogit;
               y = 16 * kt + 4 * q4 + i + 1 < lim[rt] ? y : kMaskedLogit;
             }
-            x = pack_key(x, 4 * kt + i);
-            y = pack_key(y, 4 * kt + i + 1);
-            const float t = __builtin_amdgcn_fmed3f(m1[rt], x, y);
-            m2[rt] = __builtin_amdgcn_fmed3f(m2[rt], t, pinf);
-            m1[rt] = max3(m1[rt], x, y);
+            fold_pair(x, y, 4 * kt + i, pinf, m1[rt], m2[rt]);
           }
         }
       }
@@ -459,26 +668,11 @@ __global__ __launch_bounds__(kThreads, NK == 4 && !FULLD ? 1 : 2) void score_fwd
       int widx[2], wcnt[2];
 #pragma unroll
       for (int rt = 0; rt < 2; ++rt) {
-        float a1 = m1[rt], a2 = m2[rt];
-#pragma unroll
-        for (int o = 16; o <= 32; o <<= 1) {  // with the quarter of lane ^ o
-          const LanePair p1 = o == 16 ? pair_xor16(__float_as_uint(a1)) : pair_xor32(__float_as_uint(a1));
-          const LanePair p2 = o == 16 ? pair_xor16(__float_as_uint(a2)) : pair_xor32(__float_as_uint(a2));
-          const float u = __uint_as_float(p1.a), v = __uint_as_float(p1.b);
-          a2 = max3(__uint_as_float(p2.a), __uint_as_float(p2.b), min2(u, v));
-          a1 = max3(u, v, v);
-        }
-        // the quarter holding the maximum (unique whenever the row is certified)
-        int wq = m1[rt] == a1 ? q4 : 4;
-        const LanePair w16 = pair_xor16(static_cast<uint32_t>(wq));
-        wq = min(static_cast<int>(w16.a), static_cast<int>(w16.b));
-        const LanePair w32 = pair_xor32(static_cast<uint32_t>(wq));
-        wq = min(static_cast<int>(w32.a), static_cast<int>(w32.b));
-        const int pos = static_cast<int>(__float_as_uint(a1) & 0x7fu);  // 4 kt + i
-        widx[rt] = 16 * (pos >> 2) + 4 * wq + (pos & 3);
-        const float bound = 2.f * cerr * mnorm[rt] * kmax + 0x1p-15f * fmaxf(fabsf(a1), fabsf(a2)) + 0x1p-126f;
+        const RowTop top = merge_quarters(m1[rt], m2[rt], q4);
+        widx[rt] = top.key;
+        const float bound = 2.f * cerr * mnorm[rt] * kmax + 0x1p-15f * fmaxf(fabsf(top.a1), fabsf(top.a2)) + 0x1p-126f;
         // 2: at least two candidates, or products not certainly exact in fp32
-        wcnt[rt] = (a2 >= a1 - bound || !(bsafe && msafe[rt])) ? 2 : 1;
+        wcnt[rt] = (top.a2 >= top.a1 - bound || !(bsafe && msafe[rt])) ? 2 : 1;
       }
       // lane pair (pr, hf): row wr0 + pr = 16 rt + c with rt = pr >> 4 -- this lane's c matches
       const int prt = pr >> 4;
@@ -508,22 +702,17 @@ __global__ __launch_bounds__(kThreads, NK == 4 && !FULLD ? 1 : 2) void score_fwd
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
               if (FULLD || 8 * j8 + 2 * u < h) {
-                half += static_cast<double>(prod_lo(qh[4 * j8 + u], kx[u]));
-                half += static_cast<double>(prod_hi(qh[4 * j8 + u], kx[u]));
+                half += static_cast<double>(prod_lo<DT>(qh[4 * j8 + u], kx[u]));
+                half += static_cast<double>(prod_hi<DT>(qh[4 * j8 + u], kx[u]));
               }
             }
           }
         }
       }
-      // the two halves of the row (lanes pr and pr + 32), summed
-      const uint64_t hbits = static_cast<uint64_t>(__double_as_longlong(half));
-      const LanePair hlo = pair_xor32(static_cast<uint32_t>(hbits));
-      const LanePair hhi = pair_xor32(static_cast<uint32_t>(hbits >> 32));
-      const double h0 = __longlong_as_double(static_cast<long long>((static_cast<uint64_t>(hhi.a) << 32) | hlo.a));
-      const double h1 = __longlong_as_double(static_cast<long long>((static_cast<uint64_t>(hhi.b) << 32) | hlo.b));
+      const double dot = add_halves(half);  // lanes pr and pr + 32
       if (row_ok && mycnt == 1 && hf == 0) {
         const int64_t out = (r0 + prow) * NB + cur.b;
-        scores[out] = public_score(h0 + h1, fscale);
+        scores[out] = public_score(dot, fscale);
         if (tie) tie[out] = myidx + 1;
       }
       // ambiguous rows: marked for score_fwd_resolve
@@ -542,148 +731,406 @@ __global__ __launch_bounds__(kThreads, NK == 4 && !FULLD ? 1 : 2) void score_fwd
     cur = nxt;
   }
 
-  // ---- blocks without a causal key: -inf, tie code 0 (each wave fills its rows)
-  const int64_t pstart = pin ? cu[find_seq(cu, nseq, ptok)] : 0;
-  const int pqb = pin ? static_cast<int>((ptok - pstart) / B) : NB;
-  for (int j = 0; j < 32; ++j) {
-    const int qbj = __shfl(pqb, j, kWave);
-    if (wr0 + j >= nr) break;
-    const int64_t base = (r0 + wr0 + j) * NB;
-    for (int b = qbj + 1 + lane; b < NB; b += kWave) {
-      scores[base + b] = -__builtin_inff();
-      if (tie) tie[base + b] = 0;
-    }
-  }
+  fill_future(cu, nseq, r0 + wr0, nr - wr0, G, NB, B, scores, tie);
 }
 
-// The ambiguous (row, block) pairs the main pass marked, settled exactly. Workgroup
-// (b, c) takes block b for rows [c, c + kResolveRows): it lists the marked rows in
-// order, and for each run of listed rows of one sequence stages that sequence's block
-// b in LDS; the four waves then take windows of up to kResolvePairs rows of the run
-// independently. In a window, lane l runs exact_dot's two FMA chains (over the halves
-// of the index dim) for keys l and l + 64 and every row of the window at once (each
-// key element and each query element converted to FP64 once per window), from the
-// window's query rows staged in the wave's LDS slot (sign-directed bf16), and adds
-// the halves half 0 first; the maximum is reduced over the wave, tie count and first
-// winner come from ballots. The score and tie code are written as the exact kernel
-// writes them.
-constexpr int kResolvePairs = 4;
-__global__ __launch_bounds__(256) void score_fwd_resolve(const uint16_t* __restrict__ iq,
-                                                         const uint16_t* __restrict__ ik,
-                                                         const int32_t* __restrict__ cu, int nseq, int64_t rows,
-                                                         int64_t rows_pad, int G, int Di, int NB, int B,
-                                                         double scale, const uint32_t* __restrict__ amb,
-                                                         float* __restrict__ scores, int32_t* __restrict__ tie) {
-  constexpr int KS = 136;  // key row stride in LDS (bf16): consecutive rows hit distinct 16-byte bank groups
-  constexpr int P = kResolvePairs;
-  __shared__ alignas(16) uint16_t keys[128 * KS];
-  __shared__ alignas(16) uint16_t qs[4][P][128];
-  __shared__ uint16_t list[kResolveRows];
-  __shared__ int wsum[4];
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int b = blockIdx.x;
-  const int64_t c0 = static_cast<int64_t>(blockIdx.y) * kResolveRows;
-  // ---- the marked rows of this chunk, ascending (one bitmap word per thread)
-  constexpr int NW = kResolveRows / 32;  // bitmap words of the chunk (<= threads)
-  static_assert(NW <= 256, "one bitmap word per thread");
-  uint32_t mine = tid < NW ? amb[(static_cast<int64_t>(b) * rows_pad + c0) / 32 + tid] : 0u;
-  const int cnt = __popc(mine);
-  int incl = cnt;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int y = __shfl_up(incl, o, kWave);
-    if (lane >= o) incl += y;
+// The fp32 form: every element enters the MFMA logits as two bf16 terms (three products),
+// split from the fp32 key block in LDS as the fragments are read; the certified winner's
+// exact dot reads its fp32 row from the same block. One LDS buffer (64 KiB at 128 dims), so
+// that two workgroups share a CU and one's fetch runs beside the other's products.
+template <int NK>
+struct KeyRowsF32 {
+  static constexpr int CPK = 8 * NK;  // 16-byte chunks per key row
+  // chunk of dims [4p, 4p + 4) of key `row`: swizzled so that the 16 rows of a fragment read
+  // (one chunk of each) cover all 64 banks
+  static __device__ __forceinline__ int at(int row, int p) {
+    return row * CPK + (p ^ (NK == 1 ? (row >> 1) & 7 : row & 15));
   }
-  if (lane == 63) wsum[wv] = incl;
-  if (__syncthreads_or(mine != 0u) == 0) return;  // nothing marked (uniform)
-  int o = incl - cnt;
-  for (int w = 0; w < wv; ++w) o += wsum[w];
-  for (; mine; mine &= mine - 1) list[o++] = static_cast<uint16_t>(32 * tid + __builtin_ctz(mine));
-  const int n = wsum[0] + wsum[1] + wsum[2] + wsum[3];
-  const uint16_t flip = scale < 0.0 ? 0x8000u : 0u;
-  const int h = Di / 2;  // a multiple of 4
-  __syncthreads();  // the list is complete
-  for (int i = 0; i < n;) {  // runs of rows of one sequence (uniform)
-    const int s = find_seq(cu, nseq, (c0 + list[i]) / G);
-    const int64_t start = cu[s], end = cu[s + 1];
-    const int64_t end_row = end * G - c0;  // chunk-relative end of the sequence's rows
-    int j = i + 1;
-    while (j < n && list[j] < end_row) ++j;
-    const int64_t k0 = start + static_cast<int64_t>(b) * B;
-    const int nk = static_cast<int>((k0 + B < end ? k0 + B : end) - k0);  // >= 1: a listed row sees block b
-    const int cpr = Di / 8;
-    for (int e = tid; e < nk * cpr; e += 256) {
-      const int r = e / cpr, c = e % cpr;
-      *reinterpret_cast<uint4*>(keys + r * KS + 8 * c) = *reinterpret_cast<const uint4*>(ik + (k0 + r) * Di + 8 * c);
+};
+
+template <int NK>
+__global__ __launch_bounds__(kThreads, 2) void score_fwd_f32_kernel(const float* __restrict__ iq,
+                                                                    const float* __restrict__ ik,
+                                                                    const int32_t* __restrict__ cu, int nseq,
+                                                                    int64_t rows, int G, int Di, int NB, int B,
+                                                                    double scale, const float* __restrict__ bnorm,
+                                                                    uint32_t* __restrict__ amb, int64_t rows_pad,
+                                                                    float* __restrict__ scores,
+                                                                    int32_t* __restrict__ tie) {
+  using Rows = KeyRowsF32<NK>;
+  constexpr int DP = 32 * NK, CPK = Rows::CPK, KCH = 128 * CPK / kThreads, HF = DP / 2;
+  __shared__ alignas(16) uint4 keys[128 * CPK];
+  const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, q4 = lane >> 4;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int64_t r0 = static_cast<int64_t>(gridDim.x - 1 - blockIdx.x) * kTileRows;  // heaviest tiles first
+  const int nr = static_cast<int>(rows - r0 < kTileRows ? rows - r0 : kTileRows);
+  const float fscale = static_cast<float>(fabs(scale));
+  const uint32_t flip = scale < 0.0 ? 0x80000000u : 0u;
+  constexpr float cerr = logit_error<kF32, DP>();
+  const int h = Di / 2;  // exact_dot's split point, a multiple of 4
+
+  // ---- this wave's rows: MFMA operands (rows 16 rt + c), zero past Di
+  const int wr0 = 32 * wid;
+  SplitFrag qf[2][NK];
+  int64_t mtok[2];
+#pragma unroll
+  for (int rt = 0; rt < 2; ++rt) {
+    const int rr = wr0 + 16 * rt + c;
+    mtok[rt] = rr < nr ? (r0 + rr) / G : -1;
+#pragma unroll
+    for (int kk = 0; kk < NK; ++kk) {
+      const int d0 = 32 * kk + 8 * q4;
+      Words8<kF32> w = {};
+      if (rr < nr && d0 < Di) w = load_words<kF32>(iq, (r0 + rr) * Di + d0);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) w.w[u] ^= flip;
+      qf[rt][kk] = split_frag(w.w);
     }
-    __syncthreads();  // the block is staged
-    for (int w0 = i + P * wv; w0 < j; w0 += 4 * P) {  // this wave's windows
-      const int np = j - w0 < P ? j - w0 : P;
-      for (int e = lane; e < np * Di; e += kWave) {
-        const int p = e / Di, d = e % Di;
-        qs[wv][p][d] = iq[(c0 + list[w0 + p]) * Di + d] ^ flip;
-      }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      double acc[2][2][P];  // [key lane / lane + 64][half][row]
+  }
+  // ... and the exact-dot layout: lane (pr = lane & 31, hf = lane >> 5) keeps half hf of row
+  // wr0 + pr
+  const int pr = lane & 31, hf = lane >> 5;
+  const int prow = wr0 + pr;
+  const bool pin = prow < nr;
+  float qh[HF];
+  float pn2 = 0.f;
+  bool psafe = true;
 #pragma unroll
-      for (int kh = 0; kh < 2; ++kh)
+  for (int j = 0; j < HF / 4; ++j) {
+    uint4 x = make_uint4(0u, 0u, 0u, 0u);
+    if (pin && 4 * j < h) x = *reinterpret_cast<const uint4*>(iq + (r0 + prow) * Di + hf * h + 4 * j);
+    const uint32_t xs[4] = {x.x, x.y, x.z, x.w};
 #pragma unroll
-        for (int hh = 0; hh < 2; ++hh)
+    for (int u = 0; u < 4; ++u) {
+      add_square<kF32>(xs[u], pn2, psafe);
+      qh[4 * j + u] = __uint_as_float(xs[u] ^ flip);
+    }
+  }
+  pn2 += __shfl_xor(pn2, 32, kWave);
+  psafe = psafe && __shfl_xor(static_cast<int>(psafe), 32, kWave) != 0;
+  const float pnorm = sqrtf(pn2) * 1.0001f;  // ||q|| of row prow, rounded up
+  float mnorm[2];
+  bool msafe[2];
 #pragma unroll
-          for (int p = 0; p < P; ++p) acc[kh][hh][p] = 0.0;
-      for (int d = 0; d < h; d += 4) {
+  for (int rt = 0; rt < 2; ++rt) {
+    mnorm[rt] = __shfl(pnorm, 16 * rt + c, kWave);
+    msafe[rt] = __shfl(static_cast<int>(psafe), 16 * rt + c, kWave) != 0;
+  }
+
+  int todo;
+  BlockCursor cur = tile_share(cu, nseq, r0, nr, G, B, blockIdx.y, gridDim.y, todo);
+  float pinf = __builtin_inff();
+  asm volatile("" : "+v"(pinf));
+  while (cur.s < nseq) {
+    const int64_t start = cu[cur.s], end = cu[cur.s + 1];
+    const int64_t kb = start + static_cast<int64_t>(cur.b) * B;
+    const int nk = static_cast<int>(end - kb < B ? end - kb : B);
+    // wave wid's instruction i fills physical chunks (wid KCH + i) 64 + lane; rows past the
+    // block's end repeat its last key (masked later), chunks past Di the row's last one (their
+    // query operands are zero; a block with a key that is not finite is not certified)
+    __syncthreads();  // the previous block's readers are done
 #pragma unroll
-        for (int hh = 0; hh < 2; ++hh) {
-          double qv[P][4];
+    for (int i = 0; i < KCH; ++i) {
+      const int p = (wid * KCH + i) * 64 + lane;
+      const int row = p / CPK, lc = Rows::at(row, p % CPK) - row * CPK;
+      const int rowc = row < nk ? row : nk - 1, lcc = 4 * lc < Di ? lc : Di / 4 - 1;
+      __builtin_amdgcn_global_load_lds(
+          ik + (kb + rowc) * Di + 4 * lcc,
+          (__attribute__((address_space(3))) void*)(reinterpret_cast<char*>(keys) + (wid * KCH + i) * 1024), 16, 0, 0);
+    }
+    const float bn = bnorm[kb];
+    const float kmax = fabsf(bn);
+    const bool bsafe = !__builtin_signbit(bn);
+    int lim[2];
 #pragma unroll
-          for (int p = 0; p < P; ++p) {
-            const uint2 w = *reinterpret_cast<const uint2*>(&qs[wv][p][hh * h + d]);
-            qv[p][0] = static_cast<double>(bf16_lo(w.x));
-            qv[p][1] = static_cast<double>(bf16_hi(w.x));
-            qv[p][2] = static_cast<double>(bf16_lo(w.y));
-            qv[p][3] = static_cast<double>(bf16_hi(w.y));
+    for (int rt = 0; rt < 2; ++rt) {
+      const int64_t t = mtok[rt];
+      const int64_t v = (t >= start && t < end) ? t - kb + 1 : 0;
+      lim[rt] = v <= 0 ? 0 : (v < nk ? static_cast<int>(v) : nk);
+    }
+    const bool wave_on = __ballot(lim[0] > 0 || lim[1] > 0) != 0;  // wave-uniform
+    __builtin_amdgcn_s_waitcnt(0);  // this thread's direct-to-LDS loads have landed
+    __syncthreads();
+    if (wave_on) {
+      float m1[2] = {kMaskedLogit, kMaskedLogit}, m2[2] = {kMaskedLogit, kMaskedLogit};
+      auto scan = [&](auto masked) {
+#pragma unroll
+        for (int kt = 0; kt < 8; ++kt) {
+          f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+          for (int kk = 0; kk < NK; ++kk) {
+            const uint4 a = keys[Rows::at(16 * kt + c, 8 * kk + 2 * q4)];
+            const uint4 b = keys[Rows::at(16 * kt + c, 8 * kk + 2 * q4 + 1)];
+            const uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+            const SplitFrag kf = split_frag(w);
+#pragma unroll
+            for (int rt = 0; rt < 2; ++rt) acc[rt] = mfma_split(kf, qf[rt][kk], acc[rt]);
           }
 #pragma unroll
-          for (int kh = 0; kh < 2; ++kh) {
-            const uint2 w = *reinterpret_cast<const uint2*>(keys + (lane + 64 * kh) * KS + hh * h + d);
-            const double k4[4] = {static_cast<double>(bf16_lo(w.x)), static_cast<double>(bf16_hi(w.x)),
-                                  static_cast<double>(bf16_lo(w.y)), static_cast<double>(bf16_hi(w.y))};
+          for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
-            for (int p = 0; p < P; ++p) {
-              double a = acc[kh][hh][p];
+            for (int i = 0; i < 4; i += 2) {
+              float x = acc[rt][i], y = acc[rt][i + 1];
+              if constexpr (decltype(masked)::value) {
+                x = 16 * kt + 4 * q4 + i < lim[rt] ? x : kMaskedLogit;
+                y = 16 * kt + 4 * q4 + i + 1 < lim[rt] ? y : kMaskedLogit;
+              }
+              fold_pair(x, y, 4 * kt + i, pinf, m1[rt], m2[rt]);
+            }
+        }
+      };
+      if (__ballot(lim[0] < 128 || lim[1] < 128) == 0)  // no key masked in the wave
+        scan(std::false_type{});
+      else
+        scan(std::true_type{});
+      int widx[2];
+      bool sure[2];  // exactly one candidate
 #pragma unroll
-              for (int u = 0; u < 4; ++u) a = fma(qv[p][u], k4[u], a);
-              acc[kh][hh][p] = a;
+      for (int rt = 0; rt < 2; ++rt) {
+        const RowTop top = merge_quarters(m1[rt], m2[rt], q4);
+        widx[rt] = top.key;
+        const float bound =
+            2.f * cerr * mnorm[rt] * kmax + 0x1p-15f * fmaxf(fabsf(top.a1), fabsf(top.a2)) + 0x1p-126f;
+        sure[rt] = top.a2 < top.a1 - bound && bsafe && msafe[rt];
+      }
+      // lane pair (pr, hf): row wr0 + pr = 16 rt + c with rt = pr >> 4 -- this lane's c matches
+      const int prt = pr >> 4;
+      const int myidx = prt ? widx[1] : widx[0];
+      const bool row_ok = pin && (prt ? lim[1] : lim[0]) > 0;
+      const bool mysure = row_ok && (prt ? sure[1] : sure[0]);
+      double half = 0.0;
+      if (mysure) {
+#pragma unroll
+        for (int j = 0; j < HF / 4; ++j) {
+          if (4 * j < h) {
+            const uint4 kw = keys[Rows::at(myidx, hf * (h / 4) + j)];
+            const uint32_t ks[4] = {kw.x, kw.y, kw.z, kw.w};
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+              float qv = qh[4 * j + u];
+              asm volatile("" : "+v"(qv));  // converted here: hoisted out of the block loop, 64 doubles spill
+              half = fma(static_cast<double>(qv), static_cast<double>(__uint_as_float(ks[u])), half);
             }
           }
         }
       }
+      const double dot = add_halves(half);
+      if (mysure && hf == 0) {
+        const int64_t out = (r0 + prow) * NB + cur.b;
+        scores[out] = public_score(dot, fscale);
+        if (tie) tie[out] = myidx + 1;
+      }
+      if (row_ok && !mysure && hf == 0) {  // marked for score_fwd_resolve
+        const int64_t bit = static_cast<int64_t>(cur.b) * rows_pad + r0 + prow;
+        atomicOr(amb + (bit >> 5), 1u << (bit & 31));
+      }
+    }
+    cur = next_block(cu, nseq, cur, r0, nr, G, B);
+    if (--todo <= 0) cur.s = nseq;
+  }
+  fill_future(cu, nseq, r0 + wr0, nr - wr0, G, NB, B, scores, tie);
+}
+// exact_dot (two sequential FMA chains over the halves of the index dim) with 4-element loads:
+// n % 8 == 0, rows aligned for them.
+template <int DT>
+__device__ __forceinline__ double exact_dot_wide(const void* __restrict__ a, int64_t ia, const void* __restrict__ b,
+                                                 int64_t ib, int n) {
+  const int h = n / 2;
+  auto load4 = [](const void* base, int64_t i, float (&x)[4]) {
+    if constexpr (DT == kF32) {
+      const float4 w = *reinterpret_cast<const float4*>(static_cast<const float*>(base) + i);
+      x[0] = w.x, x[1] = w.y, x[2] = w.z, x[3] = w.w;
+    } else {
+      const uint2 w = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(base) + i);
+      x[0] = lo16_f32<DT>(w.x), x[1] = hi16_f32<DT>(w.x), x[2] = lo16_f32<DT>(w.y), x[3] = hi16_f32<DT>(w.y);
+    }
+  };
+  double s0 = 0.0, s1 = 0.0;
+  for (int d = 0; d < h; d += 4) {
+    float a0[4], b0[4], a1[4], b1[4];
+    load4(a, ia + d, a0);
+    load4(b, ib + d, b0);
+    load4(a, ia + h + d, a1);
+    load4(b, ib + h + d, b1);
 #pragma unroll
-      for (int p = 0; p < P; ++p) {
-        if (p < np) {
-          const int64_t row = c0 + list[w0 + p];
-          const int vis = static_cast<int>((row / G + 1 < k0 + nk ? row / G + 1 : k0 + nk) - k0);
-          const double v0 = lane < vis ? acc[0][0][p] + acc[0][1][p] : -__builtin_inf();
-          const double v1 = lane + 64 < vis ? acc[1][0][p] + acc[1][1][p] : -__builtin_inf();
-          const double wbest = wave_max_f64(fmax(v0, v1));
-          // visible keys only: with NaN dots (skipped by the maximum) wbest may be -inf, the value
-          // of the masked lanes; a row without any non-NaN visible dot gets count 0 (code 0)
-          const uint64_t m0 = __ballot(lane < vis && v0 == wbest), m1 = __ballot(lane + 64 < vis && v1 == wbest);
-          if (lane == 0) {
-            const int count = __popcll(m0) + __popcll(m1);
-            const int first = m0 ? __builtin_ctzll(m0) : 64 + __builtin_ctzll(m1);
-            const int64_t out = row * NB + b;
-            scores[out] = public_score(wbest, static_cast<float>(fabs(scale)));
-            if (tie) tie[out] = count == 1 ? first + 1 : -count;
-          }
+    for (int u = 0; u < 4; ++u) {
+      s0 = fma(static_cast<double>(a0[u]), static_cast<double>(b0[u]), s0);
+      s1 = fma(static_cast<double>(a1[u]), static_cast<double>(b1[u]), s1);
+    }
+  }
+  return s0 + s1;
+}
+
+// Monotone map of a double that is not NaN onto uint64 (+0 and -0 collapse; never 0), and back.
+__device__ __forceinline__ uint64_t ordered_f64(double x) {
+  const uint64_t u = static_cast<uint64_t>(__double_as_longlong(x + 0.0));
+  return (u >> 63) ? ~u : (u | (uint64_t(1) << 63));
+}
+__device__ __forceinline__ double from_ordered_f64(uint64_t k) {
+  return __longlong_as_double(static_cast<long long>((k >> 63) ? (k & ~(uint64_t(1) << 63)) : ~k));
+}
+
+// The ambiguous (row, block) pairs the main pass marked, settled exactly. One wave per block
+// and kResolveRows rows: it lists the marked rows in order and takes up to 16 of them (of one
+// sequence) at a time. Their MFMA logits against the block are formed again, operands
+// straight from memory; the keys within the error bound of a row's maximum (all visible keys
+// where the row or the block is not safe) are its candidates, two or three of 128 for most
+// rows. The candidates of the 16 rows are spread over the lanes, one exact_dot each; the
+// maximum, its count and the first winner come from integer LDS atomics, so the result does
+// not depend on their order. (Re-evaluating every key of the block in FP64 took 133 us at
+// 32 768 tokens x 4 groups in bf16, this pass 54 us.)
+constexpr int kResolveGroup = 16;
+template <int DT>
+__global__ __launch_bounds__(64) void score_fwd_resolve(const void* __restrict__ iq, const void* __restrict__ ik,
+                                                        const int32_t* __restrict__ cu, int nseq, int64_t rows_pad,
+                                                        int G, int Di, int NB, int B, double scale,
+                                                        const float* __restrict__ bnorm,
+                                                        const uint32_t* __restrict__ amb, float* __restrict__ scores,
+                                                        int32_t* __restrict__ tie) {
+  constexpr int NK = 4;  // Di <= 128
+  __shared__ uint16_t list[kResolveRows];
+  __shared__ uint16_t cand[kResolveGroup * 128];  // row of the group << 7 | key
+  __shared__ uint64_t best[kResolveGroup];
+  __shared__ int count[kResolveGroup], first[kResolveGroup];
+  const int lane = threadIdx.x, c = lane & 15, q4 = lane >> 4;
+  const int b = blockIdx.x;
+  const int64_t c0 = static_cast<int64_t>(blockIdx.y) * kResolveRows;
+  static_assert(kResolveRows == 64 * 64, "one 64-bit bitmap word per lane");
+  const uint32_t* words = amb + (static_cast<int64_t>(b) * rows_pad + c0) / 32 + 2 * lane;
+  uint64_t mine = (static_cast<uint64_t>(words[1]) << 32) | words[0];
+  auto scan = [&](int x) {  // inclusive prefix over the lanes
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(x, o, kWave);
+      if (lane >= o) x += y;
+    }
+    return x;
+  };
+  {
+    const int own = __popcll(mine), incl = scan(own);
+    int o = incl - own;
+    for (; mine; mine &= mine - 1) list[o++] = static_cast<uint16_t>(64 * lane + __builtin_ctzll(mine));
+    count[0] = __shfl(incl, 63, kWave);
+  }
+  __syncthreads();
+  const int n = __builtin_amdgcn_readfirstlane(count[0]);
+  const bool neg = scale < 0.0;
+  for (int i = 0; i < n;) {
+    const int64_t row0 = c0 + __builtin_amdgcn_readfirstlane(list[i]);
+    const int s = find_seq(cu, nseq, row0 / G);
+    const int64_t start = cu[s], end = cu[s + 1];
+    const int64_t end_row = end * G - c0;  // chunk-relative end of the sequence's rows
+    const int m = __popcll(__ballot(lane < kResolveGroup && i + lane < n && list[min(i + lane, n - 1)] < end_row));
+    const int64_t k0 = start + static_cast<int64_t>(b) * B;
+    const int nk = static_cast<int>((k0 + B < end ? k0 + B : end) - k0);  // >= 1: a listed row sees block b
+    const int64_t row = c0 + list[c < m ? i + c : i];
+    const int64_t vis = row / G + 1 - k0;
+    const int lim = c < m ? static_cast<int>(vis < nk ? vis : nk) : 0;
+    // ---- approximate logits S[row c][key 16 kt + 4 q4 + i]
+    float n2 = 0.f;
+    bool safe = true;
+    f32x4 acc[8];
+#pragma unroll
+    for (int kt = 0; kt < 8; ++kt) acc[kt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kk = 0; kk < NK; ++kk) {
+      if (32 * kk < Di) {
+        const int d0 = 32 * kk + 8 * q4;
+        const bool in = d0 < Di;
+        Words8<DT> qw = load_words<DT>(iq, row * Di + (in ? d0 : 0));
+#pragma unroll
+        for (int u = 0; u < Words8<DT>::N; ++u) {
+          qw.w[u] = in ? qw.w[u] : 0u;
+          add_square<DT>(qw.w[u], n2, safe);
+          qw.w[u] ^= neg ? (DT == kF32 ? 0x80000000u : 0x80008000u) : 0u;
+        }
+        Words8<DT> kw[8];
+#pragma unroll
+        for (int kt = 0; kt < 8; ++kt) {
+          const int key = 16 * kt + c < nk ? 16 * kt + c : nk - 1;
+          kw[kt] = load_words<DT>(ik, (k0 + key) * Di + (in ? d0 : 0));
+        }
+        if constexpr (DT == kF32) {
+          const SplitFrag qf = split_frag(qw.w);
+#pragma unroll
+          for (int kt = 0; kt < 8; ++kt) acc[kt] = mfma_split(split_frag(kw[kt].w), qf, acc[kt]);
+        } else {
+          const bf16x8 qf = __builtin_bit_cast(bf16x8, make_uint4(qw.w[0], qw.w[1], qw.w[2], qw.w[3]));
+#pragma unroll
+          for (int kt = 0; kt < 8; ++kt)
+            acc[kt] = mfma_t<DT>(
+                __builtin_bit_cast(bf16x8, make_uint4(kw[kt].w[0], kw[kt].w[1], kw[kt].w[2], kw[kt].w[3])), qf,
+                acc[kt]);
         }
       }
-      __builtin_amdgcn_wave_barrier();  // qs is rewritten by the next window
     }
-    __syncthreads();  // the block's readers are done before the next run restages it
-    i = j;
+    // ---- candidates of each row
+    float mx = -__builtin_inff();
+#pragma unroll
+    for (int kt = 0; kt < 8; ++kt)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (16 * kt + 4 * q4 + j < lim) mx = fmaxf(mx, acc[kt][j]);
+#pragma unroll
+    for (int o = 16; o <= 32; o <<= 1) {
+      mx = fmaxf(mx, __shfl_xor(mx, o, kWave));
+      n2 += __shfl_xor(n2, o, kWave);
+      safe = __shfl_xor(static_cast<int>(safe), o, kWave) != 0 && safe;
+    }
+    const float bn = bnorm[k0];
+    safe = safe && !__builtin_signbit(bn);
+    const float bound = 2.f * logit_error<DT, 32 * NK>() * (sqrtf(n2) * 1.0001f) * fabsf(bn) +
+                        0x1p-20f * fabsf(mx) + 0x1p-126f;
+    uint32_t cm = 0u;
+#pragma unroll
+    for (int kt = 0; kt < 8; ++kt)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (16 * kt + 4 * q4 + j < lim && (!safe || !(acc[kt][j] < mx - bound))) cm |= 1u << (4 * kt + j);
+    const int own = __popc(cm), incl = scan(own);
+    const int total = __shfl(incl, 63, kWave);
+    int o = incl - own;
+    for (; cm; cm &= cm - 1) {
+      const int p = __builtin_ctz(cm);
+      cand[o++] = static_cast<uint16_t>(c << 7 | (16 * (p >> 2) + 4 * q4 + (p & 3)));
+    }
+    if (lane < kResolveGroup) {
+      best[lane] = 0u;
+      count[lane] = 0;
+      first[lane] = 0x7fffffff;
+    }
+    __syncthreads();
+    // ---- their exact dots (NaN dots are skipped; a row without any other visible dot keeps count 0)
+    auto value = [&](int e) -> uint64_t {
+      const int x = cand[e], key = x & 127;
+      double v = exact_dot_wide<DT>(iq, (c0 + list[i + (x >> 7)]) * Di, ik, (k0 + key) * Di, Di);
+      v = neg ? -v : v;
+      return v == v ? ordered_f64(v) : 0u;
+    };
+    uint64_t v0 = 0u;
+    for (int e = lane; e < total; e += kWave) {
+      const uint64_t v = value(e);
+      if (e == lane) v0 = v;
+      if (v) atomicMax(reinterpret_cast<unsigned long long*>(&best[cand[e] >> 7]), static_cast<unsigned long long>(v));
+    }
+    __syncthreads();
+    for (int e = lane; e < total; e += kWave) {
+      const uint64_t v = e == lane ? v0 : value(e);
+      const int g = cand[e] >> 7;
+      if (v && v == best[g]) {
+        atomicAdd(&count[g], 1);
+        atomicMin(&first[g], cand[e] & 127);
+      }
+    }
+    __syncthreads();
+    if (lane < m) {
+      const int k = count[lane];
+      const int64_t out = row * NB + b;  // lane < m: row is row `lane` of the group
+      scores[out] = public_score(k ? from_ordered_f64(best[lane]) : -__builtin_inf(), static_cast<float>(fabs(scale)));
+      if (tie) tie[out] = k == 1 ? first[lane] + 1 : -k;
+    }
+    __syncthreads();  // the lists are rewritten by the next group
+    i += m;
   }
 }
 
@@ -695,12 +1142,28 @@ int64_t score_fwd_mfma_workspace_bytes(int64_t total_tokens, int64_t rows, int64
   return ws_bitmap_offset(total_tokens) + 4 * bitmap_words(rows, NB);
 }
 
-int score_fwd_mfma_launch(const void* iq, const void* ik, const int32_t* cu, int nseq, int64_t rows, int G, int Di,
-                          int NB, int B, double scale, float* scores, int32_t* tie, void* ws, hipStream_t st) {
-  if (!ws) return kErrInvalidArgument;
-  const dim3 grid(grid_1d(rows, kTileRows)), block(kThreads);
-  const auto* q = static_cast<const uint16_t*>(iq);
-  const auto* k = static_cast<const uint16_t*>(ik);
+// Workgroups per row tile, each taking an equal run of the tile's key blocks. A tile's work
+// grows with its position in the sequence, so with one workgroup per tile the chip waits for
+// the heaviest ones unless there are many tiles per CU. A part costs its rows' set-up:
+// enough parts for 2048 workgroups while a part keeps about 16 blocks, and for 512 (two per
+// CU) while it keeps 2. Measured, us per selection with 1 / 2 / 4 / 8 parts: 256 tiles of up
+// to 64 blocks 243 / 179 / 154 / 162; with 1 / 2 / 4 parts: 1024 tiles of up to 256 blocks
+// 1275 / 1216 / 1246, 512 tiles of up to 48 blocks (score forward and backward) 472 / 437 / 450.
+static unsigned tile_parts(int64_t rows, int64_t NB) {
+  const int64_t tiles = (rows + kTileRows - 1) / kTileRows;
+  auto parts = [&](int64_t workgroups, int64_t blocks) {
+    const int64_t p = (workgroups + tiles - 1) / tiles, most = NB / blocks;
+    return p < most ? p : most;
+  };
+  const int64_t many = parts(2048, 16), fill = parts(512, 2);
+  const int64_t p = many > fill ? many : fill;
+  return static_cast<unsigned>(p < 1 ? 1 : p);
+}
+
+template <int DT>
+static int launch(const void* iq, const void* ik, const int32_t* cu, int nseq, int64_t rows, int G, int Di, int NB,
+                  int B, double scale, float* scores, int32_t* tie, void* ws, hipStream_t st) {
+  const dim3 grid(grid_1d(rows, kTileRows), tile_parts(rows, NB)), block(kThreads);
   const int64_t T = rows / G;
   char* wsb = static_cast<char*>(ws);
   float* knorm2 = reinterpret_cast<float*>(wsb);
@@ -708,19 +1171,39 @@ int score_fwd_mfma_launch(const void* iq, const void* ik, const int32_t* cu, int
   auto* amb = reinterpret_cast<uint32_t*>(wsb + ws_bitmap_offset(T));
   const int64_t words = bitmap_words(rows, NB);
   const int64_t rows_pad = rows_padded(rows);
-  hipLaunchKernelGGL(score_key_norms, dim3(grid_1d(T > words ? T : words, 256)), dim3(256), 0, st, k, T, Di,
-                     knorm2, amb, words);
-  hipLaunchKernelGGL(score_block_norms, dim3(grid_1d(T, 256)), dim3(256), 0, st, knorm2, cu, nseq, T, B, bnorm);
-#define MSA_SCORE_MFMA(NKV, FD) hipLaunchKernelGGL((score_fwd_mfma_kernel<NKV, FD>), grid, block, 0, st, q, k, cu, nseq, rows, G, Di, NB, B, scale, bnorm, amb, rows_pad, scores, tie)
+  if (B >= 64) {
+    const unsigned ng = grid_1d(T, 64), wg = grid_1d(words, 256);
+    hipLaunchKernelGGL(score_block_norms<DT>, dim3(ng > wg ? ng : wg), dim3(256), 0, st, ik, cu, nseq, T, Di, B, bnorm, amb, words);
+  } else {
+    hipLaunchKernelGGL(score_key_norms<DT>, dim3(grid_1d(T > words ? T : words, 256)), dim3(256), 0, st, ik, T, Di, knorm2, amb, words);
+    hipLaunchKernelGGL(score_small_block_norms, dim3(grid_1d(T, 256)), dim3(256), 0, st, knorm2, cu, nseq, T, B, bnorm);
+  }
   const int nk = Di <= 32 ? 1 : (Di <= 64 ? 2 : 4);
-  const bool fd = Di == 32 * nk;
-  if (nk == 1) { if (fd) MSA_SCORE_MFMA(1, true); else MSA_SCORE_MFMA(1, false); }
-  else if (nk == 2) { if (fd) MSA_SCORE_MFMA(2, true); else MSA_SCORE_MFMA(2, false); }
-  else { if (fd) MSA_SCORE_MFMA(4, true); else MSA_SCORE_MFMA(4, false); }
+  if constexpr (DT == kF32) {
+#define MSA_SCORE_F32(NKV) hipLaunchKernelGGL(score_fwd_f32_kernel<NKV>, grid, block, 0, st, static_cast<const float*>(iq), static_cast<const float*>(ik), cu, nseq, rows, G, Di, NB, B, scale, bnorm, amb, rows_pad, scores, tie)
+    if (nk == 1) MSA_SCORE_F32(1); else if (nk == 2) MSA_SCORE_F32(2); else MSA_SCORE_F32(4);
+#undef MSA_SCORE_F32
+  } else {
+#define MSA_SCORE_MFMA(NKV, FD) hipLaunchKernelGGL((score_fwd_mfma_kernel<DT, NKV, FD>), grid, block, 0, st, static_cast<const uint16_t*>(iq), static_cast<const uint16_t*>(ik), cu, nseq, rows, G, Di, NB, B, scale, bnorm, amb, rows_pad, scores, tie)
+    const bool fd = Di == 32 * nk;
+    if (nk == 1) { if (fd) MSA_SCORE_MFMA(1, true); else MSA_SCORE_MFMA(1, false); }
+    else if (nk == 2) { if (fd) MSA_SCORE_MFMA(2, true); else MSA_SCORE_MFMA(2, false); }
+    else { if (fd) MSA_SCORE_MFMA(4, true); else MSA_SCORE_MFMA(4, false); }
 #undef MSA_SCORE_MFMA
-  hipLaunchKernelGGL(score_fwd_resolve, dim3(NB, static_cast<unsigned>(rows_pad / kResolveRows)), dim3(256), 0, st,
-                     q, k, cu, nseq, rows, rows_pad, G, Di, NB, B, scale, amb, scores, tie);
+  }
+  hipLaunchKernelGGL(score_fwd_resolve<DT>, dim3(NB, static_cast<unsigned>(rows_pad / kResolveRows)), dim3(64), 0, st,
+                     iq, ik, cu, nseq, rows_pad, G, Di, NB, B, scale, bnorm, amb, scores, tie);
   return status_from(hipGetLastError());
+}
+
+int score_fwd_mfma_launch(int dt, const void* iq, const void* ik, const int32_t* cu, int nseq, int64_t rows, int G,
+                          int Di, int NB, int B, double scale, float* scores, int32_t* tie, void* ws, hipStream_t st) {
+  if (!ws) return kErrInvalidArgument;
+  switch (dt) {
+    case kF32: return launch<kF32>(iq, ik, cu, nseq, rows, G, Di, NB, B, scale, scores, tie, ws, st);
+    case kF16: return launch<kF16>(iq, ik, cu, nseq, rows, G, Di, NB, B, scale, scores, tie, ws, st);
+    default: return launch<kBF16>(iq, ik, cu, nseq, rows, G, Di, NB, B, scale, scores, tie, ws, st);
+  }
 }
 
 }  // namespace msa

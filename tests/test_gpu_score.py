@@ -299,3 +299,63 @@ def test_score_index_dims_beyond_512(dim, dtype, device):
     nb = (max(lengths) + block - 1) // block
     upstream = torch.randn((sum(lengths), groups, nb), generator=gen).to(torch.bfloat16).float()
     _run(q_cpu, k_cpu, lengths, max(lengths), block, 1.0, upstream, device)
+
+
+def _forward_on_both_paths(q_cpu, k_cpu, lengths, block, scale, device):
+    """(scores, tie codes) of the MFMA path and of the exact kernel, which takes the same
+    values when their rows do not start on 16-byte boundaries."""
+    from msa_triton_amd.index_score import _score_forward
+    from msa_triton_amd.layout import sequence_meta
+
+    def shifted(x):  # the same values, one element past a 16-byte boundary
+        flat = torch.empty(x.numel() + 1, dtype=x.dtype, device=device)
+        flat[1:] = x.to(device).flatten()
+        y = flat[1:].view(x.shape)
+        assert y.is_contiguous() and y.data_ptr() % 16
+        return y
+
+    cu = cu_tensor(lengths, device)
+    meta = sequence_meta(cu_list(lengths), block)
+    out = []
+    for place in (lambda x: x.to(device), shifted):
+        sc, tie = _score_forward(place(q_cpu), place(k_cpu), cu, meta, max(lengths) + 3 * block, block, scale, True)
+        out.append((sc.cpu().numpy(), tie.cpu().numpy()))
+    return out
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("lengths,groups,dim,block,scale", [
+    ([1], 1, 8, 128, 1.0), ([127, 0, 130], 2, 40, 128, -1.0), ([300, 1, 777], 3, 96, 64, 0.3),
+    ([129, 255], 2, 128, 7, 1.0), ([700, 333], 2, 128, 128, -0.75), ([1500], 1, 64, 100, 1.0),
+    ([513, 90], 4, 32, 33, 2.0),
+])
+@pytest.mark.parametrize("values", ["normal", "integer", "range"])
+def test_score_mfma_path_equals_the_exact_kernel(values, lengths, groups, dim, block, scale, dtype, device):
+    """fp16 and fp32 on the MFMA path against the exact kernel, bit for bit (scores and tie
+    codes): random values, small integers (exact ties) and magnitudes over the whole range of
+    the type (fp16 subnormals; fp32 elements beyond the range whose products the bf16 terms
+    hold, infinities and NaN)."""
+    gen = torch.Generator().manual_seed(dim + block + len(values))
+    total = sum(lengths)
+    if values == "integer":
+        q = torch.randint(-2, 3, (total, groups, dim), generator=gen).to(dtype)
+        k = torch.randint(-2, 3, (total, 1, dim), generator=gen).to(dtype)
+    else:
+        q = torch.randn(total, groups, dim, generator=gen)
+        k = torch.randn(total, 1, dim, generator=gen)
+        if values == "range":
+            low = -24.0 if dtype == torch.float16 else -100.0
+            q[: total // 3] *= 2.0 ** (low * torch.rand(total // 3, 1, 1, generator=gen))
+            k[total // 2:] *= 2.0 ** (low * torch.rand(total - total // 2, 1, dim, generator=gen))
+            k[:: 97, 0, 3] = 60000.0 if dtype == torch.float16 else 2.0 ** 90
+            k[5:: 211, 0, 1] = float("nan")
+            q[7:: 301, 0, 0] = float("inf")
+        q, k = q.to(dtype), k.to(dtype)
+    mfma, exact = _forward_on_both_paths(q, k, lengths, block, scale, device)
+    np.testing.assert_array_equal(mfma[0], exact[0])
+    np.testing.assert_array_equal(mfma[1], exact[1])
+    if values != "range":
+        _, exp32, exp_tie = O.index_score(q.double().numpy(), k.double().numpy(), cu_list(lengths),
+                                          max(lengths) + 3 * block, block_size=block, scale=scale)
+        np.testing.assert_array_equal(mfma[0], exp32)
+        np.testing.assert_array_equal(mfma[1], exp_tie)
