@@ -354,7 +354,7 @@ __global__ __launch_bounds__(256) void score_bwd_dq_wide(const void* __restrict_
   }
 }
 
-// dk, partial sums. One workgroup per (key block gb, segment of kDkSeg rows, chunk of
+// dk, partial sums. One workgroup per (key block gb, segment of SEG rows, chunk of
 // 128 keys). The segment's rows (t, g) of gb's sequence with t >= block start are
 // read once (block-major tie / ds) and bucketed by their unique winner with a stable
 // counting sort in LDS (per 64-row wave step the rank among equal winners comes from
@@ -375,7 +375,19 @@ __device__ __forceinline__ void dk_add_row(double (&acc)[8], double wgt, const v
   }
 }
 
-constexpr int kDkSeg = 8192;
+// Rows per segment: 8192 (long sequences: every key block has many segments), or 2048 where
+// that leaves the chip short of workgroups, as long as the FP64 partial sums stay at 4096
+// (block, segment) pairs. Measured (score backward's dk pass and reduction, Di = 128, 4 groups):
+// sequences of 2048 to 6144 tokens, 128 blocks: 183 + 13 us with 8192 rows, 126 + 16 us with 2048
+// (eight waves per workgroup instead of four: 133 + 16).
+constexpr int kDkSegLong = 8192, kDkSegShort = 2048;
+static int dk_seg(int64_t rows, int64_t total_blocks) {
+  return total_blocks * ((rows + kDkSegShort - 1) / kDkSegShort) <= 4096 ? kDkSegShort : kDkSegLong;
+}
+static int64_t dk_nseg(int64_t rows, int64_t total_blocks) {
+  const int64_t seg = dk_seg(rows, total_blocks);
+  return (rows + seg - 1) / seg;
+}
 constexpr int kDkBatch = 16;
 constexpr int kDkWideUnroll = 4;  // row-gather instructions per batch (4 rows each; two batches in flight)
 // Listed exact ties per segment (a segment with more rescans its rows per key). With 4-instruction
@@ -383,23 +395,24 @@ constexpr int kDkWideUnroll = 4;  // row-gather instructions per batch (4 rows e
 // at c4 1.13-1.17 vs 1.21-1.24 ms for the score backward with two (8-instruction batches).
 constexpr int kDkTieCap = 64;
 
-template <int DT, int DPL>
-__global__ __launch_bounds__(256, DPL >= 8 ? 2 : 3) void score_bwd_dk_part(
+template <int DT, int DPL, int SEG>
+__global__ __launch_bounds__(256, DPL >= 8 ? 2 : (SEG == kDkSegShort ? 4 : 3)) void score_bwd_dk_part(
     const void* __restrict__ iq, const void* __restrict__ ik, const int32_t* __restrict__ cu,
     const int32_t* __restrict__ cu_blocks, int nseq, const int32_t* __restrict__ tie_t,
     const float* __restrict__ ds_t, int64_t rows, int G, int Di, int B, int64_t nblk, int nseg, double scale,
     double* __restrict__ part, int dc0) {
-  __shared__ uint16_t lrow[kDkSeg];   // bucketed row offsets (within the segment)
-  __shared__ float lds_w[kDkSeg];     // their ds
+  __shared__ uint16_t lrow[SEG];   // bucketed row offsets (within the segment)
+  __shared__ float lds_w[SEG];     // their ds
   __shared__ int32_t cnt[128], bstart[128];
-  __shared__ int32_t wcnt[4][128];
+  constexpr int NW = 4;  // waves
+  __shared__ int32_t wcnt[NW][128];
   __shared__ int32_t tie_row[kDkTieCap];
   __shared__ double tie_best[kDkTieCap];
   __shared__ int32_t tie_count[kDkTieCap];
   __shared__ int32_t ntie_s;
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  // Segments are aligned to multiples of kDkSeg in the row space: key block gb takes segment
-  // S0 + sg, S0 = (its first row) / kDkSeg, clipped to its rows. Work L = workgroup index,
+  // Segments are aligned to multiples of SEG in the row space: key block gb takes segment
+  // S0 + sg, S0 = (its first row) / SEG, clipped to its rows. Work L = workgroup index,
   // S-major over (S, key block): the workgroups running together gather from the same one or
   // two 2 MiB segments of index_q. Workgroups go to the 8 XCDs round-robin, so consecutive
   // pairs run on different XCDs (contiguous runs of L per XCD would load them unevenly: the
@@ -415,25 +428,25 @@ __global__ __launch_bounds__(256, DPL >= 8 ? 2 : 3) void score_bwd_dk_part(
   const int b = static_cast<int>(gb - cu_blocks[s]);
   const int64_t start = cu[s], end = cu[s + 1];
   const int64_t k0 = start + static_cast<int64_t>(b) * B;
-  const int64_t S0 = k0 * G / kDkSeg;
+  const int64_t S0 = k0 * G / SEG;
   if (S < S0) return;  // whole workgroup: the block starts after this segment
   const int sg = static_cast<int>(S - S0);
   const int64_t w = gb * nseg + sg;  // (gb, sg): index of this pair's partial sums
-  const int64_t r_begin = S == S0 ? k0 * G : S * kDkSeg;
-  const int64_t r_stop = (S + 1) * kDkSeg < end * G ? (S + 1) * kDkSeg : end * G;
+  const int64_t r_begin = S == S0 ? k0 * G : S * SEG;
+  const int64_t r_stop = (S + 1) * SEG < end * G ? (S + 1) * SEG : end * G;
   if (r_begin >= r_stop) return;  // whole workgroup: empty segment (the reduce skips it)
   const int o_lo = 128 * kc;      // this chunk's first key offset in the block
   const int nseg_rows = static_cast<int>(r_stop - r_begin);
   const int32_t* tcol = tie_t + static_cast<int64_t>(b) * rows + r_begin;
   const float* dcol = ds_t + static_cast<int64_t>(b) * rows + r_begin;
-  // Stable counting sort by winner, one quarter of the segment per wave: wave w takes rows
+  // Stable counting sort by winner, an equal run of the segment per wave: wave w takes rows
   // kWaveRows w .. kWaveRows (w + 1) - 1 (row kWaveRows w + 64 r + lane in round r) and owns
   // the slice of every key's bucket after the slices of waves 0 .. w - 1. Each wave ranks its
   // rounds with ballots and advances its own counters, so the rounds need no workgroup
   // barrier, and every bucket still lists its rows in row order.
-  constexpr int kWaveRows = kDkSeg / 4;
+  constexpr int kWaveRows = SEG / NW;
   constexpr int kRounds = kWaveRows / 64;
-  if (tid < 128) wcnt[0][tid] = wcnt[1][tid] = wcnt[2][tid] = wcnt[3][tid] = 0;
+  for (int i = tid; i < NW * 128; i += 64 * NW) wcnt[i >> 7][i & 127] = 0;
   if (tid == 0) ntie_s = 0;
   // the wave's tie codes and ds, round r in register r: all loads in flight at once
   int32_t tcs[kRounds];
@@ -458,7 +471,12 @@ __global__ __launch_bounds__(256, DPL >= 8 ? 2 : 3) void score_bwd_dk_part(
     }
   }
   __syncthreads();
-  if (tid < 128) cnt[tid] = wcnt[0][tid] + wcnt[1][tid] + wcnt[2][tid] + wcnt[3][tid];
+  if (tid < 128) {
+    int n = 0;
+#pragma unroll
+    for (int w2 = 0; w2 < NW; ++w2) n += wcnt[w2][tid];
+    cnt[tid] = n;
+  }
   __syncthreads();
   if (tid < 64) {  // exclusive scan of the 128 bucket counts (two per lane)
     const int a0 = cnt[2 * tid], a1 = cnt[2 * tid + 1];
@@ -475,7 +493,7 @@ __global__ __launch_bounds__(256, DPL >= 8 ? 2 : 3) void score_bwd_dk_part(
   if (tid < 128) {  // each wave's next free position in each bucket
     int p = bstart[tid];
 #pragma unroll
-    for (int w2 = 0; w2 < 4; ++w2) {
+    for (int w2 = 0; w2 < NW; ++w2) {
       const int n = wcnt[w2][tid];
       wcnt[w2][tid] = p;
       p += n;
@@ -525,7 +543,7 @@ __global__ __launch_bounds__(256, DPL >= 8 ? 2 : 3) void score_bwd_dk_part(
     }
   }
   __syncthreads();
-  for (int x = wid; x < ntie; x += 4) {
+  for (int x = wid; x < ntie; x += NW) {
     const int64_t row = r_begin + tie_row[x];
     const int64_t t = row / G;
     const int64_t k1 = (k0 + B < t + 1) ? k0 + B : t + 1;
@@ -536,7 +554,7 @@ __global__ __launch_bounds__(256, DPL >= 8 ? 2 : 3) void score_bwd_dk_part(
     }
   }
   __syncthreads();
-  // ---- per-key sums: wave w takes keys w, w + 4, ... of this chunk
+  // ---- per-key sums: wave w takes keys w, w + NW, ... of this chunk
   const int64_t kchunk_end = k0 + B < end ? k0 + B : end;
   const int nkeys_c = static_cast<int>(kchunk_end - k0 - o_lo < 128 ? kchunk_end - k0 - o_lo : 128);
   if (wid >= nkeys_c) return;  // whole wave: no keys (no barrier follows)
@@ -586,7 +604,7 @@ __global__ __launch_bounds__(256, DPL >= 8 ? 2 : 3) void score_bwd_dk_part(
     auto next_of = [&](const Batch& x) {
       Batch y{x.o, x.e + kSpan, x.kend};
       if (y.e >= y.kend) {
-        y.o = x.o + 4;
+        y.o = x.o + NW;
         y = y.o < nkeys_c ? first_of(y.o) : Batch{y.o, 0, 0};
       }
       return Batch{__builtin_amdgcn_readfirstlane(y.o), __builtin_amdgcn_readfirstlane(y.e),
@@ -597,7 +615,7 @@ __global__ __launch_bounds__(256, DPL >= 8 ? 2 : 3) void score_bwd_dk_part(
 #pragma unroll
       for (int u = 0; u < kDkWideUnroll; ++u) {
         const int ee = x.e + u * kRpi + slot;
-        const int ec = ee < kDkSeg ? ee : kDkSeg - 1;  // always inside the list (value unused past the key)
+        const int ec = ee < SEG ? ee : SEG - 1;  // always inside the list (value unused past the key)
         const int r = lrow[ec];
         const float wv = lds_w[ec];
         const bool ok = ee < x.kend;
@@ -661,7 +679,7 @@ __global__ __launch_bounds__(256, DPL >= 8 ? 2 : 3) void score_bwd_dk_part(
   // other dtypes / dims: lanes over dims dc0 + DPL lane .. + DPL - 1 (index dims above 64 x DPL
   // take one launch per 64 DPL dims), query rows streamed kDkBatch at a time
   const int dbase = dc0 + DPL * lane;
-  for (int o = wid; o < nkeys_c; o += 4) {
+  for (int o = wid; o < nkeys_c; o += NW) {
     const int64_t key = k0 + o_lo + o;
     double acc[8];
 #pragma unroll
@@ -697,35 +715,34 @@ __global__ __launch_bounds__(256, DPL >= 8 ? 2 : 3) void score_bwd_dk_part(
   }
 }
 
-// dk[key][d] = sum over the key block's row segments (in order) of the partial sums.
+// dk[key][d] = sum over the key block's row segments (in order) of the partial sums. One wave
+// per key, lanes along its dims.
 template <int DT>
 __global__ __launch_bounds__(256) void score_bwd_dk_reduce(const int32_t* __restrict__ cu,
                                                            const int32_t* __restrict__ cu_blocks, int nseq,
-                                                           int64_t T, int G, int Di, int B, int nseg,
+                                                           int64_t T, int G, int Di, int B, int nseg, int seg,
                                                            const double* __restrict__ part,
                                                            void* __restrict__ dk) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (i >= T * Di) return;
-  const int64_t key = i / Di;
-  const int d = static_cast<int>(i % Di);
+  const int64_t key = static_cast<int64_t>(blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (key >= T) return;
   const int s = find_seq(cu, nseq, key);
   const int64_t start = cu[s], end = cu[s + 1];
-  const int b = static_cast<int>((key - start) / B);
-  const int o = static_cast<int>((key - start) % B);
-  const int64_t gb = cu_blocks[s] + b;
+  const uint32_t pos = static_cast<uint32_t>(key - start), b = pos / static_cast<uint32_t>(B);
+  const int o = static_cast<int>(pos - b * B);
+  const int64_t gb = cu_blocks[s] + static_cast<int64_t>(b);
   const int64_t k0 = start + static_cast<int64_t>(b) * B;
   const int kc = o / 128, kchunks = (B + 127) / 128;
-  const int64_t S0 = k0 * G / kDkSeg;  // the block's first segment (aligned to kDkSeg rows)
-  double sum = 0.0;
-  for (int sg = 0; sg < nseg; ++sg) {
-    if ((S0 + sg) * kDkSeg >= end * G) break;  // empty segment (nothing written)
-    const int64_t w = gb * nseg + sg;
-    sum += part[((w * kchunks + kc) * 128 + o % 128) * static_cast<int64_t>(Di) + d];
+  const int64_t S0 = k0 * G / seg;  // the block's first segment (aligned to seg rows)
+  const int64_t left = (end * G + seg - 1) / seg - S0;  // segments with rows (nothing written past them)
+  const int n = static_cast<int>(left < nseg ? left : nseg);
+  const double* src = part + ((gb * nseg * kchunks + kc) * 128 + (o - 128 * kc)) * Di;
+  for (int d = threadIdx.x & 63; d < Di; d += kWave) {
+    double sum = 0.0;
+#pragma unroll 4
+    for (int sg = 0; sg < n; ++sg) sum += src[static_cast<int64_t>(sg) * kchunks * 128 * Di + d];
+    store_from_f64<DT>(dk, key * Di + d, sum);
   }
-  store_from_f64<DT>(dk, i, sum);
 }
-
-static int64_t dk_nseg(int64_t rows) { return (rows + kDkSeg - 1) / kDkSeg; }
 
 template <int DT>
 int score_fwd_launch(const void* iq, const void* ik, const int32_t* cu, int nseq, int64_t rows, int G,
@@ -777,19 +794,22 @@ int score_bwd_launch(const void* iq, const void* ik, const int32_t* cu, const in
     double* part = reinterpret_cast<double*>(ds_t + rows * NB);  // 8 * rows * NB bytes in: 8-byte aligned
     const dim3 tgrid(grid_1d(rows, 64), static_cast<unsigned>((NB + 63) / 64));
     hipLaunchKernelGGL(score_bwd_transpose, tgrid, dim3(256), 0, st, tie, ds, rows, NB, cu, nseq, G, B, tie_t, ds_t);
-    const int nseg = static_cast<int>(dk_nseg(rows));
+    const int seg = dk_seg(rows, total_blocks), nseg = static_cast<int>(dk_nseg(rows, total_blocks));
     const int kchunks = (B + 127) / 128;
     const dim3 grid(static_cast<unsigned>(total_blocks * nseg), static_cast<unsigned>(kchunks));
-#define MSA_DK_PART(DPLV, DC0) hipLaunchKernelGGL((score_bwd_dk_part<DT, DPLV>), grid, dim3(256), 0, st, iq, ik, cu, cu_blocks, nseq, tie_t, ds_t, rows, G, Di, B, total_blocks, nseg, scale, part, DC0)
-    if (Di <= 64) MSA_DK_PART(1, 0);
-    else if (Di <= 128) MSA_DK_PART(2, 0);
-    else if (Di <= 256) MSA_DK_PART(4, 0);
+#define MSA_DK_PART_SEG(DPLV, DC0, SEGV) hipLaunchKernelGGL((score_bwd_dk_part<DT, DPLV, SEGV>), grid, dim3(256), 0, st, iq, ik, cu, cu_blocks, nseq, tie_t, ds_t, rows, G, Di, B, total_blocks, nseg, scale, part, DC0)
+#define MSA_DK_PART(DPLV, DC0) \
+  if (seg == kDkSegShort) MSA_DK_PART_SEG(DPLV, DC0, kDkSegShort); else MSA_DK_PART_SEG(DPLV, DC0, kDkSegLong)
+    if (Di <= 64) { MSA_DK_PART(1, 0); }
+    else if (Di <= 128) { MSA_DK_PART(2, 0); }
+    else if (Di <= 256) { MSA_DK_PART(4, 0); }
     else
-      for (int dc0 = 0; dc0 < Di; dc0 += 512) MSA_DK_PART(8, dc0);
+      for (int dc0 = 0; dc0 < Di; dc0 += 512) { MSA_DK_PART(8, dc0); }
 #undef MSA_DK_PART
+#undef MSA_DK_PART_SEG
     const int64_t T = rows / G;
-    hipLaunchKernelGGL(score_bwd_dk_reduce<DT>, dim3(grid_1d(T * Di, 256)), dim3(256), 0, st, cu, cu_blocks, nseq, T,
-                       G, Di, B, nseg, part, dk);
+    hipLaunchKernelGGL(score_bwd_dk_reduce<DT>, dim3(grid_1d(T, 4)), dim3(256), 0, st, cu, cu_blocks, nseq, T, G, Di, B,
+                       nseg, seg, part, dk);
   }
   return status_from(hipGetLastError());
 }
@@ -855,7 +875,7 @@ extern "C" int64_t msa_score_bwd_workspace_bytes(int64_t total_tokens, int64_t g
   const int64_t rows = total_tokens * groups;
   // block-major tie / ds copies, then the dk partial sums (FP64)
   const int64_t tr = rows * num_blocks * 8 + 8;
-  const int64_t nseg = dk_nseg(rows);
+  const int64_t nseg = dk_nseg(rows, total_blocks);
   const int64_t kchunks = (block_size + 127) / 128;
   const int64_t part = total_blocks * nseg * kchunks * 128 * index_dim * 8;
   return tr + part + 256;

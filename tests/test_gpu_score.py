@@ -359,3 +359,34 @@ def test_score_mfma_path_equals_the_exact_kernel(values, lengths, groups, dim, b
                                           max(lengths) + 3 * block, block_size=block, scale=scale)
         np.testing.assert_array_equal(mfma[0], exp32)
         np.testing.assert_array_equal(mfma[1], exp_tie)
+
+
+@pytest.mark.parametrize("dtype,dim", [(torch.bfloat16, 128), (torch.float32, 40)])
+@pytest.mark.parametrize("tokens,block", [(1023, 64), (1025, 128), (2600, 1)])
+def test_score_backward_row_segments(tokens, block, dtype, dim, device):
+    """The key-block pass at the edges of its 2048-row segments (two groups: 1024 tokens) and,
+    with blocks of one key, with more (block, segment) pairs than the short segments are used
+    for: gradients against the float64 sums over the winners."""
+    gen = torch.Generator().manual_seed(tokens)
+    lengths, groups = [tokens, 70], 2
+    total, nb = tokens + 70, -(-tokens // block)
+    q = torch.randn(total, groups, dim, generator=gen).to(dtype).to(device).requires_grad_()
+    k = torch.randn(total, 1, dim, generator=gen).to(dtype).to(device).requires_grad_()
+    scores = msa.m3_index_score(q, k, cu_tensor(lengths, device), tokens, block_size=block)
+    ds = torch.randn((total, groups, nb), generator=gen).to(device)
+    scores.backward(ds)
+    dq, dk = torch.zeros_like(q, dtype=torch.float64), torch.zeros(total, dim, dtype=torch.float64, device=device)
+    for a, b in ((0, tokens), (tokens, total)):
+        n, m = b - a, -(-(b - a) // block)
+        s = (q[a:b].detach().double().reshape(-1, dim) @ k[a:b, 0].detach().double().T).view(n, groups, n)
+        s = s.masked_fill(torch.ones(n, n, dtype=torch.bool, device=device).triu(1)[:, None], float("-inf"))
+        s = torch.nn.functional.pad(s, (0, m * block - n), value=float("-inf")).view(n, groups, m, block)
+        v, at = s.max(dim=3)
+        w = torch.zeros_like(s).scatter_(3, at[..., None], (ds[a:b, :, :m].double() * torch.isfinite(v))[..., None])
+        w = w.view(n * groups, m * block)[:, :n]
+        dq[a:b] = (w @ k[a:b, 0].detach().double()).view(n, groups, dim)
+        dk[a:b] = w.T @ q[a:b].detach().double().reshape(-1, dim)
+    # one rounding to the output type (2^-9 / 2^-25 of a value), from FP64 sums
+    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -23
+    assert bool(((q.grad.double() - dq).abs() <= eps * dq.abs() + 1e-12).all())
+    assert bool(((k.grad[:, 0].double() - dk).abs() <= eps * dk.abs() + 1e-12).all())
