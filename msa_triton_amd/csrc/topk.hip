@@ -29,6 +29,19 @@ __global__ __launch_bounds__(256) void topk_kernel(const float* __restrict__ sco
                   static_cast<int64_t>(gridDim.x - 1 - blockIdx.x) * 16 + (threadIdx.x >> 4), threadIdx.x & 15);
 }
 
+// Threshold and sort, 64 / CAP rows per wavefront: topk_threshold.
+template <int VPL, int CAP>
+__global__ __launch_bounds__(256) void topk_select_kernel(const float* __restrict__ scores,
+                                                          const int32_t* __restrict__ cu, int nseq, int64_t rows,
+                                                          int G, int NB, int B, int K, int L,
+                                                          int32_t* __restrict__ out) {
+  __shared__ uint2 cand[4][64];
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t wave = static_cast<int64_t>(gridDim.x - 1 - blockIdx.x) * 4 + wid;
+  if (wave * (64 / CAP) >= rows) return;
+  topk_threshold<VPL, CAP>(scores, cu, nseq, rows, G, NB, B, K, L, out, wave, threadIdx.x & 63, cand[wid]);
+}
+
 // One wavefront per row for long rows (more than 1024 blocks): topk_row64.
 template <int VPL>
 __global__ __launch_bounds__(256) void topk_wave_kernel(const float* __restrict__ scores,
@@ -64,9 +77,20 @@ int topk_launch(const float* scores, const int32_t* cu_seqlens, int nseq, int64_
   hipLaunchKernelGGL(topk_kernel<V>, grid, block, 0, st, scores, cu_seqlens, nseq, rows, G, NB, B, K, L, indices)
 #define MSA_TOPK_WAVE(V) \
   hipLaunchKernelGGL(topk_wave_kernel<V>, dim3(grid_1d(rows, 4)), block, 0, st, scores, cu_seqlens, nseq, rows, G, NB, B, K, L, indices)
+#define MSA_TOPK_SELECT(V)                                                                                              \
+  if (K <= kSelectPairSlots)                                                                                          \
+    hipLaunchKernelGGL((topk_select_kernel<V, 32>), dim3(grid_1d(rows, 8)), block, 0, st, scores, cu_seqlens, nseq, rows, G, NB, B, K, L, indices); \
+  else                                                                                                                \
+    hipLaunchKernelGGL((topk_select_kernel<V, 64>), dim3(grid_1d(rows, 4)), block, 0, st, scores, cu_seqlens, nseq, rows, G, NB, B, K, L, indices)
   if (NB <= 16) MSA_TOPK_LAUNCH(1);
   else if (NB <= 32) MSA_TOPK_LAUNCH(2);
   else if (NB <= 64) MSA_TOPK_LAUNCH(4);
+  else if (K <= kSelectMostSlots && NB <= 1024) {
+    if (NB <= 128) { MSA_TOPK_SELECT(2); }
+    else if (NB <= 256) { MSA_TOPK_SELECT(4); }
+    else if (NB <= 512) { MSA_TOPK_SELECT(8); }
+    else { MSA_TOPK_SELECT(16); }
+  }
   else if (NB <= 128) MSA_TOPK_LAUNCH(8);
   else if (NB <= 256) MSA_TOPK_LAUNCH(16);
   else if (NB <= 512) MSA_TOPK_LAUNCH(32);
@@ -75,6 +99,7 @@ int topk_launch(const float* scores, const int32_t* cu_seqlens, int nseq, int64_
   else if (NB <= 4096) MSA_TOPK_WAVE(64);
   else hipLaunchKernelGGL(topk_stream_kernel, dim3(grid_1d(rows, 4)), block, 0, st, scores, cu_seqlens, nseq, rows, G, NB, B, K, L, indices);
 #undef MSA_TOPK_LAUNCH
+#undef MSA_TOPK_SELECT
 #undef MSA_TOPK_WAVE
   return status_from(hipGetLastError());
 }

@@ -214,3 +214,29 @@ def test_topk_rows_beyond_4096_blocks(tokens, block, k, local, device):
                       local_blocks=local)
     ref = O.topk(scores.numpy(), [0, tokens], block_size=block, topk_blocks=k, local_blocks=local)
     np.testing.assert_array_equal(got.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("blocks,topk,local", [(65, 1, 0), (128, 24, 1), (129, 25, 2), (200, 64, 0), (300, 16, 3),
+                                               (512, 32, 2), (513, 33, 1), (700, 65, 1), (1024, 24, 24),
+                                               (1024, 64, 1)])
+@pytest.mark.parametrize("kind", ["normal", "ties", "equal", "special"])
+def test_topk_threshold_and_sort(kind, blocks, topk, local, device):
+    """Rows of 65 to 1024 blocks: both sort widths, their slot limits and one beyond, with
+    distinct values, many equal ones (more than the sort holds), rows of one value, and
+    infinities, NaN and -0."""
+    gen = torch.Generator().manual_seed(blocks + topk)
+    lengths, groups, block = [2 * blocks - 1, 70], 3, 2
+    total = sum(lengths)
+    scores = torch.randn(total, groups, blocks, generator=gen)
+    if kind == "ties":
+        scores = torch.randint(0, 4, scores.shape, generator=gen).float()
+    elif kind == "equal":
+        scores = torch.full_like(scores, -0.5)
+    elif kind == "special":
+        u = torch.rand(scores.shape, generator=gen)
+        for low, value in ((0.0, float("-inf")), (0.3, float("inf")), (0.32, float("nan")), (0.34, -0.0), (0.4, 0.0)):
+            scores[(u >= low) & (u < low + (0.3 if low == 0.0 else 0.02))] = value
+    cu = cu_tensor(lengths)
+    got = msa.m3_topk(scores.to(device), cu.to(device), block_size=block, topk_blocks=topk, local_blocks=local)
+    expected = O.topk(scores.numpy(), cu.tolist(), block_size=block, topk_blocks=topk, local_blocks=local)
+    np.testing.assert_array_equal(got.cpu().numpy(), expected)
