@@ -991,7 +991,7 @@ static BwdLayout bwd_layout(int64_t T, int64_t Hq, int64_t G, int64_t D, int64_t
   int64_t sepi = static_cast<int64_t>(kStatItemRows) / (R > 0 ? R : 1);
   if (sepi < 1) sepi = 1;
   b.stat_plan = kv_plan_layout(T, rows, G, K, tc, sepi);
-  b.main_plan = kv_plan_layout(T, rows, G, K, tc, kMainEdges);
+  b.main_plan = kv_plan_layout(T, rows, G, K, tc, kv_item_edges(tc, G, K, kMainEdges, 64));
   b.stat_base = 0;
   b.main_base = b.stat_plan.bytes;
   b.spart = b.main_base + b.main_plan.bytes;

@@ -100,6 +100,18 @@ struct KvPlan {
   int64_t bounds, starts, items, order, bytes;  // byte offsets of the arrays inside the plan area, total size
 };
 
+// CSR edges per work item: `most` where a chunk's tc G K edges then give 512 items (two per
+// CU), fewer down to `least` where they do not: an item's edges run one tile after the other
+// in one workgroup, so the few items of a small call leave most CUs idle. Measured at 1280
+// tokens, 2 groups, 4 slots, 8 heads of 64 dims (512 / 128 / 64 / 32 edges): backward main
+// pass 114 / 34 / 22 / 16 us, KL main pass 86 / 26 / 17 / 13, the sums over the items' dK, dV
+// and d_ik partials 6 / 16 / 24 / 39. Above that, smaller items cost more than they balance:
+// 8192 tokens, 2 groups, 16 heads of 256 dims, 512 / 256 / 128 edges: step 3610 / 3700 / 3736 us.
+inline int64_t kv_item_edges(int64_t tc, int64_t G, int64_t K, int64_t most, int64_t least) {
+  const int64_t e = tc * G * K / 512 / 16 * 16;
+  return e > most ? most : (e > least ? e : (least < most ? least : most));
+}
+
 KvPlan kv_plan_layout(int64_t T, int64_t rows, int64_t G, int64_t K, int64_t tc, int64_t epi);
 
 // Fills bounds[(nch + 1) x rows], starts[nch x (rows + 1)] and items[nch x max_items]
