@@ -165,6 +165,12 @@ int64_t msa_attn_bwd_workspace_bytes(int32_t dtype, int64_t total_tokens, int64_
                                      int64_t kv_groups, int64_t head_dim, int64_t topk_slots,
                                      int64_t total_blocks, int64_t block_size);
 
+/* Bytes of workspace that let the fp32 backward share the rows of one key tile between several
+ * workgroups (FP64 partial sums of dK and dV); optional: with NULL, or fewer bytes, one
+ * workgroup takes them all, which is slower for small token counts. 0 where it is not used
+ * (other types, head dims that are not 32, 64, 96 or 128, many tokens). 8-byte aligned. */
+int64_t msa_attn_bwd_split_bytes(int32_t dtype, int64_t total_tokens, int64_t kv_groups, int64_t head_dim);
+
 /* Stage 3 backward: dQ, dK, dV (each nullable; all NULL is a no-op) of the
  * attention computed by msa_attn_fwd with the same row_state. Replaces the
  * autograd backward of triton/sparse_attention.py:361-394 (_backward_kernel,

@@ -1,7 +1,8 @@
 // C ABI for stage 3 (sparse GQA attention forward / backward).
 // bf16 and fp16 inputs whose shape fits the MFMA templates run the KV-major MFMA kernels
-// (attn_kv_fwd.hip, attn_kv_bwd.hip); fp32 inputs and other shapes run the VALU kernels
-// (attn_scalar.hip).
+// (attn_kv_fwd.hip, attn_kv_bwd.hip); fp32 inputs run FP64 kernels (attn_f64_mfma.hip, or
+// attn_scalar.hip outside its shapes) and other shapes those of attn_scalar.hip.
+#include "attn_f64_mfma.hpp"
 #include "attn_mfma.hpp"
 #include "common.hpp"
 
@@ -15,8 +16,8 @@ int attn_dq_valu_dispatch(const void*, const void*, const void*, const void*, co
                           const int32_t*, int, int64_t, int, int, int, int, int, double, void*, hipStream_t);
 template <int DT>
 int attn_dkdv_valu_dispatch(const void*, const void*, const void*, const void*, const double*, const int32_t*,
-                            const int32_t*, const int32_t*, const int32_t*, int, int64_t, int, int, int, int, double,
-                            void*, void*, hipStream_t);
+                            const int32_t*, int64_t, const int32_t*, const int32_t*, int, int64_t, int, int, int, int, double,
+                            void*, void*, void*, int64_t, hipStream_t);
 
 // Input types the MFMA kernels take (exact products in fp32 for both).
 static bool mfma_dtype(int32_t dtype) { return dtype == kBF16 || dtype == kF16; }
@@ -75,6 +76,13 @@ extern "C" int64_t msa_attn_bwd_workspace_bytes(int32_t dtype, int64_t total_tok
   return attn_bwd_kv_workspace_bytes(total_tokens, q_heads, kv_groups, head_dim, topk_slots, total_blocks);
 }
 
+extern "C" int64_t msa_attn_bwd_split_bytes(int32_t dtype, int64_t total_tokens, int64_t kv_groups,
+                                            int64_t head_dim) {
+  if (dtype != kF32 || total_tokens <= 0 || kv_groups <= 0 || head_dim <= 0 || head_dim > 2048) return 0;
+  if (!attn_f64_dims_fit(static_cast<int>(head_dim), {})) return 0;
+  return attn_f64_dkdv_workspace_bytes(total_tokens, kv_groups, head_dim);
+}
+
 extern "C" int msa_attn_bwd(const void* q, const void* k, const void* v, int32_t dtype, const void* out,
                             const void* grad_out, double* row_state, const float* out_f32, const int32_t* indices,
                             const int32_t* cu_seqlens, int64_t num_seqs, int64_t total_tokens, int64_t q_heads,
@@ -109,8 +117,8 @@ extern "C" int msa_attn_bwd(const void* q, const void* k, const void* v, int32_t
   }
   if (rc != kOk || !need_kv) return rc;
   switch (dtype) {
-    case kF32: return attn_dkdv_valu_dispatch<kF32>(q, k, v, grad_out, row_state, cu_seqlens, cu_block_lens, row_ptr, query_indices, nseq, total_tokens, Hq, G, D, B, scale, grad_k, grad_v, st);
-    case kF16: return attn_dkdv_valu_dispatch<kF16>(q, k, v, grad_out, row_state, cu_seqlens, cu_block_lens, row_ptr, query_indices, nseq, total_tokens, Hq, G, D, B, scale, grad_k, grad_v, st);
-    default: return attn_dkdv_valu_dispatch<kBF16>(q, k, v, grad_out, row_state, cu_seqlens, cu_block_lens, row_ptr, query_indices, nseq, total_tokens, Hq, G, D, B, scale, grad_k, grad_v, st);
+    case kF32: return attn_dkdv_valu_dispatch<kF32>(q, k, v, grad_out, row_state, cu_seqlens, cu_block_lens, total_blocks, row_ptr, query_indices, nseq, total_tokens, Hq, G, D, B, scale, grad_k, grad_v, workspace, workspace_bytes, st);
+    case kF16: return attn_dkdv_valu_dispatch<kF16>(q, k, v, grad_out, row_state, cu_seqlens, cu_block_lens, total_blocks, row_ptr, query_indices, nseq, total_tokens, Hq, G, D, B, scale, grad_k, grad_v, workspace, workspace_bytes, st);
+    default: return attn_dkdv_valu_dispatch<kBF16>(q, k, v, grad_out, row_state, cu_seqlens, cu_block_lens, total_blocks, row_ptr, query_indices, nseq, total_tokens, Hq, G, D, B, scale, grad_k, grad_v, workspace, workspace_bytes, st);
   }
 }

@@ -23,6 +23,7 @@
 //                    dK += dS q, dV += p/mass dO over the R heads of each edge.
 // The query pass forms dQ = scale/mass * (sum p (dp-c) k - delta * sum p k),
 // which needs one pass over the keys instead of two.
+#include "attn_f64_mfma.hpp"
 #include "common.hpp"
 
 namespace msa {
@@ -695,6 +696,11 @@ template <int DT, int DPL>
 int attn_valu_launch_fwd(const void* q, const void* k, const void* v, const int32_t* idx, const int32_t* cu,
                          int nseq, int64_t T, int Hq, int G, int D, int K, int B, double scale, void* out,
                          float* lse, double* rs, float* o32, hipStream_t st) {
+  if constexpr (DT == kF32) {
+    if (attn_f64_dims_fit(D, {q, k, v}) && attn_f64_heads_fit(Hq / G))
+      return attn_f64_fwd_launch(static_cast<const float*>(q), static_cast<const float*>(k), static_cast<const float*>(v),
+                                 idx, cu, nseq, T, Hq, G, D, K, B, scale, static_cast<float*>(out), lse, rs, o32, st);
+  }
   if (rows_fit(D, q, k, v)) {
 #define MSA_FWD_ROWS(LPRV) hipLaunchKernelGGL((attn_fwd_rows<DT, LPRV>), dim3(grid_1d(T * Hq, 4)), dim3(256), 4 * D * sizeof(float), st, q, k, v, idx, cu, nseq, T, Hq, G, D, K, B, scale, out, lse, rs, o32)
     MSA_ROWS_SWITCH(D, MSA_FWD_ROWS);
@@ -711,6 +717,12 @@ template <int DT, int DPL>
 int attn_valu_launch_dq(const void* q, const void* k, const void* v, const void* out, const void* dout, double* rs,
                         const int32_t* idx, const int32_t* cu, int nseq, int64_t T, int Hq, int G, int D, int K,
                         int B, double scale, void* dq, hipStream_t st) {
+  if constexpr (DT == kF32) {
+    if (attn_f64_dims_fit(D, {q, k, v, out, dout}) && attn_f64_heads_fit(Hq / G))
+      return attn_f64_dq_launch(static_cast<const float*>(q), static_cast<const float*>(k), static_cast<const float*>(v),
+                                static_cast<const float*>(out), static_cast<const float*>(dout), rs, idx, cu, nseq, T, Hq,
+                                G, D, K, B, scale, static_cast<float*>(dq), st);
+  }
   if (rows_fit(D, q, k, v, dout)) {
 #define MSA_DQ_ROWS(LPRV) hipLaunchKernelGGL((attn_bwd_dq_rows<DT, LPRV>), dim3(grid_1d(T * Hq, 4)), dim3(256), 8 * D * sizeof(float), st, q, k, v, out, dout, rs, idx, cu, nseq, T, Hq, G, D, K, B, scale, dq)
     MSA_ROWS_SWITCH(D, MSA_DQ_ROWS);
@@ -725,9 +737,16 @@ int attn_valu_launch_dq(const void* q, const void* k, const void* v, const void*
 
 template <int DT, int DPL>
 int attn_valu_launch_dkdv(const void* q, const void* k, const void* v, const void* dout, const double* rs,
-                          const int32_t* cu, const int32_t* cu_blocks, const int32_t* row_ptr, const int32_t* qidx,
-                          int nseq, int64_t T, int Hq, int G, int D, int B, double scale, void* dk, void* dv,
-                          hipStream_t st) {
+                          const int32_t* cu, const int32_t* cu_blocks, int64_t total_blocks, const int32_t* row_ptr,
+                          const int32_t* qidx, int nseq, int64_t T, int Hq, int G, int D, int B, double scale, void* dk,
+                          void* dv, void* ws, int64_t ws_bytes, hipStream_t st) {
+  if constexpr (DT == kF32) {
+    if (attn_f64_dims_fit(D, {q, k, v, dout, rs}))
+      return attn_f64_dkdv_launch(static_cast<const float*>(q), static_cast<const float*>(k),
+                                  static_cast<const float*>(v), static_cast<const float*>(dout), rs, cu, cu_blocks,
+                                  total_blocks, row_ptr, qidx, nseq, T, Hq, G, D, B, scale, static_cast<float*>(dk),
+                                  static_cast<float*>(dv), ws, ws_bytes, st);
+  }
   if (rows_fit(D, q, k, v, dout, rs)) {
 #define MSA_DKDV_ROWS(LPRV, NCV) hipLaunchKernelGGL((attn_bwd_dkdv_rows<DT, LPRV, NCV>), dim3(grid_1d(T * G, 4)), dim3(256), 0, st, q, k, v, dout, rs, cu, cu_blocks, row_ptr, qidx, nseq, T, Hq, G, D, B, scale, dk, dv)
     switch (D) {  // 2-byte types at D = 128: 16 dims a lane; otherwise 8
@@ -773,11 +792,11 @@ int attn_dq_valu_dispatch(const void* q, const void* k, const void* v, const voi
 
 template <int DT>
 int attn_dkdv_valu_dispatch(const void* q, const void* k, const void* v, const void* dout, const double* rs,
-                            const int32_t* cu, const int32_t* cu_blocks, const int32_t* row_ptr, const int32_t* qidx,
-                            int nseq, int64_t T, int Hq, int G, int D, int B, double scale, void* dk, void* dv,
-                            hipStream_t st) {
-  return MSA_DPL_DISPATCH(D, attn_valu_launch_dkdv, q, k, v, dout, rs, cu, cu_blocks, row_ptr, qidx, nseq, T, Hq, G,
-                          D, B, scale, dk, dv, st);
+                            const int32_t* cu, const int32_t* cu_blocks, int64_t total_blocks, const int32_t* row_ptr,
+                            const int32_t* qidx, int nseq, int64_t T, int Hq, int G, int D, int B, double scale, void* dk,
+                            void* dv, void* ws, int64_t ws_bytes, hipStream_t st) {
+  return MSA_DPL_DISPATCH(D, attn_valu_launch_dkdv, q, k, v, dout, rs, cu, cu_blocks, total_blocks, row_ptr, qidx, nseq, T, Hq, G,
+                          D, B, scale, dk, dv, ws, ws_bytes, st);
 }
 
 #define MSA_INSTANTIATE_VALU(DT)                                                                                    \
@@ -788,8 +807,9 @@ int attn_dkdv_valu_dispatch(const void* q, const void* k, const void* v, const v
                                          const int32_t*, const int32_t*, int, int64_t, int, int, int, int, int,      \
                                          double, void*, hipStream_t);                                                \
   template int attn_dkdv_valu_dispatch<DT>(const void*, const void*, const void*, const void*, const double*,       \
-                                           const int32_t*, const int32_t*, const int32_t*, const int32_t*, int,      \
-                                           int64_t, int, int, int, int, double, void*, void*, hipStream_t);
+                                           const int32_t*, const int32_t*, int64_t, const int32_t*, const int32_t*,  \
+                                           int, int64_t, int, int, int, int, double, void*, void*, void*, int64_t,   \
+                                           hipStream_t);
 MSA_INSTANTIATE_VALU(kF32)
 MSA_INSTANTIATE_VALU(kF16)
 MSA_INSTANTIATE_VALU(kBF16)

@@ -119,6 +119,8 @@ def _attn_backward(q, k, v, indices, cu, out, row_state, grad_output, meta, bloc
             csr = _k2q.build_k2q_csr(indices, cu if seqs is None else seqs, block_size=block_size)
         elif ws_bytes > 0:
             csr = _k2q._build_device(indices, cu, meta, groups, slots, seqs)
+        if need_kv and ws_bytes == 0:  # fp32: partial sums of the KV pass
+            ws_bytes = lib.msa_attn_bwd_split_bytes(dtype, total, groups, dim)
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=device) if ws_bytes > 0 else None
         with torch.cuda.device(device):
             status = lib.msa_attn_bwd(

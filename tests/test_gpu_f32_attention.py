@@ -1,0 +1,70 @@
+"""fp32 attention on the FP64 matrix products against the FP64 oracle, and where it ends."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import msa_triton_amd as msa
+from oracle import msa_oracle as O
+from tests.helpers import cu_tensor, np64, random_selection
+
+pytestmark = pytest.mark.gpu
+
+
+def _close_f32(actual, expected, what):
+    """FP64 arithmetic rounded once to fp32: within 2^-23 of each value, plus the FP64 sums'
+    own rounding (1e-11: 2^-53 of sums of up to ~1e4 in magnitude)."""
+    act = actual.detach().cpu().numpy().astype(np.float64)
+    worst = np.max(np.abs(act - expected) - 2.0 ** -23 * np.abs(expected))
+    assert worst <= 1e-11, f"{what}: {worst}"
+
+
+@pytest.mark.parametrize("dimension", [32, 64, 96, 128])
+@pytest.mark.parametrize("lengths,groups,ratio,block,topk", [
+    ([1], 1, 8, 128, 1), ([17, 0, 15, 130], 2, 4, 16, 3), ([300, 33], 1, 8, 128, 2), ([95, 64], 2, 3, 5, 6),
+    ([210], 1, 5, 100, 2), ([257], 2, 8, 200, 1), ([40, 90], 2, 2, 24, 3), ([70], 1, 12, 16, 4),
+])
+def test_f32_forward_backward_against_fp64(lengths, groups, ratio, block, topk, dimension, device):
+    """3 to 8 heads per group (matrix products in every pass), and 2 and 12 (the query passes on
+    the vector unit); tiles of fewer than 16 keys and rows, blocks above 128 keys, slots with
+    -1 and future ids."""
+    gen = torch.Generator().manual_seed(dimension + block)
+    total = sum(lengths)
+    q, k, v, dout = (torch.randn(total, n, dimension, generator=gen)
+                     for n in (groups * ratio, groups, groups, groups * ratio))
+    ids = random_selection(total, groups, topk, lengths, block, 1, gen)
+    ids[2::5, :, -1] = 1000  # after every query
+    cu = cu_tensor(lengths)
+    out, lse, dq, dk, dv = O.sparse_attention(np64(q), np64(k), np64(v), ids.numpy(), cu.numpy(), block_size=block,
+                                              scale=None, dout=np64(dout))
+    leaves = [x.to(device).requires_grad_() for x in (q, k, v)]
+    got, got_lse = msa.m3_sparse_attention(*leaves, ids.to(device), cu.to(device), max(lengths), block_size=block,
+                                           return_lse=True)
+    got.backward(dout.to(device))
+    finite = np.isfinite(lse)
+    assert np.array_equal(finite, np.isfinite(got_lse.cpu().numpy()))
+    _close_f32(got_lse[torch.from_numpy(finite).to(device)], lse[finite], "lse")
+    for actual, ref, what in zip((got, *(x.grad for x in leaves)), (out, dq, dk, dv), ("out", "dq", "dk", "dv")):
+        _close_f32(actual, ref, what)
+
+
+def test_f32_rows_off_16_byte_boundaries_equal_aligned_ones(device):
+    """The same values one element past a 16-byte boundary take the vector kernels: both within
+    one fp32 rounding of the same FP64 result."""
+    gen = torch.Generator().manual_seed(3)
+    lengths, groups, ratio, dimension, block, topk = [150, 37], 2, 4, 64, 32, 3
+    total = sum(lengths)
+    values = [torch.randn(total, n, dimension, generator=gen) for n in (groups * ratio, groups, groups)]
+    ids = random_selection(total, groups, topk, lengths, block, 1, gen).to(device)
+    cu = cu_tensor(lengths, device)
+
+    def shifted(x):
+        flat = torch.empty(x.numel() + 1, device=device)
+        flat[1:] = x.to(device).flatten()
+        return flat[1:].view(x.shape)
+
+    a = msa.m3_sparse_attention(*(x.to(device) for x in values), ids, cu, max(lengths), block_size=block)
+    b = msa.m3_sparse_attention(*(shifted(x) for x in values), ids, cu, max(lengths), block_size=block)
+    assert bool(((a - b).abs() <= 2.0 ** -22 * b.abs()).all())
