@@ -145,7 +145,7 @@ def _pmc_rows(directory, counter, unit=1024.0):
 def summarize_pmc(config, fetch_dir, write_dir):
     """Per-entry HBM bytes of one msa_attn_fwd and one msa_attn_bwd call from two --pmc-pass runs.
     The calibration copy (the largest copy dispatch) moves COPY bytes each way; each counter is scaled
-    so that it reads exactly that. The forward call's dispatches run from its first kv_chunk_bounds up
+    so that it reads exactly that. The forward call's dispatches run from its first kv_plan_kernel up
     to the first backward kernel (kv_bwd_*), the backward call's from there to the end."""
     copy_bytes = 64 << 22  # 256 MiB
     out = {"config": config, "counters": ["FETCH_SIZE", "WRITE_SIZE"],
@@ -163,7 +163,7 @@ def summarize_pmc(config, fetch_dir, write_dir):
         out["calibration"][f"{key}_scale"] = round(scale, 4)
         first_bwd = next(i for i, r in enumerate(rows) if "kv_bwd_" in r[1])
         last_bwd = max(i for i, r in enumerate(rows) if "kv_bwd_" in r[1])
-        first_fwd = max(i for i, r in enumerate(rows[:first_bwd]) if "kv_chunk_bounds" in r[1])
+        first_fwd = max(i for i, r in enumerate(rows[:first_bwd]) if "kv_plan_kernel" in r[1])
         for i, (_, name, value) in enumerate(rows):
             if "copy" in name.lower():
                 continue

@@ -1055,8 +1055,8 @@ int attn_bwd_kv(int dt, const void* q, const void* k, const void* v, const void*
   }
   {
     ProfScope ps(kProfBwdPlan, st);
-    kv_plan_launch(L.stat_plan, row_ptr, qidx, T, sbase, st, false);  // row order measured faster here
-    kv_plan_launch(L.main_plan, row_ptr, qidx, T, mbase, st);
+    // (the statistics pass measured faster in row order)
+    kv_plan_launch({{L.stat_plan, sbase, false}, {L.main_plan, mbase, true}}, row_ptr, qidx, T, st);
   }
   const KvPlan& sp = L.stat_plan;
   const KvPlan& mp = L.main_plan;

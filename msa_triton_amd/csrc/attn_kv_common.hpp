@@ -8,6 +8,8 @@
 // contiguous range. A plan lists, per chunk, work items (row, first edge) of at
 // most `epi` edges each.
 #pragma once
+#include <initializer_list>
+
 #include "attn_mfma.hpp"
 #include "mfma_util.hpp"
 
@@ -114,12 +116,18 @@ inline int64_t kv_item_edges(int64_t tc, int64_t G, int64_t K, int64_t most, int
 
 KvPlan kv_plan_layout(int64_t T, int64_t rows, int64_t G, int64_t K, int64_t tc, int64_t epi);
 
-// Fills bounds[(nch + 1) x rows], starts[nch x (rows + 1)] and items[nch x max_items]
-// (int2: row, first edge) in the plan area at `base`, and with `ordered` also
-// order[nch x max_items] (per chunk, the item indices largest first: the dispatch order
-// of the KV-major kernels; a kernel given no order takes the items in row order).
-void kv_plan_launch(const KvPlan& p, const int32_t* row_ptr, const int32_t* qidx, int64_t T, void* base,
-                    hipStream_t st, bool ordered = true);
+// Fills, for each plan, bounds[(nch + 1) x rows], starts[nch x (rows + 1)] and items[nch x
+// max_items] (int2: row, first edge) in the plan area at `base`, and with `ordered` also
+// order[nch x max_items] (per chunk, the item indices largest first: the dispatch order of the
+// KV-major kernels; a kernel given no order takes the items in row order). One launch for the
+// one or two plans of a call, which share their rows and chunks.
+struct KvPlanAt {
+  const KvPlan& plan;
+  void* base;
+  bool ordered;
+};
+void kv_plan_launch(std::initializer_list<KvPlanAt> plans, const int32_t* row_ptr, const int32_t* qidx, int64_t T,
+                    hipStream_t st);
 
 // Per chunk views of a launched plan.
 inline const int32_t* kv_plan_hi(const KvPlan& p, const void* base, int64_t c) {

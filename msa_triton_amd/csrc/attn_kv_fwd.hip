@@ -71,45 +71,45 @@ struct FwdSmem {
 
 }  // namespace
 
-// Per row, the first edge whose query token is >= c * tc, for c = 0..nch
-// (bounds[c * rows + row]); bound nch is the row end. One wavefront per row, one
-// lane per chunk boundary (independent binary searches over the row's edges).
-__global__ __launch_bounds__(256) void kv_chunk_bounds(const int32_t* __restrict__ row_ptr,
+// The work plans of a call, one workgroup per (chunk, plan). For chunk c of plan y:
+//   bounds[c * rows + row]: the row's first edge whose query token is >= c * tc (bound nch:
+//     the row's end), by binary search over the row's edges;
+//   item_start[c * (rows + 1) + row]: exclusive prefix over rows of ceil(edges / epi) work
+//     items, the chunk total at index rows;
+//   items[c * max_items + i] = (row, first edge of the item);
+//   order[slot] (if not null): the items by decreasing edge count (a counting sort on
+//     epi - edges, clamped to kOrderBuckets - 1): launched in this order, the short items
+//     (row tails) are the last to start, so the workgroups of a launch finish closer
+//     together. Items of equal size take their slots in no fixed order (integer atomics); no
+//     result depends on it, as each item writes only its own outputs, indexed by item.
+// Bound by launches and latency: as three kernels per plan (bounds, prefix, order), the plans
+// of a forward and backward took 8 launches (63 us at 32 768 tokens and 16 slots, 45 at 8192, 33 at 1280), as
+// one kernel each 2 (77, 26 and 14 us).
+constexpr int kOrderBuckets = 1024;
+constexpr int kMaxPlans = 2;
+struct PlanOut {
+  int epi;
+  int64_t max_items;
+  int32_t *bounds, *starts, *order;
+  int2* items;
+};
+struct PlanOuts {
+  PlanOut p[kMaxPlans];
+};
+__global__ __launch_bounds__(1024) void kv_plan_kernel(const int32_t* __restrict__ row_ptr,
                                                        const int32_t* __restrict__ qidx, int64_t rows, int64_t T,
-                                                       int64_t tc, int nch, int32_t* __restrict__ bounds) {
-  const int64_t r = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  if (r >= rows) return;
-  const int32_t a = row_ptr[r], b = row_ptr[r + 1];
-  for (int c = threadIdx.x & 63; c <= nch; c += kWave) {
-    const int64_t t = c * tc < T ? c * tc : T;
-    int32_t lo = a, hi = b;
-    while (lo < hi) {
-      const int32_t mid = lo + ((hi - lo) >> 1);  // lo + hi may exceed INT32_MAX
-      if (qidx[mid] < t) lo = mid + 1; else hi = mid;
-    }
-    bounds[c * rows + r] = (c == nch) ? b : lo;
-  }
-}
-
-// For chunk blockIdx.x: the exclusive prefix over rows of ceil(edges / epi) work
-// items, item_start[c * (rows + 1) + row], with the chunk total at index rows,
-// and the item table items[c * max_items + i] = (row, first edge of the item).
-__global__ __launch_bounds__(1024) void kv_item_scan(const int32_t* __restrict__ bounds, int64_t rows, int epi,
-                                                      int64_t max_items, int32_t* __restrict__ item_start,
-                                                      int2* __restrict__ items) {
+                                                       int64_t tc, int nch, PlanOuts outs, int row_order) {
   __shared__ int32_t wsum[16];
-  __shared__ int32_t carry_s;
-  const int64_t c = blockIdx.x;
-  const int32_t* lo_b = bounds + c * rows;
-  const int32_t* hi_b = bounds + (c + 1) * rows;
-  int32_t* out = item_start + c * (rows + 1);
-  if (threadIdx.x == 0) carry_s = 0;
-  __syncthreads();
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  for (int64_t base = 0; base < rows; base += 1024) {
-    const int64_t r = base + threadIdx.x;
-    const int32_t n = r < rows ? (hi_b[r] - lo_b[r] + epi - 1) / epi : 0;
-    int32_t x = n;
+  __shared__ int32_t cnt[kOrderBuckets];
+  const PlanOut po = outs.p[blockIdx.y];
+  const int c = blockIdx.x, epi = po.epi;
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  int32_t* starts = po.starts + c * (rows + 1);
+  int2* items = po.items + c * po.max_items;
+  int32_t* order = po.order ? po.order + c * po.max_items : nullptr;
+  // exclusive prefix of x over the workgroup; total in `sum`
+  auto prefix = [&](int32_t x, int32_t& sum) {
+    const int32_t own = x;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
       const int32_t y = __shfl_up(x, o, kWave);
@@ -117,103 +117,85 @@ __global__ __launch_bounds__(1024) void kv_item_scan(const int32_t* __restrict__
     }
     if (lane == 63) wsum[wid] = x;
     __syncthreads();
-    if (threadIdx.x < 16) {
-      int32_t w = wsum[threadIdx.x];
+    int32_t before = 0;
+    sum = 0;
 #pragma unroll
-      for (int o = 1; o < 16; o <<= 1) {
-        const int32_t y = __shfl_up(w, o, 16);
-        if (static_cast<int>(threadIdx.x) >= o) w += y;
-      }
-      wsum[threadIdx.x] = w;
+    for (int w = 0; w < 16; ++w) {
+      const int32_t y = wsum[w];
+      before += w < wid ? y : 0;
+      sum += y;
     }
     __syncthreads();
-    const int32_t carry = carry_s;
-    if (r < rows) {
-      const int32_t first = carry + (wid > 0 ? wsum[wid - 1] : 0) + x - n;
-      out[r] = first;
-      int2* dst = items + c * max_items + first;  // first + n <= chunk total <= max_items
-      for (int32_t j = 0; j < n; ++j) dst[j] = make_int2(static_cast<int32_t>(r), lo_b[r] + j * epi);
+    return before + x - own;
+  };
+  // the row's edges of this chunk, [x, y): both ends searched side by side (their loads overlap)
+  auto edges_of = [&](int64_t r) {
+    const int32_t a = row_ptr[r], b = row_ptr[r + 1];
+    const int64_t t0 = c * tc, t1 = (c + 1) * tc;
+    int32_t lo0 = a, hi0 = c == 0 ? a : b, lo1 = c == nch - 1 ? b : a, hi1 = b;
+    while (lo0 < hi0 || lo1 < hi1) {
+      const int32_t m0 = lo0 + ((hi0 - lo0) >> 1), m1 = lo1 + ((hi1 - lo1) >> 1);  // (lo + hi may exceed INT32_MAX)
+      const int32_t q0 = lo0 < hi0 ? qidx[m0] : 0, q1 = lo1 < hi1 ? qidx[m1] : 0;
+      if (lo0 < hi0) { if (q0 < t0) lo0 = m0 + 1; else hi0 = m0; }
+      if (lo1 < hi1) { if (q1 < t1) lo1 = m1 + 1; else hi1 = m1; }
     }
-    __syncthreads();
-    if (threadIdx.x == 0) carry_s = carry + wsum[15];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) out[rows] = carry_s;
-}
-
-// For chunk blockIdx.x: order[slot] = the chunk's work items by decreasing edge count
-// (a counting sort on epi - edges, clamped to kOrderBuckets - 1). Launched in this
-// order, the short items (row tails) are the last to start, so the workgroups of a
-// launch finish closer together. Items of equal size take their slots in no fixed
-// order (integer atomics); no result depends on it, as each item writes only its own
-// outputs, indexed by item.
-constexpr int kOrderBuckets = 1024;
-__global__ __launch_bounds__(1024) void kv_item_order(const int32_t* __restrict__ bounds, int64_t rows, int epi,
-                                                       int64_t max_items, const int32_t* __restrict__ item_start,
-                                                       const int2* __restrict__ items, int32_t* __restrict__ order,
-                                                       int row_order) {
-  __shared__ int32_t cnt[kOrderBuckets];
-  __shared__ int32_t wsum[16];
-  const int64_t c = blockIdx.x;
-  const int32_t* hi_b = bounds + (c + 1) * rows;
-  const int2* its = items + c * max_items;
-  int32_t* out = order + c * max_items;
-  const int32_t n = item_start[c * (rows + 1) + rows];
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  if (row_order) {  // the identity (testing hook)
-    for (int32_t i = tid; i < n; i += 1024) out[i] = i;
-    return;
-  }
-  auto bucket = [&](int32_t i) {
-    const int2 it = its[i];
-    const int32_t left = hi_b[it.x] - it.y;  // edges from the item's first to the row's end
+    return make_int2(lo0, lo1);
+  };
+  // an item of `left` remaining edges: its bucket
+  auto bucket = [&](int32_t left) {
     const int32_t b = epi - (left < epi ? left : epi);
     return b < kOrderBuckets ? b : kOrderBuckets - 1;
   };
-  // Most items are full (bucket 0): those take one LDS atomic per wave, ranked by ballot.
   cnt[tid] = 0;
   __syncthreads();
-  for (int32_t i0 = 0; i0 < n; i0 += 1024) {  // whole waves iterate together (ballots)
-    const int32_t i = i0 + tid;
-    const int32_t b = i < n ? bucket(i) : -1;
-    const uint64_t full = __ballot(b == 0);
-    if (full != 0 && lane == static_cast<int>(__ffsll(static_cast<long long>(full)) - 1))
-      atomicAdd(&cnt[0], __popcll(full));
-    if (b > 0) atomicAdd(&cnt[b], 1);
-  }
-  __syncthreads();
-  // exclusive prefix over the buckets (thread tid owns bucket tid)
-  const int32_t own = cnt[tid];
-  int32_t x = own;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int32_t y = __shfl_up(x, o, kWave);
-    if (lane >= o) x += y;
-  }
-  if (lane == 63) wsum[wid] = x;
-  __syncthreads();
-  if (tid < 16) {
-    int32_t w = wsum[tid];
-#pragma unroll
-    for (int o = 1; o < 16; o <<= 1) {
-      const int32_t y = __shfl_up(w, o, 16);
-      if (tid >= o) w += y;
+  int32_t carry = 0, first = 0;
+  int2 mine = make_int2(0, 0);  // this thread's (last) row
+  for (int64_t base = 0; base < rows; base += 1024) {
+    const int64_t r = base + tid;
+    mine = r < rows ? edges_of(r) : make_int2(0, 0);
+    const int32_t lo = mine.x, hi = mine.y;
+    if (r < rows) {
+      po.bounds[c * rows + r] = lo;
+      if (c == nch - 1) po.bounds[nch * rows + r] = hi;
     }
-    wsum[tid] = w;
+    const int32_t n = (hi - lo + epi - 1) / epi;
+    int32_t sum;
+    first = carry + prefix(n, sum);
+    carry += sum;
+    if (r < rows) {
+      starts[r] = first;  // first + n <= chunk total <= max_items
+      for (int32_t j = 0; j < n; ++j) items[first + j] = make_int2(static_cast<int32_t>(r), lo + j * epi);
+      if (order && n > 0) {  // all of the row's items but the last are full
+        if (row_order) {
+          for (int32_t j = 0; j < n; ++j) order[first + j] = first + j;  // the identity (testing hook)
+        } else {
+          if (n > 1) atomicAdd(&cnt[0], n - 1);
+          atomicAdd(&cnt[bucket(hi - lo - (n - 1) * epi)], 1);
+        }
+      }
+    }
   }
+  if (tid == 0) starts[rows] = carry;
+  if (!order || row_order) return;  // whole workgroup
   __syncthreads();
-  cnt[tid] = (wid > 0 ? wsum[wid - 1] : 0) + x - own;
+  int32_t all;
+  const int32_t slot0 = prefix(cnt[tid], all);  // (its barriers order the reads and this write)
+  cnt[tid] = slot0;
   __syncthreads();
-  for (int32_t i0 = 0; i0 < n; i0 += 1024) {
-    const int32_t i = i0 + tid;
-    const int32_t b = i < n ? bucket(i) : -1;
-    const uint64_t full = __ballot(b == 0);
-    const int lead = full != 0 ? static_cast<int>(__ffsll(static_cast<long long>(full))) - 1 : 0;
-    int32_t base = 0;
-    if (full != 0 && lane == lead) base = atomicAdd(&cnt[0], __popcll(full));
-    base = __shfl(base, lead, kWave);
-    if (b == 0) out[base + __popcll(full & ((uint64_t(1) << lane) - 1))] = i;
-    else if (b > 0) out[atomicAdd(&cnt[b], 1)] = i;
+  for (int64_t base = 0; base < rows; base += 1024) {
+    const int64_t r = base + tid;
+    if (r >= rows) continue;
+    if (rows > 1024) {  // more than one row per thread: its values of the first pass again
+      mine = edges_of(r);
+      first = starts[r];
+    }
+    const int32_t hi = mine.y, lo = mine.x;
+    const int32_t n = (hi - lo + epi - 1) / epi;
+    if (n > 1) {
+      const int32_t s = atomicAdd(&cnt[0], n - 1);
+      for (int32_t j = 0; j < n - 1; ++j) order[s + j] = first + j;
+    }
+    if (n > 0) order[atomicAdd(&cnt[bucket(hi - lo - (n - 1) * epi)], 1)] = first + n - 1;
   }
 }
 
@@ -617,21 +599,23 @@ KvPlan kv_plan_layout(int64_t T, int64_t rows, int64_t G, int64_t K, int64_t tc,
   return p;
 }
 
-void kv_plan_launch(const KvPlan& p, const int32_t* row_ptr, const int32_t* qidx, int64_t T, void* base,
-                    hipStream_t st, bool ordered) {
-  if (p.rows <= 0) return;
-  char* b = static_cast<char*>(base);
-  int32_t* bounds = reinterpret_cast<int32_t*>(b + p.bounds);
-  hipLaunchKernelGGL(kv_chunk_bounds, dim3(grid_1d(p.rows, 4)), dim3(256), 0, st, row_ptr, qidx, p.rows, T, p.tc,
-                     static_cast<int>(p.nch), bounds);
-  hipLaunchKernelGGL(kv_item_scan, dim3(static_cast<unsigned>(p.nch)), dim3(1024), 0, st, bounds, p.rows,
-                     static_cast<int>(p.epi), p.max_items, reinterpret_cast<int32_t*>(b + p.starts),
-                     reinterpret_cast<int2*>(b + p.items));
-  if (ordered)
-    hipLaunchKernelGGL(kv_item_order, dim3(static_cast<unsigned>(p.nch)), dim3(1024), 0, st, bounds, p.rows,
-                       static_cast<int>(p.epi), p.max_items, reinterpret_cast<const int32_t*>(b + p.starts),
-                       reinterpret_cast<const int2*>(b + p.items), reinterpret_cast<int32_t*>(b + p.order),
-                       g_item_order.load(std::memory_order_relaxed) ? 0 : 1);
+void kv_plan_launch(std::initializer_list<KvPlanAt> plans, const int32_t* row_ptr, const int32_t* qidx, int64_t T,
+                    hipStream_t st) {
+  const KvPlan& p0 = plans.begin()->plan;  // the plans of one call share rows, chunks and tokens per chunk
+  if (p0.rows <= 0) return;
+  PlanOuts outs = {};
+  unsigned n = 0;
+  for (const KvPlanAt& x : plans) {
+    char* b = static_cast<char*>(x.base);
+    outs.p[n++] = PlanOut{static_cast<int>(x.plan.epi),
+                          x.plan.max_items,
+                          reinterpret_cast<int32_t*>(b + x.plan.bounds),
+                          reinterpret_cast<int32_t*>(b + x.plan.starts),
+                          x.ordered ? reinterpret_cast<int32_t*>(b + x.plan.order) : nullptr,
+                          reinterpret_cast<int2*>(b + x.plan.items)};
+  }
+  hipLaunchKernelGGL(kv_plan_kernel, dim3(static_cast<unsigned>(p0.nch), n), dim3(1024), 0, st, row_ptr, qidx, p0.rows, T,
+                     p0.tc, static_cast<int>(p0.nch), outs, g_item_order.load(std::memory_order_relaxed) ? 0 : 1);
 }
 
 struct FwdLayout {
@@ -675,7 +659,7 @@ int attn_fwd_kv(int dt, const void* q, const void* k, const void* v, const int32
   auto* ob = static_cast<uint16_t*>(out);
   {
     ProfScope ps(kProfFwdPlan, st);
-    kv_plan_launch(pl, row_ptr, qidx, T, base, st);
+    kv_plan_launch({{pl, base, true}}, row_ptr, qidx, T, st);
   }
   for (int64_t c = 0; c < pl.nch; ++c) {
     const int64_t t0 = c * pl.tc, t1 = t0 + pl.tc < T ? t0 + pl.tc : T;

@@ -824,7 +824,7 @@ extern "C" int msa_indexer_kl(const void* index_q, const void* index_k, const vo
   const int need_diq = grad_index_q != nullptr, need_dik = grad_index_k != nullptr;
 
   if (need_dik) hipLaunchKernelGGL(kl_zero, dim3(grid_1d(T * Di, 256)), dim3(256), 0, st, acc, T * Di);
-  kv_plan_launch(pl, row_ptr, query_indices, T, base, st);
+  kv_plan_launch({{pl, base, true}}, row_ptr, query_indices, T, st);
   for (int64_t ch = 0; ch < pl.nch; ++ch) {
     const int64_t t0 = ch * pl.tc, t1 = t0 + pl.tc < T ? t0 + pl.tc : T;
     const int it0 = static_cast<int>(t0);

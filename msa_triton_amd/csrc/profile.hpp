@@ -10,10 +10,10 @@ namespace msa {
 
 // Kernel kinds, in the order msa_profile_end reports them.
 enum ProfKind {
-  kProfFwdPlan = 0,        // kv_chunk_bounds + kv_item_scan of the forward
+  kProfFwdPlan = 0,        // kv_plan_kernel of the forward
   kProfFwdPartial,         // attn_fwd_partial_kernel
   kProfFwdCombine,         // attn_fwd_combine
-  kProfBwdPlan,            // kv_chunk_bounds + kv_item_scan of the backward (both plans)
+  kProfBwdPlan,            // kv_plan_kernel of the backward (both plans)
   kProfBwdCenter,          // kv_bwd_center
   kProfBwdStats,           // kv_bwd_stats_kernel
   kProfBwdStatsCombine,    // kv_bwd_stats_combine
