@@ -19,7 +19,7 @@
 //   4. k2q_scatter_par : per (tile, group), a stable counting sort of the tile's
 //                    edges on their block id places each edge at row_ptr[row] +
 //                    tile offset + its rank among the tile's edges of that row.
-//   5. k2q_tail    : entries at or beyond row_ptr[rows] become -1.
+//                    Entries at or beyond row_ptr[rows] become -1.
 #include <algorithm>
 #include <mutex>
 
@@ -184,9 +184,17 @@ __global__ __launch_bounds__(256) void k2q_scatter_par(const int32_t* __restrict
                                                        const int32_t* __restrict__ cu_blocks,
                                                        const int64_t* __restrict__ tri_prefix, int nseq, int G,
                                                        int K, int B, const int32_t* __restrict__ row_ptr,
+                                                       int64_t rows, int64_t capacity,
                                                        int32_t* __restrict__ counters,
                                                        int32_t* __restrict__ query_idx,
                                                        int32_t* __restrict__ slot_idx) {
+  // entries at or beyond row_ptr[rows] become -1: the grid's workgroups share them (a launch
+  // of its own took 3 to 5 us)
+  for (int64_t i = row_ptr[rows] + (static_cast<int64_t>(blockIdx.y) * gridDim.x + blockIdx.x) * 256 + threadIdx.x;
+       i < capacity; i += static_cast<int64_t>(gridDim.x) * gridDim.y * 256) {
+    query_idx[i] = -1;
+    slot_idx[i] = -1;
+  }
   __shared__ int32_t running[kParIds];
   __shared__ int32_t wcnt[4][kParIds];
   __shared__ int32_t rbase[kParIds];  // row_ptr[row of id] + the tile's offset inside that row
@@ -265,17 +273,6 @@ __global__ __launch_bounds__(256) void k2q_scatter_par(const int32_t* __restrict
   }
 }
 
-__global__ __launch_bounds__(256) void k2q_tail(const int32_t* __restrict__ row_ptr, int64_t rows,
-                                                int64_t capacity, int32_t* __restrict__ query_idx,
-                                                int32_t* __restrict__ slot_idx) {
-  const int64_t used = row_ptr[rows];
-  for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x + used; i < capacity;
-       i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-    query_idx[i] = -1;
-    slot_idx[i] = -1;
-  }
-}
-
 __global__ __launch_bounds__(256) void fill_i32(int32_t* __restrict__ dst, int64_t n, int32_t value) {
   for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
        i += static_cast<int64_t>(gridDim.x) * blockDim.x)
@@ -306,7 +303,7 @@ namespace msa {
 
 namespace {
 
-// The five launches of the build over a caller-provided int32 workspace of
+// The four launches of the build over a caller-provided int32 workspace of
 // counter_elems + total_blocks * groups entries (the tile histograms are cleared by
 // k2q_count itself and the row totals are written before they are read, so the
 // workspace may hold anything on entry).
@@ -331,10 +328,8 @@ int k2q_build_launch(const int32_t* indices, const int32_t* cu_seqlens, const in
                      nseq, G, rows, counters, totals);
   hipLaunchKernelGGL(k2q_ptrscan, dim3(1), dim3(1024), 0, st, totals, rows, row_ptr);
   hipLaunchKernelGGL(k2q_scatter_par, dim3(static_cast<unsigned>(total_blocks), static_cast<unsigned>(G)),
-                     dim3(256), 0, st, indices, cu_seqlens, cu_block_lens, tri_prefix, nseq, G, K, B, row_ptr,
-                     counters, query_indices, slot_indices);
-  hipLaunchKernelGGL(k2q_tail, dim3(capped_grid(capacity)), dim3(256), 0, st, row_ptr, rows, capacity,
-                     query_indices, slot_indices);
+                     dim3(256), 0, st, indices, cu_seqlens, cu_block_lens, tri_prefix, nseq, G, K, B, row_ptr, rows,
+                     capacity, counters, query_indices, slot_indices);
   return status_from(hipGetLastError());
 }
 
