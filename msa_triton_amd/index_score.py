@@ -34,7 +34,7 @@ def _score_forward(q, k, cu, meta, max_seqlen, block_size, scale, save_state):
     if total:
         lib = _lib.lib()
         workspace = torch.empty(lib.msa_score_fwd_workspace_bytes(total, groups, blocks), dtype=torch.uint8, device=q.device)
-        with torch.cuda.device(q.device):
+        with _lib.on_device(q.device):
             status = lib.msa_score_fwd(
                 q.data_ptr(), k.data_ptr(), _lib.DTYPE_CODE[q.dtype], cu.data_ptr(), meta.num_seqs,
                 total, groups, dim, blocks, block_size, scale, scores.data_ptr(),
@@ -57,7 +57,7 @@ def _score_backward(q, k, cu, tie, grad_scores, meta, blocks, scale, need_q, nee
         ws_bytes = (lib.msa_score_bwd_workspace_bytes(total, groups, blocks, dim, meta.block_size,
                                                      meta.total_blocks) if dk is not None else 0)
         workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=q.device)
-        with torch.cuda.device(q.device):
+        with _lib.on_device(q.device):
             status = lib.msa_score_bwd(
                 q.data_ptr(), k.data_ptr(), _lib.DTYPE_CODE[q.dtype], cu.data_ptr(), cu_blocks.data_ptr(),
                 tie.data_ptr(), ds.data_ptr(), meta.num_seqs, total, groups, dim, blocks,
@@ -174,7 +174,7 @@ class _IndexScoreTopk(torch.autograd.Function):
         if total:
             lib = _lib.lib()
             workspace = torch.empty(lib.msa_score_fwd_workspace_bytes(total, groups, blocks), dtype=torch.uint8, device=q.device)
-            with torch.cuda.device(q.device):
+            with _lib.on_device(q.device):
                 status = lib.msa_index_score_topk(
                     q.data_ptr(), k.data_ptr(), _lib.DTYPE_CODE[q.dtype], cu.data_ptr(), meta.num_seqs,
                     total, groups, dim, blocks, block_size, scale, topk_blocks, local_blocks, scores.data_ptr(),

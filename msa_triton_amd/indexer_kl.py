@@ -33,7 +33,7 @@ import torch
 
 from . import _lib
 from . import k2q as _k2q
-from .layout import PackedSequences, prepared_for, sequence_lengths, sequence_meta
+from .layout import PackedSequences, call_sequences, prepared_for, sequence_lengths, sequence_meta
 
 
 def _launch(iq, ik, q, k, indices, cu, meta, seqs, block_size, index_scale, scale, want_rows, need_q, need_k,
@@ -65,7 +65,7 @@ def _launch(iq, ik, q, k, indices, cu, meta, seqs, block_size, index_scale, scal
     if total:
         csr = _k2q._build_device(indices, cu, meta, groups, slots, seqs)
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
-        with torch.cuda.device(device):
+        with _lib.on_device(device):
             status = lib.msa_indexer_kl(
                 iq.data_ptr(), ik.data_ptr(), q.data_ptr(), k.data_ptr(), _lib.DTYPE_CODE[iq.dtype],
                 indices.data_ptr(), cu.data_ptr(), meta.num_seqs, total, heads, groups, dim, dim_i, slots,
@@ -170,6 +170,8 @@ def m3_indexer_kl(
         for length in lengths:
             bounds.append(bounds[-1] + length)
         meta = sequence_meta(bounds, block_size)
+        # cu_seqlens was read once above; the block metadata reaches the device in one copy
+        seqs = call_sequences(cu, meta, groups) if total else None
     else:
         meta = seqs.meta
     loss, rows = _IndexerKL.apply(index_q, index_k, q, k, indices, cu, meta, seqs, block_size, float(index_scale),

@@ -97,7 +97,7 @@ def _build_device(indices, cu_seqlens, meta, groups, slots, seqs=None) -> K2QCSR
     query_indices = torch.empty(capacity, dtype=torch.int32, device=device)
     slot_indices = torch.empty(capacity, dtype=torch.int32, device=device)
     workspace = torch.empty(max(1, counter_elems + num_rows), dtype=torch.int32, device=device)
-    with torch.cuda.device(device):
+    with _lib.on_device(device):
         status = _lib.lib().msa_k2q_build(
             indices.data_ptr(), cu_seqlens.data_ptr(), cu_block_lens.data_ptr(), tri.data_ptr(),
             meta.num_seqs, total, groups, slots, meta.block_size, meta.total_blocks, counter_elems,
@@ -133,7 +133,7 @@ def sub_block_selection(indices, meta, block_size, seqs, fits):
         if not fits(factor, sub, sub_meta):
             break
         split = torch.empty((total, groups, slots * factor), dtype=torch.int32, device=indices.device)
-        with torch.cuda.device(indices.device):
+        with _lib.on_device(indices.device):
             status = _lib.lib().msa_split_block_indices(indices.data_ptr(), total * groups, slots, factor,
                                                         split.data_ptr(), _lib.stream_of(indices.device))
         _lib.check(status, "msa_split_block_indices")

@@ -74,7 +74,7 @@ def _attn_forward(q, k, v, indices, cu, meta, block_size, scale, seqs, public_cs
             else:
                 csr = _k2q._build_device(indices, cu, meta, groups, slots, seqs)
             workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
-        with torch.cuda.device(q.device):
+        with _lib.on_device(q.device):
             status = lib.msa_attn_fwd(
                 q.data_ptr(), k.data_ptr(), v.data_ptr(), dtype, indices.data_ptr(), cu.data_ptr(),
                 meta.num_seqs, total, heads, groups, dim, slots, block_size, scale,
@@ -122,7 +122,7 @@ def _attn_backward(q, k, v, indices, cu, out, row_state, grad_output, meta, bloc
         if need_kv and ws_bytes == 0:  # fp32: partial sums of the KV pass
             ws_bytes = lib.msa_attn_bwd_split_bytes(dtype, total, groups, dim)
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=device) if ws_bytes > 0 else None
-        with torch.cuda.device(device):
+        with _lib.on_device(device):
             status = lib.msa_attn_bwd(
                 q.data_ptr(), k.data_ptr(), v.data_ptr(), dtype, out.data_ptr(), dout.data_ptr(),
                 row_state.data_ptr(), _lib.ptr(out_f32), indices.data_ptr(), cu.data_ptr(), meta.num_seqs, total,

@@ -49,7 +49,7 @@ def m3_topk(scores, cu_seqlens, *, block_size=128, topk_blocks=16, local_blocks=
         return result.fill_(-1)
     scores = scores.contiguous()
     cu = cu.contiguous()
-    with torch.cuda.device(scores.device):
+    with _lib.on_device(scores.device):
         status = _lib.lib().msa_topk(
             scores.data_ptr(), cu.data_ptr(), len(boundaries) - 1, total, groups, blocks, block_size,
             topk_blocks, local_blocks, result.data_ptr(), _lib.stream_of(scores.device),
