@@ -128,7 +128,7 @@ int msa_score_bwd(const void* index_q, const void* index_k, int32_t dtype,
                   int64_t index_dim, int64_t num_blocks, int64_t block_size, int64_t total_blocks,
                   double scale, void* grad_q, void* grad_k, void* workspace, void* stream);
 
-/* Stage 3 forward workspace in bytes; 0 means this configuration runs the VALU
+/* Stage 3 forward workspace in bytes; 0 means this configuration runs the FP64
  * kernels, which need neither the CSR nor a workspace. Non-zero (the KV-major MFMA
  * kernels) for bf16 and fp16 inputs with head ratio <= 512, head dim 8..256 a
  * multiple of 8 and blocks of at most 128 keys. */
@@ -159,7 +159,7 @@ int msa_attn_fwd(const void* q, const void* k, const void* v, int32_t dtype, con
                  const int32_t* slot_indices, void* workspace, int64_t workspace_bytes, void* out,
                  float* lse, double* row_state, float* out_f32, void* stream);
 
-/* Stage 3 backward workspace in bytes; 0 means this configuration runs the VALU
+/* Stage 3 backward workspace in bytes; 0 means this configuration runs the FP64
  * kernels, which need no workspace. */
 int64_t msa_attn_bwd_workspace_bytes(int32_t dtype, int64_t total_tokens, int64_t q_heads,
                                      int64_t kv_groups, int64_t head_dim, int64_t topk_slots,
