@@ -76,10 +76,20 @@ struct RowFrag {
   static constexpr bool TAIL = D % 64 != 0;
   float4 x[NA > 0 ? NA : 1];
   float2 t;
+  // (global loads are asked for by name: a row that is chosen from two arrays would be read with
+  // flat ones)
   __device__ __forceinline__ void load(const float* __restrict__ row, int c) {
+    typedef const __attribute__((address_space(1))) float* Global;
+    typedef const __attribute__((address_space(1))) f32x4* Global4;
 #pragma unroll
-    for (int a = 0; a < NA; ++a) x[a] = *reinterpret_cast<const float4*>(row + 64 * a + 4 * c);
-    if constexpr (TAIL) t = *reinterpret_cast<const float2*>(row + 64 * NA + 2 * c);
+    for (int a = 0; a < NA; ++a) {
+      const f32x4 y = *(Global4)(row + 64 * a + 4 * c);
+      x[a] = make_float4(y[0], y[1], y[2], y[3]);
+    }
+    if constexpr (TAIL) {
+      const Global y = (Global)(row + 64 * NA + 2 * c);
+      t = make_float2(y[0], y[1]);
+    }
   }
   // out[tile] += a^T . this row
   __device__ __forceinline__ void accumulate(double a, f64x4 (&out)[D / 16]) const {
@@ -337,6 +347,8 @@ __global__ __launch_bounds__(64 * kQueryWaves, 2) void attn_f64_dq(
   }
 }
 
+alignas(16) __device__ const float kZeroRow[128] = {};
+
 // dK, dV of 16 keys of one group: rows (edge, head) of the block's CSR row, 16 per step. With
 // `part`, blockIdx.z of gridDim.z workgroups share the rows and leave FP64 sums there
 // ([split][dK, dV][key][group][dim], added by attn_f64_dkdv_reduce); without, one workgroup
@@ -368,8 +380,10 @@ __global__ __launch_bounds__(64 * kKeyWaves, 2) void attn_f64_dkdv(
   f64x4 ak[NT], av[NT];
 #pragma unroll
   for (int n = 0; n < NT; ++n) ak[n] = av[n] = f64x4{0.0, 0.0, 0.0, 0.0};
-  for (int64_t i0 = 16 * (wid + kKeyWaves * static_cast<int64_t>(blockIdx.z)); i0 < nrows;
-       i0 += 16 * kKeyWaves * gridDim.z) {
+  const int64_t first = 16 * (wid + kKeyWaves * static_cast<int64_t>(blockIdx.z));
+  const int64_t stride = 16 * kKeyWaves * static_cast<int64_t>(gridDim.z);
+  uint64_t left_out = 0;
+  for (int64_t i0 = first; i0 < nrows; i0 += stride) {
     // this lane's row (c): its token and (token, head); past the end the last row, masked
     const int64_t i = i0 + c < nrows ? i0 + c : nrows - 1;
     const int64_t eo = nrows <= 0x7fffffff ? static_cast<uint32_t>(i) / static_cast<uint32_t>(R) : i / R;
@@ -388,6 +402,7 @@ __global__ __launch_bounds__(64 * kKeyWaves, 2) void attn_f64_dkdv(
     const f64x4 dp = dot_rows<D>(rf, cf);
     double p[4], ds[4];
     int64_t off[4];
+    bool zero[4];
 #pragma unroll
     for (int s4 = 0; s4 < 4; ++s4) {
       const int rr = 4 * s4 + q4;
@@ -399,12 +414,19 @@ __global__ __launch_bounds__(64 * kKeyWaves, 2) void attn_f64_dkdv(
       const bool ok = i0 + rr < nrows && c < nk && tr >= kb + c;
       p[s4] = ok ? exp(x[s4] * scale - a.x) / a.y : 0.0;
       ds[s4] = ok ? p[s4] * ((dp[s4] - b.x) - b.y) * scale : 0.0;
+      // A masked pair has weight 0, but 0 times a row that holds an infinity or a NaN is NaN
+      // (such a row's products with any key are not finite, and sums of finite fp32 products stay
+      // far inside the FP64 range): the matrix product takes zeros for this row, and what it gives
+      // to the keys that it does attend to is added at the end.
+      const uint64_t odd = __ballot(!ok && !(fabs(x[s4]) < __builtin_inf() && fabs(dp[s4]) < __builtin_inf()));
+      zero[s4] = (odd >> (16 * q4) & 0xffff) != 0;
+      left_out |= odd;
     }
 #pragma unroll
     for (int s4 = 0; s4 < 4; ++s4) {
       RowFrag<D> gr, qr;
-      gr.load(dout + off[s4], c);
-      qr.load(q + off[s4], c);
+      gr.load(zero[s4] ? kZeroRow : dout + off[s4], c);
+      qr.load(zero[s4] ? kZeroRow : q + off[s4], c);
       gr.accumulate(p[s4], av);
       qr.accumulate(ds[s4], ak);
       if (D == 128) __builtin_amdgcn_sched_barrier(0);  // (one step's rows at a time: registers)
@@ -423,6 +445,31 @@ __global__ __launch_bounds__(64 * kKeyWaves, 2) void attn_f64_dkdv(
         }
     }
     __syncthreads();
+  }
+  // the rows left out: a wave at a time, one row at a time, lane (key c, dims q4, q4 + 4, ...)
+  for (int w = 0; __syncthreads_or(left_out != 0) && w < kKeyWaves; ++w) {
+    for (int64_t i = first; wid == w && i < nrows; i += (i & 15) == 15 ? stride - 15 : 1) {
+      const int64_t t = qidx[e0 + i / R], th = t * Hq + static_cast<int64_t>(g) * R + i % R;
+      const int64_t off0 = ((kb + (c < nk ? c : nk - 1)) * G + g) * D;
+      double x = 0.0, dp = 0.0;
+#pragma unroll 1
+      for (int d = q4; d < D; d += 4) {
+        x = fma(static_cast<double>(q[th * D + d]), static_cast<double>(k[off0 + d]), x);
+        dp = fma(static_cast<double>(dout[th * D + d]), static_cast<double>(v[off0 + d]), dp);
+      }
+      x = quarter_sum(x);
+      dp = quarter_sum(dp);
+      const bool ok = c < nk && t >= kb + c;
+      if (__ballot(!ok && !(fabs(x) < __builtin_inf() && fabs(dp) < __builtin_inf())) == 0) continue;
+      const double* a = row_state + th * 4;  // lse, mass, c, delta
+      const double p = exp(x * scale - a[0]) / a[1], ds = p * ((dp - a[2]) - a[3]) * scale;
+      if (ok)
+#pragma unroll 1
+        for (int d = q4; d < D; d += 4) {
+          kbuf[c][d] = fma(ds, static_cast<double>(q[th * D + d]), kbuf[c][d]);
+          vbuf[c][d] = fma(p, static_cast<double>(dout[th * D + d]), vbuf[c][d]);
+        }
+    }
   }
   for (int e = tid; e < nk * D; e += 64 * kKeyWaves) {
     const int kk = e / D, d = e % D;

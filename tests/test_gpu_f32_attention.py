@@ -68,3 +68,32 @@ def test_f32_rows_off_16_byte_boundaries_equal_aligned_ones(device):
     a = msa.m3_sparse_attention(*(x.to(device) for x in values), ids, cu, max(lengths), block_size=block)
     b = msa.m3_sparse_attention(*(shifted(x) for x in values), ids, cu, max(lengths), block_size=block)
     assert bool(((a - b).abs() <= 2.0 ** -22 * b.abs()).all())
+
+
+@pytest.mark.parametrize("dimension", [32, 64, 96, 128])
+@pytest.mark.parametrize("tensor", ["q", "dout"])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_f32_non_finite_query_row_stays_with_the_keys_it_sees(value, tensor, dimension, device):
+    """A token whose q or dO row (one head) holds a NaN or an infinity: dK and dV of the keys it does
+    not see, later ones of its own block among them, are those of the call in which its dO is zero."""
+    gen = torch.Generator().manual_seed(dimension)
+    lengths, groups, ratio, block, topk = [70, 41], 2, 4, 32, 2
+    total, bad = sum(lengths), 37  # token 37: position 5 of its block of 32 keys, tile of 16 keys 32..47
+    q, k, v, dout = (torch.randn(total, n, dimension, generator=gen)
+                     for n in (groups * ratio, groups, groups, groups * ratio))
+    ids = random_selection(total, groups, topk, lengths, block, 1, gen)
+    cu = cu_tensor(lengths)
+    without = dout.clone()
+    without[bad] = 0.0
+    _, _, _, dk, dv = O.sparse_attention(np64(q), np64(k), np64(v), ids.numpy(), cu.numpy(), block_size=block,
+                                         scale=None, dout=np64(without))
+    dout[bad] = 0.0
+    (q if tensor == "q" else dout)[bad, 1, dimension // 2] = value
+    leaves = [x.to(device).requires_grad_() for x in (q, k, v)]
+    got = msa.m3_sparse_attention(*leaves, ids.to(device), cu.to(device), max(lengths), block_size=block)
+    got.backward(dout.to(device))
+    seen = torch.zeros(total, dtype=torch.bool)
+    seen[:bad + 1] = True  # (a superset: both selected blocks are earlier keys)
+    for leaf, ref, what in ((leaves[1], dk, "dk"), (leaves[2], dv, "dv")):
+        _close_f32(leaf.grad[~seen.to(device)], ref[~seen.numpy()], what)
+        _close_f32(leaf.grad[:, 1], ref[:, 1], what + " of the other group")
