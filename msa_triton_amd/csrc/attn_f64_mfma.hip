@@ -112,6 +112,9 @@ __device__ __forceinline__ int tile_dim(int n, int c) {
   return n < 4 * (D / 64) ? 64 * (n / 4) + 4 * c + n % 4 : 64 * (D / 64) + 2 * c + (n - 4 * (D / 64));
 }
 
+// Stands in for a row that must not enter a product (0 times an infinity or a NaN is NaN).
+alignas(16) __device__ const float kZeroRow[128] = {};
+
 // The sum (maximum) over the lanes c, c + 16, c + 32, c + 48.
 __device__ __forceinline__ double quarter_sum(double x) {
   x += __shfl_xor(x, 16, kWave);
@@ -186,7 +189,7 @@ __global__ __launch_bounds__(64 * kQueryWaves, 2) void attn_f64_fwd(
     kf.load(k + at(c), q4);
     RowFrag<D> vf[4];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) vf[s].load(v + at(4 * s + q4), c);
+    for (int s = 0; s < 4; ++s) vf[s].load(4 * s + q4 < nk ? v + at(4 * s + q4) : kZeroRow, c);
     const f64x4 x = dot_rows<D>(kf, qf);  // [key 4 s + q4][head c]
     double p[4], mt = -__builtin_inf();
 #pragma unroll
@@ -305,8 +308,9 @@ __global__ __launch_bounds__(64 * kQueryWaves, 2) void attn_f64_dq(
     for (int s = 0; s < 4; ++s) {
       RowFrag<D> kr;
       kr.load(k + at(4 * s + q4), c);
-      const double p = live && 4 * s + q4 < nk ? exp(x[s] * scale - row_lse) : 0.0;
-      const double u = p * (dp[s] - cen);
+      const bool ok = live && 4 * s + q4 < nk;
+      const double p = ok ? exp(x[s] * scale - row_lse) : 0.0;
+      const double u = ok ? p * (dp[s] - cen) : 0.0;  // (past nk dp repeats the last key's, which may be infinite)
       mass += p;
       delta += u;
       const double p8 = __shfl_xor(p, 8, kWave);  // p of head c - 8
@@ -346,8 +350,6 @@ __global__ __launch_bounds__(64 * kQueryWaves, 2) void attn_f64_dq(
     }
   }
 }
-
-alignas(16) __device__ const float kZeroRow[128] = {};
 
 // dK, dV of 16 keys of one group: rows (edge, head) of the block's CSR row, 16 per step. With
 // `part`, blockIdx.z of gridDim.z workgroups share the rows and leave FP64 sums there

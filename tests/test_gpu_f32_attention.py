@@ -97,3 +97,50 @@ def test_f32_non_finite_query_row_stays_with_the_keys_it_sees(value, tensor, dim
     for leaf, ref, what in ((leaves[1], dk, "dk"), (leaves[2], dv, "dv")):
         _close_f32(leaf.grad[~seen.to(device)], ref[~seen.numpy()], what)
         _close_f32(leaf.grad[:, 1], ref[:, 1], what + " of the other group")
+
+
+@pytest.mark.parametrize("dimension", [32, 64, 96, 128])
+def test_f32_infinite_value_at_the_end_of_a_partial_tile(dimension, device):
+    """V = inf at the last key of a partial tile of 16 keys: inf in the output of the rows that see it
+    (not the NaN that 0 times a repetition of that key would give), the rest as without it."""
+    gen = torch.Generator().manual_seed(dimension)
+    lengths, groups, ratio, block = [21], 1, 4, 21
+    total = sum(lengths)
+    q, k, v = (torch.randn(total, n, dimension, generator=gen) for n in (ratio, groups, groups))
+    ids = torch.zeros(total, groups, 1, dtype=torch.int32)
+    cu = cu_tensor(lengths)
+    v[20, 0, 3] = 0.0
+    out, _, _, _, _ = O.sparse_attention(np64(q), np64(k), np64(v), ids.numpy(), cu.numpy(), block_size=block,
+                                         scale=None, dout=np64(q))
+    v[20, 0, 3] = float("inf")  # tile of keys 16..20, seen by token 20 only
+    got = msa.m3_sparse_attention(*(x.to(device) for x in (q, k, v)), ids.to(device), cu.to(device), total,
+                                  block_size=block)
+    assert bool((got[20, :, 3] == float("inf")).all())
+    rest = torch.ones(total, ratio, dimension, dtype=torch.bool)
+    rest[20, :, 3] = False
+    _close_f32(got[rest.to(device)], out[rest.numpy()], "out")
+
+
+@pytest.mark.parametrize("dimension", [32, 64, 96, 128])
+def test_f32_infinite_value_counts_once_in_the_row_statistics(dimension, device):
+    """A row whose only infinite dP is that of the last key of a partial tile of 16 keys: its delta
+    (row_state[3]) is inf, not the NaN that a repetition of that key with weight 0 would give."""
+    total, ratio = 17, 4
+    q = torch.zeros(total, ratio, dimension)
+    k = torch.zeros(total, 1, dimension)
+    v = torch.zeros(total, 1, dimension)
+    v[16, 0, 0] = float("inf")  # second tile: one key of 16, seen by token 16 only
+    out = torch.zeros(total, ratio, dimension)
+    dout = torch.zeros(total, ratio, dimension)
+    dout[16, :, 0] = 1.0
+    from msa_triton_amd.layout import prepare_sequences
+    from msa_triton_amd.sparse_attention import _attn_backward
+
+    seqs = prepare_sequences(torch.tensor([0, total], dtype=torch.int32, device=device), block_size=32)
+    state = torch.zeros(total, ratio, 4, dtype=torch.float64, device=device)
+    state[..., 0] = torch.arange(1, total + 1, dtype=torch.float64, device=device).log()[:, None]  # lse of equal logits
+    state[..., 1] = 1.0
+    ids = torch.zeros(total, 1, 1, dtype=torch.int32, device=device)
+    _attn_backward(*(x.to(device) for x in (q, k, v)), ids, seqs.cu_seqlens, out.to(device), state, dout.to(device),
+                   seqs.meta, 32, 1.0, seqs, True, False, False)
+    assert bool((state[16, :, 3] == float("inf")).all())
