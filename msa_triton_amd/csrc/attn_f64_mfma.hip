@@ -209,9 +209,10 @@ __global__ __launch_bounds__(64 * kQueryWaves, 2) void attn_f64_fwd(
       }
       m = mn;
     }
+    const double base = mn == -__builtin_inf() ? 0.0 : mn;  // (only logits of -inf so far: weights 0, not NaN)
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-      p[s] = 4 * s + q4 < nk ? exp(p[s] - mn) : 0.0;
+      p[s] = 4 * s + q4 < nk ? exp(p[s] - base) : 0.0;
       l += p[s];
       vf[s].accumulate(p[s], o);
     }

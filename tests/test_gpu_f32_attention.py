@@ -144,3 +144,24 @@ def test_f32_infinite_value_counts_once_in_the_row_statistics(dimension, device)
     _attn_backward(*(x.to(device) for x in (q, k, v)), ids, seqs.cu_seqlens, out.to(device), state, dout.to(device),
                    seqs.meta, 32, 1.0, seqs, True, False, False)
     assert bool((state[16, :, 3] == float("inf")).all())
+
+
+@pytest.mark.parametrize("dimension", [32, 128])
+def test_f32_tile_of_minus_infinite_logits(dimension, device):
+    """Keys whose logits are -inf have weight 0, also when they fill the first tile of 16 keys: the
+    output and lse are those of the remaining keys, and 0 and -inf where no other key is visible."""
+    gen = torch.Generator().manual_seed(dimension)
+    total, ratio, block = 90, 4, 128
+    q, k, v = (torch.randn(total, n, dimension, generator=gen) for n in (ratio, 1, 1))
+    q = q.abs()
+    ids = torch.zeros(total, 1, 1, dtype=torch.int32)
+    cu = cu_tensor([total])
+    k[:16, 0, 0] = -1e30  # (for the oracle: exp of its logits is 0 as well)
+    out, lse, _, _, _ = O.sparse_attention(np64(q), np64(k), np64(v), ids.numpy(), cu.numpy(), block_size=block,
+                                           scale=None, dout=np64(q))
+    k[:16, 0, 0] = -float("inf")
+    got, got_lse = msa.m3_sparse_attention(*(x.to(device) for x in (q, k, v)), ids.to(device), cu.to(device), total,
+                                           block_size=block, return_lse=True)
+    assert bool((got[:16] == 0).all()) and bool((got_lse[:16] == -float("inf")).all())
+    _close_f32(got[16:], out[16:], "out")
+    _close_f32(got_lse[16:], lse[16:], "lse")
