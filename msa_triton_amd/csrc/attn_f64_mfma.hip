@@ -361,21 +361,47 @@ __global__ __launch_bounds__(64 * kKeyWaves, 2) void attn_f64_dkdv(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
     const float* __restrict__ dout, const double* __restrict__ row_state, const int32_t* __restrict__ cu,
     const int32_t* __restrict__ cu_blocks, const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ qidx,
-    int nseq, int64_t T, int Hq, int G, int B, double scale, float* __restrict__ dk, float* __restrict__ dv,
-    double* __restrict__ part) {
+    int nseq, int64_t T, int Hq, int G, int B, int64_t compact, double scale, float* __restrict__ dk,
+    float* __restrict__ dv, double* __restrict__ part) {
   constexpr int NT = D / 16;
   __shared__ double kbuf[16][D], vbuf[16][D];
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, q4 = lane >> 4;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // blockIdx.y = key tile of the block, blockIdx.x = (block, group) row
-  const int64_t row = blockIdx.x, gb = row / G;
-  const int g = static_cast<int>(row % G);
-  int s = upper_index(cu_blocks, nseq + 1, gb);
-  while (s < nseq && cu_blocks[s + 1] <= gb) ++s;
-  const int64_t kb = cu[s] + (gb - cu_blocks[s]) * B + 16 * static_cast<int64_t>(blockIdx.y);
-  const int64_t bend = cu[s] + (gb - cu_blocks[s] + 1) * B;
-  const int64_t kend = bend < cu[s + 1] ? bend : cu[s + 1];
-  if (kb >= kend) return;  // whole workgroup: the (short) block has no such tile
+  int64_t row, kb, kend;
+  const int g = static_cast<int>(blockIdx.x % G);
+  const int64_t x = blockIdx.x / G;
+  if (compact == 0) {  // x: block * tiles of a whole block + tile
+    const int64_t per_block = (static_cast<int64_t>(B) + 15) / 16, gb = x / per_block;
+    if (gb >= cu_blocks[nseq]) return;  // whole workgroup
+    int s = upper_index(cu_blocks, nseq + 1, gb);
+    while (s < nseq && cu_blocks[s + 1] <= gb) ++s;
+    const int64_t first = cu[s] + (gb - cu_blocks[s]) * B;
+    kb = first + 16 * (x - gb * per_block);
+    kend = first + B < cu[s + 1] ? first + B : cu[s + 1];
+    row = gb * G + g;
+  } else {
+    // x: a number of a tile. Tile i of block gb has the number first / 16 + gb + i (first: the
+    // block's first token): no two tiles share one, as a block of n keys has at most n / 16 + 1,
+    // and all are below T / 16 + blocks. The even numbers go first: with blocks of 16 keys
+    // every other number has no tile, and workgroups go to the XCDs round-robin.
+    const int64_t w = x < compact ? 2 * x : 2 * (x - compact) + 1;
+    int s = 0;  // the last sequence whose first tile is not after w
+    for (int hi = nseq; hi - s > 1;) {
+      const int mid = (s + hi) >> 1;
+      if (cu[mid] / 16 + static_cast<int64_t>(cu_blocks[mid]) <= w) s = mid; else hi = mid;
+    }
+    const int64_t start = cu[s], gb0 = cu_blocks[s];
+    int64_t b = 0;  // its last block whose first tile is not after w
+    for (int64_t hi = cu_blocks[s + 1] - gb0; hi - b > 1;) {
+      const int64_t mid = (b + hi) >> 1;
+      if ((start + mid * B) / 16 + gb0 + mid <= w) b = mid; else hi = mid;
+    }
+    const int64_t first = start + b * B;
+    kb = first + 16 * (w - first / 16 - gb0 - b);
+    kend = first + B < cu[s + 1] ? first + B : cu[s + 1];
+    row = (gb0 + b) * G + g;
+  }
+  if (kb >= kend) return;  // whole workgroup: no such tile
   const int nk = static_cast<int>(kend - kb < 16 ? kend - kb : 16);
   const int64_t e0 = row_ptr[row];
   const int R = Hq / G;
@@ -551,17 +577,25 @@ int64_t attn_f64_dkdv_workspace_bytes(int64_t T, int64_t G, int64_t D) {
 }
 
 int attn_f64_dkdv_launch(const float* q, const float* k, const float* v, const float* dout, const double* rs,
-                         const int32_t* cu, const int32_t* cu_blocks, int64_t total_blocks, const int32_t* row_ptr,
-                         const int32_t* qidx, int nseq, int64_t T, int Hq, int G, int D, int B, double scale, float* dk,
-                         float* dv, void* ws, int64_t ws_bytes, hipStream_t st) {
-  if (total_blocks <= 0) return kOk;
+                         const int32_t* cu, const int32_t* cu_blocks, const int32_t* row_ptr, const int32_t* qidx,
+                         int nseq, int64_t T, int Hq, int G, int D, int B, double scale, float* dk, float* dv, void* ws,
+                         int64_t ws_bytes, hipStream_t st) {
   // a caller without the workspace gets the unsplit pass
   const int64_t need = attn_f64_dkdv_workspace_bytes(T, G, D);
   const bool split = ws && need > 0 && ws_bytes >= need && (reinterpret_cast<uintptr_t>(ws) & 7) == 0;
   const int splits = split ? dkdv_splits(T, G) : 1;
   double* part = split ? static_cast<double*>(ws) : nullptr;
-  const dim3 grid(static_cast<unsigned>(total_blocks * G), static_cast<unsigned>((B + 15) / 16), splits);
-#define MSA_F64_DKDV(DV) hipLaunchKernelGGL(attn_f64_dkdv<DV>, grid, dim3(64 * kKeyWaves), 0, st, q, k, v, dout, rs, cu, cu_blocks, row_ptr, qidx, nseq, T, Hq, G, B, scale, dk, dv, part)
+  // One workgroup per tile of every block, a block's tiles side by side (they gather the same rows; with
+  // one block's tiles far apart 4 sequences of 2048 tokens took 8790 us for the backward, so 6257), or,
+  // where whole blocks would give more than two numbers per tile (short sequences, blocks far longer
+  // than they), numbered by tile: 8 sequences of 1024 tokens in blocks of 2^19 keys 8815 -> 5538 us.
+  // blocks: at least as many as there are; numbers without a tile come last, as far as possible
+  // (spread evenly between the others they leave shader engines idle: 8 x 1024, 8668 us).
+  const int64_t blocks = T / B + nseq < T ? T / B + nseq : T, tiles = T / 16 + blocks;
+  const int64_t per_block = (static_cast<int64_t>(B) + 15) / 16;
+  const int64_t compact = per_block * blocks > 2 * tiles ? (tiles + 1) / 2 : 0;
+  const dim3 grid(static_cast<unsigned>((compact ? 2 * compact : blocks * per_block) * G), 1, splits);
+#define MSA_F64_DKDV(DV) hipLaunchKernelGGL(attn_f64_dkdv<DV>, grid, dim3(64 * kKeyWaves), 0, st, q, k, v, dout, rs, cu, cu_blocks, row_ptr, qidx, nseq, T, Hq, G, B, compact, scale, dk, dv, part)
   MSA_F64_DIMS(MSA_F64_DKDV)
 #undef MSA_F64_DKDV
   if (split)

@@ -18,9 +18,9 @@ int attn_f64_dq_launch(const float* q, const float* k, const float* v, const flo
                        const int32_t* idx, const int32_t* cu, int nseq, int64_t T, int Hq, int G, int D, int K, int B,
                        double scale, float* dq, hipStream_t st);
 int attn_f64_dkdv_launch(const float* q, const float* k, const float* v, const float* dout, const double* rs,
-                         const int32_t* cu, const int32_t* cu_blocks, int64_t total_blocks, const int32_t* row_ptr,
-                         const int32_t* qidx, int nseq, int64_t T, int Hq, int G, int D, int B, double scale, float* dk,
-                         float* dv, void* ws, int64_t ws_bytes, hipStream_t st);
+                         const int32_t* cu, const int32_t* cu_blocks, const int32_t* row_ptr, const int32_t* qidx,
+                         int nseq, int64_t T, int Hq, int G, int D, int B, double scale, float* dk, float* dv, void* ws,
+                         int64_t ws_bytes, hipStream_t st);
 
 // FP64 partial sums of the KV pass where its rows are shared by several workgroups; 0: none.
 int64_t attn_f64_dkdv_workspace_bytes(int64_t T, int64_t G, int64_t D);

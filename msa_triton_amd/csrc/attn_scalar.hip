@@ -735,14 +735,14 @@ int attn_valu_launch_dq(const void* q, const void* k, const void* v, const void*
 
 template <int DT, int DPL>
 int attn_valu_launch_dkdv(const void* q, const void* k, const void* v, const void* dout, const double* rs,
-                          const int32_t* cu, const int32_t* cu_blocks, int64_t total_blocks, const int32_t* row_ptr,
+                          const int32_t* cu, const int32_t* cu_blocks, const int32_t* row_ptr,
                           const int32_t* qidx, int nseq, int64_t T, int Hq, int G, int D, int B, double scale, void* dk,
                           void* dv, void* ws, int64_t ws_bytes, hipStream_t st) {
   if constexpr (DT == kF32) {
     if (attn_f64_dims_fit(D, {q, k, v, dout, rs}))
       return attn_f64_dkdv_launch(static_cast<const float*>(q), static_cast<const float*>(k),
                                   static_cast<const float*>(v), static_cast<const float*>(dout), rs, cu, cu_blocks,
-                                  total_blocks, row_ptr, qidx, nseq, T, Hq, G, D, B, scale, static_cast<float*>(dk),
+                                  row_ptr, qidx, nseq, T, Hq, G, D, B, scale, static_cast<float*>(dk),
                                   static_cast<float*>(dv), ws, ws_bytes, st);
   }
   if (rows_fit(D, q, k, v, dout, rs)) {
@@ -790,10 +790,10 @@ int attn_dq_valu_dispatch(const void* q, const void* k, const void* v, const voi
 
 template <int DT>
 int attn_dkdv_valu_dispatch(const void* q, const void* k, const void* v, const void* dout, const double* rs,
-                            const int32_t* cu, const int32_t* cu_blocks, int64_t total_blocks, const int32_t* row_ptr,
+                            const int32_t* cu, const int32_t* cu_blocks, const int32_t* row_ptr,
                             const int32_t* qidx, int nseq, int64_t T, int Hq, int G, int D, int B, double scale, void* dk,
                             void* dv, void* ws, int64_t ws_bytes, hipStream_t st) {
-  return MSA_DPL_DISPATCH(D, attn_valu_launch_dkdv, q, k, v, dout, rs, cu, cu_blocks, total_blocks, row_ptr, qidx, nseq, T, Hq, G,
+  return MSA_DPL_DISPATCH(D, attn_valu_launch_dkdv, q, k, v, dout, rs, cu, cu_blocks, row_ptr, qidx, nseq, T, Hq, G,
                           D, B, scale, dk, dv, ws, ws_bytes, st);
 }
 
@@ -805,7 +805,7 @@ int attn_dkdv_valu_dispatch(const void* q, const void* k, const void* v, const v
                                          const int32_t*, const int32_t*, int, int64_t, int, int, int, int, int,      \
                                          double, void*, hipStream_t);                                                \
   template int attn_dkdv_valu_dispatch<DT>(const void*, const void*, const void*, const void*, const double*,       \
-                                           const int32_t*, const int32_t*, int64_t, const int32_t*, const int32_t*,  \
+                                           const int32_t*, const int32_t*, const int32_t*, const int32_t*,           \
                                            int, int64_t, int, int, int, int, double, void*, void*, void*, int64_t,   \
                                            hipStream_t);
 MSA_INSTANTIATE_VALU(kF32)

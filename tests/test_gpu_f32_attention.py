@@ -165,3 +165,55 @@ def test_f32_tile_of_minus_infinite_logits(dimension, device):
     assert bool((got[:16] == 0).all()) and bool((got_lse[:16] == -float("inf")).all())
     _close_f32(got[16:], out[16:], "out")
     _close_f32(got_lse[16:], lse[16:], "lse")
+
+
+def _grads(q, k, v, dout, ids, cu, longest, block):
+    leaves = [x.clone().requires_grad_() for x in (q, k, v)]
+    msa.m3_sparse_attention(*leaves, ids, cu, longest, block_size=block).backward(dout)
+    return [x.grad for x in leaves]
+
+
+@pytest.mark.parametrize("block", [1 << 20, 2 ** 31 - 17, 2 ** 31 - 1])
+def test_f32_backward_with_a_block_far_above_the_sequences(block, device):
+    """The KV pass's workgroups follow the tokens, not the block size: the same bits as with blocks
+    of the longest sequence, up to the largest block size."""
+    gen = torch.Generator(device=device).manual_seed(1)
+    lengths, ratio, dimension = [70, 3, 0, 41], 4, 64
+    total = sum(lengths)
+    q, k, v, dout = (torch.randn(total, n, dimension, generator=gen, device=device) for n in (ratio, 1, 1, ratio))
+    ids = torch.zeros(total, 1, 1, dtype=torch.int32, device=device)
+    cu = cu_tensor(lengths, device)
+    for a, b in zip(_grads(q, k, v, dout, ids, cu, 70, block), _grads(q, k, v, dout, ids, cu, 70, 70)):
+        assert torch.equal(a, b)
+
+
+def test_f32_backward_does_not_take_the_number_of_blocks_from_the_caller(device):
+    """total_blocks of msa_attn_bwd describes the edge rows of the KV-major kernels; the fp32 pass
+    writes every key whatever it says."""
+    from msa_triton_amd import _lib
+    from msa_triton_amd.k2q import build_k2q_csr
+
+    gen = torch.Generator(device=device).manual_seed(2)
+    lengths, ratio, dimension, block = [70, 41], 4, 64, 16
+    total = sum(lengths)
+    q, k, v, dout = (torch.randn(total, n, dimension, generator=gen, device=device) for n in (ratio, 1, 1, ratio))
+    ids = random_selection(total, 1, 2, lengths, block, 1, torch.Generator().manual_seed(2)).to(device)
+    cu = cu_tensor(lengths, device)
+    want = _grads(q, k, v, dout, ids, cu, 70, block)
+    csr = build_k2q_csr(ids, cu, block_size=block)
+    out, lse = torch.empty_like(q), torch.empty(total, ratio, device=device)
+    state = torch.empty(total, ratio, 4, dtype=torch.float64, device=device)
+    scale, lib, stream = dimension ** -0.5, _lib.lib(), _lib.stream_of(q.device)
+    sizes = (2, total, ratio, 1, dimension, 2, block, scale)
+    assert lib.msa_attn_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), 0, ids.data_ptr(), cu.data_ptr(), *sizes, None, 0,
+                            None, None, None, None, 0, out.data_ptr(), lse.data_ptr(), state.data_ptr(), None,
+                            stream) == 0
+    for total_blocks in (0, 1):
+        got = [torch.full_like(x, float("nan")) for x in (q, k, v)]
+        assert lib.msa_attn_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), 0, out.data_ptr(), dout.data_ptr(),
+                                state.data_ptr(), None, ids.data_ptr(), cu.data_ptr(), *sizes,
+                                csr.cu_block_lens.data_ptr(), total_blocks, csr.row_ptr.data_ptr(),
+                                csr.query_indices.data_ptr(), csr.slot_indices.data_ptr(),
+                                *(x.data_ptr() for x in got), None, 0, stream) == 0
+        for a, b, what in zip(got, want, ("dq", "dk", "dv")):
+            assert bool(((a - b).abs() <= 2.0 ** -22 * b.abs() + 1e-11).all()), (total_blocks, what)
