@@ -461,8 +461,10 @@ __global__ __launch_bounds__(64 * kKeyWaves, 2) void attn_f64_dkdv(
       if (D == 128) __builtin_amdgcn_sched_barrier(0);  // (one step's rows at a time: registers)
     }
   }
-  // the waves' sums in wave order
-  for (int w = 0; w < kKeyWaves; ++w) {
+  // the sums of the waves that had rows, in wave order
+  const int64_t steps = (nrows + 15) / 16 - kKeyWaves * static_cast<int64_t>(blockIdx.z);
+  const int waves = steps < 1 ? 1 : (steps < kKeyWaves ? static_cast<int>(steps) : kKeyWaves);
+  for (int w = 0; w < waves; ++w) {
     if (wid == w) {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
