@@ -16,7 +16,7 @@ int attn_dq_valu_dispatch(const void*, const void*, const void*, const void*, co
                           const int32_t*, int, int64_t, int, int, int, int, int, double, void*, hipStream_t);
 template <int DT>
 int attn_dkdv_valu_dispatch(const void*, const void*, const void*, const void*, const double*, const int32_t*,
-                            const int32_t*, const int32_t*, const int32_t*, int, int64_t, int, int, int, int, double,
+                            const int32_t*, const int32_t*, const int32_t*, int, int64_t, int, int, int, int, int, double,
                             void*, void*, void*, int64_t, hipStream_t);
 
 // Input types the MFMA kernels take (exact products in fp32 for both).
@@ -117,8 +117,8 @@ extern "C" int msa_attn_bwd(const void* q, const void* k, const void* v, int32_t
   }
   if (rc != kOk || !need_kv) return rc;
   switch (dtype) {
-    case kF32: return attn_dkdv_valu_dispatch<kF32>(q, k, v, grad_out, row_state, cu_seqlens, cu_block_lens, row_ptr, query_indices, nseq, total_tokens, Hq, G, D, B, scale, grad_k, grad_v, workspace, workspace_bytes, st);
-    case kF16: return attn_dkdv_valu_dispatch<kF16>(q, k, v, grad_out, row_state, cu_seqlens, cu_block_lens, row_ptr, query_indices, nseq, total_tokens, Hq, G, D, B, scale, grad_k, grad_v, workspace, workspace_bytes, st);
-    default: return attn_dkdv_valu_dispatch<kBF16>(q, k, v, grad_out, row_state, cu_seqlens, cu_block_lens, row_ptr, query_indices, nseq, total_tokens, Hq, G, D, B, scale, grad_k, grad_v, workspace, workspace_bytes, st);
+    case kF32: return attn_dkdv_valu_dispatch<kF32>(q, k, v, grad_out, row_state, cu_seqlens, cu_block_lens, row_ptr, query_indices, nseq, total_tokens, Hq, G, D, K, B, scale, grad_k, grad_v, workspace, workspace_bytes, st);
+    case kF16: return attn_dkdv_valu_dispatch<kF16>(q, k, v, grad_out, row_state, cu_seqlens, cu_block_lens, row_ptr, query_indices, nseq, total_tokens, Hq, G, D, K, B, scale, grad_k, grad_v, workspace, workspace_bytes, st);
+    default: return attn_dkdv_valu_dispatch<kBF16>(q, k, v, grad_out, row_state, cu_seqlens, cu_block_lens, row_ptr, query_indices, nseq, total_tokens, Hq, G, D, K, B, scale, grad_k, grad_v, workspace, workspace_bytes, st);
   }
 }

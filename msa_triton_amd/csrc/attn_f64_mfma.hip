@@ -24,6 +24,8 @@
 // (of u = p (dp - c) and of p) in one product: rows 0-7 of the A operand are u, 8-15 p.
 // KV pass: one workgroup per 16 keys and group, the rows (edge, head) of the block's CSR row
 // 16 at a time, dealt to 8 waves; the waves' sums are added in wave order.
+#include <algorithm>
+
 #include "attn_f64_mfma.hpp"
 
 namespace msa {
@@ -361,7 +363,7 @@ __global__ __launch_bounds__(64 * kKeyWaves, 2) void attn_f64_dkdv(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
     const float* __restrict__ dout, const double* __restrict__ row_state, const int32_t* __restrict__ cu,
     const int32_t* __restrict__ cu_blocks, const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ qidx,
-    int nseq, int64_t T, int Hq, int G, int B, int64_t compact, double scale, float* __restrict__ dk,
+    int nseq, int64_t T, int Hq, int G, int B, int64_t compact, int fewest, double scale, float* __restrict__ dk,
     float* __restrict__ dv, double* __restrict__ part) {
   constexpr int NT = D / 16;
   __shared__ double kbuf[16][D], vbuf[16][D];
@@ -406,6 +408,7 @@ __global__ __launch_bounds__(64 * kKeyWaves, 2) void attn_f64_dkdv(
   const int64_t e0 = row_ptr[row];
   const int R = Hq / G;
   const int64_t nrows = (row_ptr[row + 1] - e0) * R;
+  if (nrows * nk < fewest) return;  // whole workgroup: left to the vector kernel
   f64x4 ak[NT], av[NT];
 #pragma unroll
   for (int n = 0; n < NT; ++n) ak[n] = av[n] = f64x4{0.0, 0.0, 0.0, 0.0};
@@ -578,15 +581,23 @@ int64_t attn_f64_dkdv_workspace_bytes(int64_t T, int64_t G, int64_t D) {
   return n > 1 ? int64_t{16} * n * T * G * D : 0;
 }
 
+F64Tile attn_f64_mean_tile(int64_t T, int nseq, int R, int K, int B) {
+  const double blocks = static_cast<double>(T / B + nseq < T ? T / B + nseq : T), keys = T / blocks;
+  const double slots = std::min<double>(K, (std::max(1.0, blocks / nseq) + 1) / 2);  // that exist
+  return F64Tile{R * keys * slots, std::min(16.0, keys)};
+}
+
 int attn_f64_dkdv_launch(const float* q, const float* k, const float* v, const float* dout, const double* rs,
                          const int32_t* cu, const int32_t* cu_blocks, const int32_t* row_ptr, const int32_t* qidx,
-                         int nseq, int64_t T, int Hq, int G, int D, int B, double scale, float* dk, float* dv, void* ws,
-                         int64_t ws_bytes, hipStream_t st) {
+                         int nseq, int64_t T, int Hq, int G, int D, int K, int B, int fewest, double scale, float* dk,
+                         float* dv, void* ws, int64_t ws_bytes, hipStream_t st) {
   // a caller without the workspace gets the unsplit pass
   const int64_t need = attn_f64_dkdv_workspace_bytes(T, G, D);
   const bool split = ws && need > 0 && ws_bytes >= need && (reinterpret_cast<uintptr_t>(ws) & 7) == 0;
-  const int splits = split ? dkdv_splits(T, G) : 1;
-  double* part = split ? static_cast<double*>(ws) : nullptr;
+  // (a share of at least two steps on average: with fewer its zeros and the sum cost more than they give)
+  const double most = attn_f64_mean_tile(T, nseq, Hq / G, K, B).rows / 32;
+  const int splits = split ? std::max(1, static_cast<int>(std::min<double>(dkdv_splits(T, G), most))) : 1;
+  double* part = splits > 1 ? static_cast<double*>(ws) : nullptr;
   // One workgroup per tile of every block, a block's tiles side by side (they gather the same rows; with
   // one block's tiles far apart 4 sequences of 2048 tokens took 8790 us for the backward, so 6257), or,
   // where whole blocks would give more than two numbers per tile (short sequences, blocks far longer
@@ -597,10 +608,10 @@ int attn_f64_dkdv_launch(const float* q, const float* k, const float* v, const f
   const int64_t per_block = (static_cast<int64_t>(B) + 15) / 16;
   const int64_t compact = per_block * blocks > 2 * tiles ? (tiles + 1) / 2 : 0;
   const dim3 grid(static_cast<unsigned>((compact ? 2 * compact : blocks * per_block) * G), 1, splits);
-#define MSA_F64_DKDV(DV) hipLaunchKernelGGL(attn_f64_dkdv<DV>, grid, dim3(64 * kKeyWaves), 0, st, q, k, v, dout, rs, cu, cu_blocks, row_ptr, qidx, nseq, T, Hq, G, B, compact, scale, dk, dv, part)
+#define MSA_F64_DKDV(DV) hipLaunchKernelGGL(attn_f64_dkdv<DV>, grid, dim3(64 * kKeyWaves), 0, st, q, k, v, dout, rs, cu, cu_blocks, row_ptr, qidx, nseq, T, Hq, G, B, compact, fewest, scale, dk, dv, part)
   MSA_F64_DIMS(MSA_F64_DKDV)
 #undef MSA_F64_DKDV
-  if (split)
+  if (splits > 1)
     hipLaunchKernelGGL(attn_f64_dkdv_reduce, dim3(grid_1d(T * G * D, 256)), dim3(256), 0, st, part, splits, T * G * D, dk,
                        dv);
   return status_from(hipGetLastError());

@@ -474,7 +474,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_valu(
     const void* __restrict__ q, const void* __restrict__ k, const void* __restrict__ v,
     const void* __restrict__ dout, const double* __restrict__ row_state, const int32_t* __restrict__ cu, const int32_t* __restrict__ cu_blocks, const int32_t* __restrict__ row_ptr,
     const int32_t* __restrict__ qidx, int nseq, int64_t T, int Hq, int G, int D, int B, double scale,
-    void* __restrict__ dk, void* __restrict__ dv, int dc0) {
+    void* __restrict__ dk, void* __restrict__ dv, int few_only, int dc0) {
   const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int64_t jg = static_cast<int64_t>(blockIdx.x) * 4 + wid;
   if (jg >= T * G) return;
@@ -485,6 +485,10 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_valu(
   const int64_t row = (static_cast<int64_t>(cu_blocks[s]) + blk) * G + g;
   const int64_t e0 = row_ptr[row], e1 = row_ptr[row + 1];
   const int R = Hq / G;
+  if (few_only) {  // the other keys are the matrix kernel's
+    const int64_t first = cu[s] + blk * B, end = first + B < cu[s + 1] ? first + B : cu[s + 1];
+    if (!f64_few_pairs((e1 - e0) * R, j - first, end - first)) return;  // whole wave
+  }
   // This launch's dims are dc0 + lane + 64 i (i < DPL). When they are all of D the key
   // and value rows stay in registers for the logits; otherwise (D above 64 x DPL, one
   // launch per 64 DPL dims) the logits loop over every dim from memory, in the same order.
@@ -555,7 +559,8 @@ __global__ __launch_bounds__(256, DT == kF32 || NC == 2 ? 2 : 3) void attn_bwd_d
     const void* __restrict__ q, const void* __restrict__ k, const void* __restrict__ v,
     const void* __restrict__ dout, const double* __restrict__ row_state, const int32_t* __restrict__ cu,
     const int32_t* __restrict__ cu_blocks, const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ qidx,
-    int nseq, int64_t T, int Hq, int G, int D, int B, double scale, void* __restrict__ dk, void* __restrict__ dv) {
+    int nseq, int64_t T, int Hq, int G, int D, int B, double scale, void* __restrict__ dk, void* __restrict__ dv,
+    int few_only) {
   constexpr int RPW = kWave / LPR;
   const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int64_t jg = static_cast<int64_t>(blockIdx.x) * 4 + wid;
@@ -568,6 +573,10 @@ __global__ __launch_bounds__(256, DT == kF32 || NC == 2 ? 2 : 3) void attn_bwd_d
   const int64_t row = (static_cast<int64_t>(cu_blocks[s]) + blk) * G + g;
   const int64_t e0 = row_ptr[row], e1 = row_ptr[row + 1];
   const int R = Hq / G;
+  if (few_only) {  // the other keys are the matrix kernel's
+    const int64_t first = cu[s] + blk * B, end = first + B < cu[s + 1] ? first + B : cu[s + 1];
+    if (!f64_few_pairs((e1 - e0) * R, j - first, end - first)) return;  // whole wave
+  }
   constexpr int E = 8 * NC;  // dims per lane: [E dch, E dch + E)
   float kr[E], vr[E];
 #pragma unroll
@@ -736,17 +745,25 @@ int attn_valu_launch_dq(const void* q, const void* k, const void* v, const void*
 template <int DT, int DPL>
 int attn_valu_launch_dkdv(const void* q, const void* k, const void* v, const void* dout, const double* rs,
                           const int32_t* cu, const int32_t* cu_blocks, const int32_t* row_ptr,
-                          const int32_t* qidx, int nseq, int64_t T, int Hq, int G, int D, int B, double scale, void* dk,
-                          void* dv, void* ws, int64_t ws_bytes, hipStream_t st) {
+                          const int32_t* qidx, int nseq, int64_t T, int Hq, int G, int D, int K, int B, double scale,
+                          void* dk, void* dv, void* ws, int64_t ws_bytes, hipStream_t st) {
+  int few_only = 0;
   if constexpr (DT == kF32) {
-    if (attn_f64_dims_fit(D, {q, k, v, dout, rs}))
-      return attn_f64_dkdv_launch(static_cast<const float*>(q), static_cast<const float*>(k),
-                                  static_cast<const float*>(v), static_cast<const float*>(dout), rs, cu, cu_blocks,
-                                  row_ptr, qidx, nseq, T, Hq, G, D, B, scale, static_cast<float*>(dk),
-                                  static_cast<float*>(dv), ws, ws_bytes, st);
+    if (attn_f64_dims_fit(D, {q, k, v, dout, rs})) {
+      // The tiles with few pairs are looked for where the mean tile has at most four times as few:
+      // elsewhere there can be some, but the launch costs more than they do.
+      const F64Tile mean = attn_f64_mean_tile(T, nseq, Hq / G, K, B);
+      few_only = mean.rows * mean.keys < 4 * kF64FewestPairs;
+      const int rc = attn_f64_dkdv_launch(static_cast<const float*>(q), static_cast<const float*>(k),
+                                          static_cast<const float*>(v), static_cast<const float*>(dout), rs, cu,
+                                          cu_blocks, row_ptr, qidx, nseq, T, Hq, G, D, K, B,
+                                          few_only ? kF64FewestPairs : 0, scale, static_cast<float*>(dk),
+                                          static_cast<float*>(dv), ws, ws_bytes, st);
+      if (rc != kOk || !few_only) return rc;
+    }
   }
   if (rows_fit(D, q, k, v, dout, rs)) {
-#define MSA_DKDV_ROWS(LPRV, NCV) hipLaunchKernelGGL((attn_bwd_dkdv_rows<DT, LPRV, NCV>), dim3(grid_1d(T * G, 4)), dim3(256), 0, st, q, k, v, dout, rs, cu, cu_blocks, row_ptr, qidx, nseq, T, Hq, G, D, B, scale, dk, dv)
+#define MSA_DKDV_ROWS(LPRV, NCV) hipLaunchKernelGGL((attn_bwd_dkdv_rows<DT, LPRV, NCV>), dim3(grid_1d(T * G, 4)), dim3(256), 0, st, q, k, v, dout, rs, cu, cu_blocks, row_ptr, qidx, nseq, T, Hq, G, D, B, scale, dk, dv, few_only)
     switch (D) {  // 2-byte types at D = 128: 16 dims a lane; otherwise 8
       case 8: MSA_DKDV_ROWS(1, 1); break;
       case 16: MSA_DKDV_ROWS(2, 1); break;
@@ -762,7 +779,7 @@ int attn_valu_launch_dkdv(const void* q, const void* k, const void* v, const voi
   }
   for (int dc0 = 0; dc0 < D; dc0 += DPL * kWave)
     hipLaunchKernelGGL((attn_bwd_dkdv_valu<DT, DPL>), dim3(grid_1d(T * G, 4)), dim3(256), 0, st, q, k, v, dout, rs,
-                       cu, cu_blocks, row_ptr, qidx, nseq, T, Hq, G, D, B, scale, dk, dv, dc0);
+                       cu, cu_blocks, row_ptr, qidx, nseq, T, Hq, G, D, B, scale, dk, dv, few_only, dc0);
   return status_from(hipGetLastError());
 }
 
@@ -791,10 +808,10 @@ int attn_dq_valu_dispatch(const void* q, const void* k, const void* v, const voi
 template <int DT>
 int attn_dkdv_valu_dispatch(const void* q, const void* k, const void* v, const void* dout, const double* rs,
                             const int32_t* cu, const int32_t* cu_blocks, const int32_t* row_ptr,
-                            const int32_t* qidx, int nseq, int64_t T, int Hq, int G, int D, int B, double scale, void* dk,
-                            void* dv, void* ws, int64_t ws_bytes, hipStream_t st) {
+                            const int32_t* qidx, int nseq, int64_t T, int Hq, int G, int D, int K, int B, double scale,
+                            void* dk, void* dv, void* ws, int64_t ws_bytes, hipStream_t st) {
   return MSA_DPL_DISPATCH(D, attn_valu_launch_dkdv, q, k, v, dout, rs, cu, cu_blocks, row_ptr, qidx, nseq, T, Hq, G,
-                          D, B, scale, dk, dv, ws, ws_bytes, st);
+                          D, K, B, scale, dk, dv, ws, ws_bytes, st);
 }
 
 #define MSA_INSTANTIATE_VALU(DT)                                                                                    \
@@ -806,8 +823,8 @@ int attn_dkdv_valu_dispatch(const void* q, const void* k, const void* v, const v
                                          double, void*, hipStream_t);                                                \
   template int attn_dkdv_valu_dispatch<DT>(const void*, const void*, const void*, const void*, const double*,       \
                                            const int32_t*, const int32_t*, const int32_t*, const int32_t*,           \
-                                           int, int64_t, int, int, int, int, double, void*, void*, void*, int64_t,   \
-                                           hipStream_t);
+                                           int, int64_t, int, int, int, int, int, double, void*, void*, void*,       \
+                                           int64_t, hipStream_t);
 MSA_INSTANTIATE_VALU(kF32)
 MSA_INSTANTIATE_VALU(kF16)
 MSA_INSTANTIATE_VALU(kBF16)

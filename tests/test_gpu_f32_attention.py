@@ -21,8 +21,13 @@ def _close_f32(actual, expected, what):
     assert worst <= 1e-11, f"{what}: {worst}"
 
 
+_FEW = [1] * 9 + [2, 0, 3, 5, 130, 1, 33]
+
+
 @pytest.mark.parametrize("dimension", [32, 64, 96, 128])
 @pytest.mark.parametrize("lengths,groups,ratio,block,topk", [
+    # tiles with fewer than 100 (row, key) pairs (the KV pass's vector kernel) beside others
+    (_FEW, 2, 4, 16, 3), (_FEW, 1, 1, 128, 2), ([60, 41], 2, 1, 5, 4), ([100], 1, 6, 1, 8),
     ([1], 1, 8, 128, 1), ([17, 0, 15, 130], 2, 4, 16, 3), ([300, 33], 1, 8, 128, 2), ([95, 64], 2, 3, 5, 6),
     ([210], 1, 5, 100, 2), ([257], 2, 8, 200, 1), ([40, 90], 2, 2, 24, 3), ([70], 1, 12, 16, 4),
 ])
