@@ -17,6 +17,8 @@
 // block's rows once per row segment and adds each row into its winner's FP64 LDS
 // row (rows in order; segments summed in order). Both accumulate in FP64 in a fixed
 // order (no float atomics), then round to the input dtype.
+#include <algorithm>
+
 #include "common.hpp"
 #include "score_mfma.hpp"
 #include "topk_row.hpp"
@@ -375,18 +377,44 @@ __device__ __forceinline__ void dk_add_row(double (&acc)[8], double wgt, const v
   }
 }
 
-// Rows per segment: 8192 (long sequences: every key block has many segments), or 2048 where
-// that leaves the chip short of workgroups, as long as the FP64 partial sums stay at 4096
-// (block, segment) pairs. Measured (score backward's dk pass and reduction, Di = 128, 4 groups):
-// sequences of 2048 to 6144 tokens, 128 blocks: 183 + 13 us with 8192 rows, 126 + 16 us with 2048
-// (eight waves per workgroup instead of four: 133 + 16).
+// Rows per segment. kDkSegLong, or kDkSegShort where that leaves the chip short of workgroups: a key
+// block's rows are then shared by up to four times as many, at four times the FP64 partial sums
+// (written, read and added). Measured, score backward, Di = 128 in bf16, 4 groups, blocks of 128 keys,
+// us with long / short segments: one sequence of 4096 tokens 143 / 92, of 8192 176 / 191, of 16384
+// 381 / 505; 4 of 4096 240 / 222, 8 of 4096 376 / 450, 16 of 2048 325 / 327, 64 of 1024 485 / 549.
+// That is in units, 128 keys times the long segments that they meet (and one for the straddled one):
+// 96, 320, 1152; 384, 768, 512, 1024. Up to 512 take the short segments. Blocks above 128 keys read their
+// rows once per 128 keys, so count as many times: one of 8192 tokens in blocks of 256 133 / 173 (640
+// units). A sequence of one short segment is not split any further: 64 sequences of 256 tokens,
+// 2 groups, 101 / 118 (256 units); there 128 units are the limit.
+// The passes for other dims and fp32 spend far longer on each row (fp32, 4 of 4096 tokens, 1329 /
+// 572; Di = 64, one of 16384 1042 / 744; Di = 512, 4 of 4096 4951 / 3497): short segments
+// wherever their sums stay within kDkShortBytes (Di = 256, 8 of 4096, 576 MiB: 2373 / 2601).
+// That bounds what the short segments add to the workspace.
 constexpr int kDkSegLong = 8192, kDkSegShort = 2048;
-static int dk_seg(int64_t rows, int64_t total_blocks) {
-  return total_blocks * ((rows + kDkSegShort - 1) / kDkSegShort) <= 4096 ? kDkSegShort : kDkSegLong;
-}
-static int64_t dk_nseg(int64_t rows, int64_t total_blocks) {
-  const int64_t seg = dk_seg(rows, total_blocks);
-  return (rows + seg - 1) / seg;
+constexpr int64_t kDkShortBytes = int64_t{512} << 20;
+struct DkSegments {
+  int rows;            // per segment
+  int64_t all;         // segments of the row space
+  int64_t per_block;   // those of one key block, at most: the longest sequence's, and one more as
+                       // segments are aligned to the row space and not to the sequence
+  int64_t part_bytes;  // of the partial sums
+};
+// gathers16: 2-byte rows of 128 dims (the pass with 16-byte gathers).
+static DkSegments dk_segments(int64_t rows, int64_t G, int64_t NB, int64_t B, int64_t Di, int64_t total_blocks,
+                              bool gathers16) {
+  const int64_t seq_rows = std::min(rows, NB > rows / G / B ? rows : NB * B * G);
+  const int64_t keys = (B + 127) / 128 * 128;
+  auto of = [&](int seg) {
+    const int64_t all = (rows + seg - 1) / seg, own = std::min(all, (seq_rows + seg - 1) / seg + 1);
+    return DkSegments{seg, all, own, total_blocks * own * keys * Di * 8};
+  };
+  const DkSegments l = of(kDkSegLong), s = of(kDkSegShort);
+  const int64_t units = (rows / G + 127) / 128 * (1 + (seq_rows + kDkSegLong - 1) / kDkSegLong) * ((B + 127) / 128);
+  bool use_short = s.part_bytes <= kDkShortBytes;
+  if (seq_rows <= kDkSegShort) use_short = use_short && units <= 128;
+  else if (gathers16) use_short = use_short && units <= 512;
+  return use_short ? s : l;
 }
 constexpr int kDkBatch = 16;
 constexpr int kDkWideUnroll = 4;  // row-gather instructions per batch (4 rows each; two batches in flight)
@@ -417,9 +445,7 @@ __global__ __launch_bounds__(256, DPL >= 8 ? 2 : (SEG == kDkSegShort ? 4 : 3)) v
   // two 2 MiB segments of index_q. Workgroups go to the 8 XCDs round-robin, so consecutive
   // pairs run on different XCDs (contiguous runs of L per XCD would load them unevenly: the
   // nonempty pairs are concentrated in the low segments at one long sequence).
-  const int64_t nwork = nblk * nseg;
   const int64_t lw = blockIdx.x;
-  if (lw >= nwork) return;  // whole workgroup (padding)
   const int64_t S = lw / nblk;
   const int64_t gb = lw % nblk;
   const int kc = blockIdx.y, kchunks = gridDim.y;
@@ -794,9 +820,10 @@ int score_bwd_launch(const void* iq, const void* ik, const int32_t* cu, const in
     double* part = reinterpret_cast<double*>(ds_t + rows * NB);  // 8 * rows * NB bytes in: 8-byte aligned
     const dim3 tgrid(grid_1d(rows, 64), static_cast<unsigned>((NB + 63) / 64));
     hipLaunchKernelGGL(score_bwd_transpose, tgrid, dim3(256), 0, st, tie, ds, rows, NB, cu, nseq, G, B, tie_t, ds_t);
-    const int seg = dk_seg(rows, total_blocks), nseg = static_cast<int>(dk_nseg(rows, total_blocks));
+    const DkSegments segs = dk_segments(rows, G, NB, B, Di, total_blocks, DT != kF32 && Di == 128);
+    const int seg = segs.rows, nseg = static_cast<int>(segs.per_block);
     const int kchunks = (B + 127) / 128;
-    const dim3 grid(static_cast<unsigned>(total_blocks * nseg), static_cast<unsigned>(kchunks));
+    const dim3 grid(static_cast<unsigned>(total_blocks * segs.all), static_cast<unsigned>(kchunks));
 #define MSA_DK_PART_SEG(DPLV, DC0, SEGV) hipLaunchKernelGGL((score_bwd_dk_part<DT, DPLV, SEGV>), grid, dim3(256), 0, st, iq, ik, cu, cu_blocks, nseq, tie_t, ds_t, rows, G, Di, B, total_blocks, nseg, scale, part, DC0)
 #define MSA_DK_PART(DPLV, DC0) \
   if (seg == kDkSegShort) MSA_DK_PART_SEG(DPLV, DC0, kDkSegShort); else MSA_DK_PART_SEG(DPLV, DC0, kDkSegLong)
@@ -875,9 +902,10 @@ extern "C" int64_t msa_score_bwd_workspace_bytes(int64_t total_tokens, int64_t g
   const int64_t rows = total_tokens * groups;
   // block-major tie / ds copies, then the dk partial sums (FP64)
   const int64_t tr = rows * num_blocks * 8 + 8;
-  const int64_t nseg = dk_nseg(rows, total_blocks);
-  const int64_t kchunks = (block_size + 127) / 128;
-  const int64_t part = total_blocks * nseg * kchunks * 128 * index_dim * 8;
+  // (the input type is not known here: the larger of the two passes')
+  int64_t part = 0;
+  for (const bool gathers16 : {false, index_dim == 128})
+    part = std::max(part, dk_segments(rows, groups, num_blocks, block_size, index_dim, total_blocks, gathers16).part_bytes);
   return tr + part + 256;
 }
 

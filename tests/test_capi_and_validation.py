@@ -45,6 +45,24 @@ def test_library_exports_every_declared_symbol():
     assert set(_lib.SIGNATURES) == set(decls)
 
 
+@pytest.mark.parametrize("tokens,groups,dim,block", [
+    (16384, 4, 128, 128), (16384, 4, 512, 128), (32768, 4, 128, 1024), (65536, 8, 512, 4096), (8192, 4, 128, 1),
+])
+def test_score_backward_workspace_of_short_segments_is_bounded(tokens, groups, dim, block):
+    """Beyond the block-major copies of tie and ds, the partial sums take what segments of 8192 rows
+    need, or at most 512 MiB; and no more for a pack than its longest sequence needs."""
+    rows, blocks = tokens * groups, tokens // block
+    copies = rows * blocks * 8 + 8 + 256
+    chunk = (block + 127) // 128 * 128 * dim * 8
+    bytes_of = _lib.lib().msa_score_bwd_workspace_bytes
+    assert bytes_of(tokens, groups, blocks, dim, block, blocks) <= copies + max(
+        blocks * -(-rows // 8192) * chunk, 512 << 20)
+    if blocks >= 8:  # eight sequences
+        own = -(-rows // 8 // 8192) + 1
+        assert bytes_of(tokens, groups, blocks // 8, dim, block, blocks) <= copies + max(
+            blocks * own * chunk, 512 << 20)
+
+
 def test_host_only_helpers():
     handle = _lib.lib()
     cb = np.array([0, 2, 3], dtype=np.int32)

@@ -365,18 +365,33 @@ def test_score_mfma_path_equals_the_exact_kernel(values, lengths, groups, dim, b
 @pytest.mark.parametrize("tokens,block", [(1023, 64), (1025, 128), (2600, 1)])
 def test_score_backward_row_segments(tokens, block, dtype, dim, device):
     """The key-block pass at the edges of its 2048-row segments (two groups: 1024 tokens) and,
-    with blocks of one key, with more (block, segment) pairs than the short segments are used
-    for: gradients against the float64 sums over the winners."""
-    gen = torch.Generator().manual_seed(tokens)
-    lengths, groups = [tokens, 70], 2
-    total, nb = tokens + 70, -(-tokens // block)
+    with blocks of one key, with larger partial sums than the short segments are used for (128
+    dims): gradients against the float64 sums over the winners."""
+    _check_score_backward([tokens, 70], 2, block, dtype, dim, device)
+
+
+@pytest.mark.parametrize("dtype,dim", [(torch.bfloat16, 128), (torch.float16, 64), (torch.float32, 40)])
+@pytest.mark.parametrize("lengths,groups,block", [
+    ([900, 2050, 70, 1100], 2, 128),  # sums for the longest sequence's segments, not the pack's
+    ([130, 700, 1024, 900], 4, 64),   # sequences that straddle segments of 2048 rows
+    ([700] * 5, 3, 300),              # blocks of more than 128 keys
+    ([400] * 30, 5, 128),             # sequences of one short segment, and enough of them for the long ones
+])
+def test_score_backward_segments_of_packed_sequences(lengths, groups, block, dtype, dim, device):
+    _check_score_backward(lengths, groups, block, dtype, dim, device)
+
+
+def _check_score_backward(lengths, groups, block, dtype, dim, device):
+    gen = torch.Generator().manual_seed(lengths[0])
+    total, longest = sum(lengths), max(lengths)
+    nb, bounds = -(-longest // block), cu_list(lengths)
     q = torch.randn(total, groups, dim, generator=gen).to(dtype).to(device).requires_grad_()
     k = torch.randn(total, 1, dim, generator=gen).to(dtype).to(device).requires_grad_()
-    scores = msa.m3_index_score(q, k, cu_tensor(lengths, device), tokens, block_size=block)
+    scores = msa.m3_index_score(q, k, cu_tensor(lengths, device), longest, block_size=block)
     ds = torch.randn((total, groups, nb), generator=gen).to(device)
     scores.backward(ds)
     dq, dk = torch.zeros_like(q, dtype=torch.float64), torch.zeros(total, dim, dtype=torch.float64, device=device)
-    for a, b in ((0, tokens), (tokens, total)):
+    for a, b in zip(bounds, bounds[1:]):
         n, m = b - a, -(-(b - a) // block)
         s = (q[a:b].detach().double().reshape(-1, dim) @ k[a:b, 0].detach().double().T).view(n, groups, n)
         s = s.masked_fill(torch.ones(n, n, dtype=torch.bool, device=device).triu(1)[:, None], float("-inf"))
@@ -386,7 +401,8 @@ def test_score_backward_row_segments(tokens, block, dtype, dim, device):
         w = w.view(n * groups, m * block)[:, :n]
         dq[a:b] = (w @ k[a:b, 0].detach().double()).view(n, groups, dim)
         dk[a:b] = w.T @ q[a:b].detach().double().reshape(-1, dim)
-    # one rounding to the output type (2^-9 / 2^-25 of a value), from FP64 sums
-    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -23
-    assert bool(((q.grad.double() - dq).abs() <= eps * dq.abs() + 1e-12).all())
-    assert bool(((k.grad[:, 0].double() - dk).abs() <= eps * dk.abs() + 1e-12).all())
+    # one rounding to the output type (2^-9, 2^-12 or 2^-25 of a value; fp16 subnormals 2^-25), from FP64 sums
+    eps = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -10, torch.float32: 2.0 ** -23}[dtype]
+    tiny = 2.0 ** -24 if dtype == torch.float16 else 1e-12
+    assert bool(((q.grad.double() - dq).abs() <= eps * dq.abs() + tiny).all())
+    assert bool(((k.grad[:, 0].double() - dk).abs() <= eps * dk.abs() + tiny).all())
