@@ -213,6 +213,12 @@ __device__ __forceinline__ uint32_t bitonic_sort_u32(uint32_t x) {
 // 64-bit maximum per slot: 65 536 tokens x 8 groups, 512 blocks, 32 slots 757 -> 325 us;
 // 32 768 x 4, 256 blocks, 16 slots 71 -> 52 us.
 constexpr int kSelectMostSlots = 64, kSelectPairSlots = 24;
+// A row's threshold and two sorts cost the same for one slot as for 24, the argmax of topk_row16 by
+// the slot: rows of up to 128 (256) blocks take that one up to these many slots. Argmax / sort, us,
+// 262 144 rows: 128 blocks with 4 slots 49 / 83, 10 65 / 85, 12 74 / 84, 16 87 / 83; 256 blocks with 4 76 / 97, 8 93 /
+// 100, 10 101 / 100; 16 384 rows: 128 blocks with 4 5.4 / 7.4, 10 7.6 / 7.6, 256 with 7 9.3 / 8.6; 257 blocks and
+// more: sort (320 blocks, one slot, 262 144 rows: 202 / 107).
+constexpr int kArgmaxSlots128 = 11, kArgmaxSlots256 = 7;
 template <int VPL, int CAP>
 __device__ __forceinline__ void topk_threshold(const float* __restrict__ scores, const int32_t* __restrict__ cu,
                                                int nseq, int64_t rows, int G, int NB, int B, int K, int L,
@@ -316,8 +322,8 @@ __device__ __forceinline__ void topk_threshold(const float* __restrict__ scores,
 }
 
 // Host launch of the stand-alone selection (topk.hip): 16-lane rows up to 64 blocks,
-// threshold and sort up to 1024 (16-lane rows there for more than 64 slots), one wavefront
-// per row with the row in registers up to 4096, streamed above.
+// threshold and sort up to 1024 (16-lane rows there for more than 64 slots, and up to 256
+// blocks for few), one wavefront per row with the row in registers up to 4096, streamed above.
 int topk_launch(const float* scores, const int32_t* cu_seqlens, int nseq, int64_t rows, int G, int NB, int B, int K,
                 int L, int32_t* indices, hipStream_t st);
 

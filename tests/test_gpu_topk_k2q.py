@@ -216,7 +216,7 @@ def test_topk_rows_beyond_4096_blocks(tokens, block, k, local, device):
     np.testing.assert_array_equal(got.cpu().numpy(), ref)
 
 
-@pytest.mark.parametrize("blocks,topk,local", [(65, 1, 0), (128, 24, 1), (129, 25, 2), (200, 64, 0), (300, 16, 3),
+@pytest.mark.parametrize("blocks,topk,local", [(128, 11, 1), (128, 12, 1), (129, 7, 2), (256, 8, 0), (65, 1, 0), (128, 24, 1), (129, 25, 2), (200, 64, 0), (300, 16, 3),
                                                (512, 32, 2), (513, 33, 1), (700, 65, 1), (1024, 24, 24),
                                                (1024, 64, 1)])
 @pytest.mark.parametrize("kind", ["normal", "ties", "equal", "special"])
