@@ -47,6 +47,7 @@
 // next block barrier.
 // A negative scale flips the query signs once (exact), so every comparison is
 // on the directed dot.
+#include <algorithm>
 #include <type_traits>
 
 #include "mfma_util.hpp"
@@ -970,16 +971,19 @@ __device__ __forceinline__ double from_ordered_f64(uint64_t k) {
   return __longlong_as_double(static_cast<long long>((k >> 63) ? (k & ~(uint64_t(1) << 63)) : ~k));
 }
 
-// The ambiguous (row, block) pairs the main pass marked, settled exactly. One wave per block
-// and kResolveRows rows: it lists the marked rows in order and takes up to 16 of them (of one
-// sequence) at a time. Their MFMA logits against the block are formed again, operands
+// The ambiguous (row, block) pairs the main pass marked, settled exactly. For a block and
+// kResolveRows rows one wave, or where that gives the chip few (calls of few blocks: short
+// sequences) up to kResolveShares, lists the marked rows in order and takes its share of them, up
+// to 16 (of one sequence) at a time: about 4 us each, one after the other (341 sequences of 24
+// tokens, 2 groups, fp32: 4 waves 165 us, the selection 294, now 91; shared beyond 512 waves the groups
+// are smaller and there are more of them: 64 blocks, 8192 tokens, 4 groups, fp16, 2048 waves: 131 for 127). Their MFMA logits against the block are formed again, operands
 // straight from memory; the keys within the error bound of a row's maximum (all visible keys
 // where the row or the block is not safe) are its candidates, two or three of 128 for most
 // rows. The candidates of the 16 rows are spread over the lanes, one exact_dot each; the
 // maximum, its count and the first winner come from integer LDS atomics, so the result does
 // not depend on their order. (Re-evaluating every key of the block in FP64 took 133 us at
 // 32 768 tokens x 4 groups in bf16, this pass 54 us.)
-constexpr int kResolveGroup = 16;
+constexpr int kResolveGroup = 16, kResolveShares = 64, kResolveWaves = 512;
 template <int DT>
 __global__ __launch_bounds__(64) void score_fwd_resolve(const void* __restrict__ iq, const void* __restrict__ ik,
                                                         const int32_t* __restrict__ cu, int nseq, int64_t rows_pad,
@@ -1013,9 +1017,11 @@ __global__ __launch_bounds__(64) void score_fwd_resolve(const void* __restrict__
     count[0] = __shfl(incl, 63, kWave);
   }
   __syncthreads();
-  const int n = __builtin_amdgcn_readfirstlane(count[0]);
+  // (the lists are in order, so a share's groups are those of its rows: each row once)
+  const int marked = __builtin_amdgcn_readfirstlane(count[0]), shares = gridDim.z;
+  const int n = marked * (static_cast<int>(blockIdx.z) + 1) / shares;
   const bool neg = scale < 0.0;
-  for (int i = 0; i < n;) {
+  for (int i = marked * static_cast<int>(blockIdx.z) / shares; i < n;) {
     const int64_t row0 = c0 + __builtin_amdgcn_readfirstlane(list[i]);
     const int s = find_seq(cu, nseq, row0 / G);
     const int64_t start = cu[s], end = cu[s + 1];
@@ -1191,8 +1197,10 @@ static int launch(const void* iq, const void* ik, const int32_t* cu, int nseq, i
     else { if (fd) MSA_SCORE_MFMA(4, true); else MSA_SCORE_MFMA(4, false); }
 #undef MSA_SCORE_MFMA
   }
-  hipLaunchKernelGGL(score_fwd_resolve<DT>, dim3(NB, static_cast<unsigned>(rows_pad / kResolveRows)), dim3(64), 0, st,
-                     iq, ik, cu, nseq, rows_pad, G, Di, NB, B, scale, bnorm, amb, scores, tie);
+  const int64_t chunks = rows_pad / kResolveRows;
+  const int64_t shares = std::max<int64_t>(1, std::min<int64_t>(kResolveShares, kResolveWaves / (NB * chunks)));
+  hipLaunchKernelGGL(score_fwd_resolve<DT>, dim3(NB, static_cast<unsigned>(chunks), static_cast<unsigned>(shares)), dim3(64), 0,
+                     st, iq, ik, cu, nseq, rows_pad, G, Di, NB, B, scale, bnorm, amb, scores, tie);
   return status_from(hipGetLastError());
 }
 
