@@ -60,6 +60,7 @@ namespace {
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 
 constexpr int kTileRows = 128;  // 4 waves x 32 rows
+constexpr int kShortSeq = 16;   // tokens of the longest sequence that score_fwd_short takes
 constexpr int kThreads = 256;
 
 // Workspace: squared key norms (fp32 per key), the key blocks' norms (fp32, at each
@@ -298,16 +299,17 @@ __device__ __forceinline__ int last_block_of(const int32_t* __restrict__ cu, int
   return static_cast<int>((t - start) / B);
 }
 
-// Next (s, b) after c; s == nseq when the tile has no more blocks.
+// Next (s, b) after c; s == nseq when the tile has no more blocks. Sequences of up to `shortest`
+// tokens (0: the empty ones) are left out.
 __device__ __forceinline__ BlockCursor next_block(const int32_t* __restrict__ cu, int nseq, BlockCursor c,
-                                                  int64_t r0, int nr, int G, int B) {
+                                                  int64_t r0, int nr, int G, int B, int shortest) {
   if (c.b < c.b_last) {
     ++c.b;
     return c;
   }
   const int64_t t_last = (r0 + nr - 1) / G;
   for (int s = c.s + 1; s < nseq && cu[s] <= t_last; ++s) {
-    if (cu[s + 1] > cu[s]) return BlockCursor{s, 0, last_block_of(cu, s, r0, nr, G, B)};
+    if (cu[s + 1] - cu[s] > shortest) return BlockCursor{s, 0, last_block_of(cu, s, r0, nr, G, B)};
   }
   return BlockCursor{nseq, 0, -1};
 }
@@ -315,17 +317,17 @@ __device__ __forceinline__ BlockCursor next_block(const int32_t* __restrict__ cu
 // Part `part` of `parts` equal runs of the tile's (sequence, block) pairs: its first pair and
 // their number.
 __device__ __forceinline__ BlockCursor tile_share(const int32_t* __restrict__ cu, int nseq, int64_t r0, int nr, int G,
-                                                  int B, int part, int parts, int& todo) {
+                                                  int B, int shortest, int part, int parts, int& todo) {
   const int64_t t_last = (r0 + nr - 1) / G;
   const int s0 = find_seq(cu, nseq, r0 / G);
   int pairs = 0;
   for (int s = s0; s < nseq && cu[s] <= t_last; ++s)
-    if (cu[s + 1] > cu[s]) pairs += last_block_of(cu, s, r0, nr, G, B) + 1;
+    if (cu[s + 1] - cu[s] > shortest) pairs += last_block_of(cu, s, r0, nr, G, B) + 1;
   int skip = static_cast<int>(static_cast<int64_t>(pairs) * part / parts);
   todo = static_cast<int>(static_cast<int64_t>(pairs) * (part + 1) / parts) - skip;
   if (todo <= 0) return BlockCursor{nseq, 0, -1};
   for (int s = s0; s < nseq && cu[s] <= t_last; ++s) {
-    if (cu[s + 1] <= cu[s]) continue;
+    if (cu[s + 1] - cu[s] <= shortest) continue;
     const int last = last_block_of(cu, s, r0, nr, G, B);
     if (skip <= last) return BlockCursor{s, skip, last};
     skip -= last + 1;
@@ -380,8 +382,9 @@ __device__ __forceinline__ float signed_norm2(const void* __restrict__ ik, int64
 // the shuffles).
 template <int DT>
 __global__ __launch_bounds__(256) void score_block_norms(const void* __restrict__ ik, const int32_t* __restrict__ cu,
-                                                         int nseq, int64_t T, int Di, int B, float* __restrict__ bnorm,
-                                                         uint32_t* __restrict__ amb, int64_t amb_words) {
+                                                         int nseq, int64_t T, int Di, int B, int shortest,
+                                                         float* __restrict__ bnorm, uint32_t* __restrict__ amb,
+                                                         int64_t amb_words) {
   __shared__ float part[256];
   __shared__ float wmax[2];
   const int64_t a = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
@@ -395,7 +398,7 @@ __global__ __launch_bounds__(256) void score_block_norms(const void* __restrict_
     const int32_t t = static_cast<int32_t>(base) + lane;
     const int s = find_seq_near(cu, nseq, t);
     end = cu[s + 1];
-    starts = (t - cu[s]) % B == 0;
+    starts = end - cu[s] > shortest && (t - cu[s]) % B == 0;
   }
   for (uint64_t m = __ballot(starts); m; m &= m - 1) {
     const int l = __builtin_ctzll(m);
@@ -453,7 +456,7 @@ __global__ __launch_bounds__(256) void score_small_block_norms(const float* __re
 
 // Two workgroups per CU; one for the widest partial-width variant (index dim 72..120),
 // whose register staging of the next block does not fit beside two.
-template <int DT, int NK, bool FULLD>
+template <int DT, int NK, bool FULLD, int SHORTEST>
 __global__ __launch_bounds__(kThreads, NK == 4 && !FULLD ? 1 : 2) void score_fwd_mfma_kernel(const uint16_t* __restrict__ iq,
                                                                      const uint16_t* __restrict__ ik,
                                                                      const int32_t* __restrict__ cu, int nseq,
@@ -597,7 +600,7 @@ __global__ __launch_bounds__(kThreads, NK == 4 && !FULLD ? 1 : 2) void score_fwd
   };
 
   int todo;
-  BlockCursor cur = tile_share(cu, nseq, r0, nr, G, B, blockIdx.y, gridDim.y, todo);
+  BlockCursor cur = tile_share(cu, nseq, r0, nr, G, B, SHORTEST, blockIdx.y, gridDim.y, todo);
   const float cn = block_norm(cur);
   fetch(cur, ik, sm.k[0]);
   commit(0);
@@ -607,7 +610,7 @@ __global__ __launch_bounds__(kThreads, NK == 4 && !FULLD ? 1 : 2) void score_fwd
   bool bsafe = !__builtin_signbit(cn);  // -0 marks an unsafe block too
   int buf = 0;
   while (cur.s < nseq) {
-    BlockCursor nxt = next_block(cu, nseq, cur, r0, nr, G, B);
+    BlockCursor nxt = next_block(cu, nseq, cur, r0, nr, G, B, SHORTEST);
     if (--todo <= 0) nxt.s = nseq;
     const float nn = block_norm(nxt);
     // The next block's fetch and this block's LDS reads go through the restrict-qualified
@@ -749,7 +752,7 @@ struct KeyRowsF32 {
   }
 };
 
-template <int NK>
+template <int NK, int SHORTEST>
 __global__ __launch_bounds__(kThreads, 2) void score_fwd_f32_kernel(const float* __restrict__ iq,
                                                                     const float* __restrict__ ik,
                                                                     const int32_t* __restrict__ cu, int nseq,
@@ -819,7 +822,7 @@ __global__ __launch_bounds__(kThreads, 2) void score_fwd_f32_kernel(const float*
   }
 
   int todo;
-  BlockCursor cur = tile_share(cu, nseq, r0, nr, G, B, blockIdx.y, gridDim.y, todo);
+  BlockCursor cur = tile_share(cu, nseq, r0, nr, G, B, SHORTEST, blockIdx.y, gridDim.y, todo);
   float pinf = __builtin_inff();
   asm volatile("" : "+v"(pinf));
   while (cur.s < nseq) {
@@ -926,7 +929,7 @@ __global__ __launch_bounds__(kThreads, 2) void score_fwd_f32_kernel(const float*
         atomicOr(amb + (bit >> 5), 1u << (bit & 31));
       }
     }
-    cur = next_block(cu, nseq, cur, r0, nr, G, B);
+    cur = next_block(cu, nseq, cur, r0, nr, G, B, SHORTEST);
     if (--todo <= 0) cur.s = nseq;
   }
   fill_future(cu, nseq, r0 + wr0, nr - wr0, G, NB, B, scores, tie);
@@ -960,6 +963,45 @@ __device__ __forceinline__ double exact_dot_wide(const void* __restrict__ a, int
     }
   }
   return s0 + s1;
+}
+
+// Rows of sequences of up to kShortSeq tokens, 16 lanes each, one key per lane: every visible key's
+// exact dot, the maximum, its count and first key (a NaN dot is no candidate). A sequence is one
+// step of the MFMA kernels' tiles, of 128 keys and 64 or 128 rows, whatever its length: packs of
+// short ones took up to 64 such steps per tile, and the norms of 64 blocks one after the other.
+// Bound by the FP64 chains and their conversions (a wave's four rows take as long for one key
+// as for 16: 75 to 133 us for 131 072 rows). us, MFMA steps / here, 2 groups of 128 dims: fp16,
+// 8192 sequences of one token 356 / 43, 1024 of 8 69 / 31, 512 of 16 47 / 35, 65 536 of one 768 / 139,
+// 8192 of 8 154 / 134, 4096 of 16 103 / 175; fp32, 8192 of one 762 / 41, 682 of 12 124 / 32, 4096 of 16 255 /
+// 170. (For many fp16 or bf16 sequences of 9 to 16 the steps are the faster: not taken apart.)
+template <int DT>
+__global__ __launch_bounds__(256) void score_fwd_short(const void* __restrict__ iq, const void* __restrict__ ik,
+                                                       const int32_t* __restrict__ cu, int nseq, int64_t rows, int G,
+                                                       int Di, int NB, double scale, float* __restrict__ scores,
+                                                       int32_t* __restrict__ tie) {
+  const int64_t row = static_cast<int64_t>(blockIdx.x) * 16 + (threadIdx.x >> 4);
+  if (row >= rows) return;
+  const int sub = threadIdx.x & 15;
+  const int64_t t = row / G;
+  const int s = find_seq(cu, nseq, t);
+  const int64_t start = cu[s];
+  if (cu[s + 1] - start > kShortSeq) return;  // all 16 lanes
+  double best = -__builtin_inf();
+  bool seen = start + sub <= t;
+  if (seen) {
+    const double v = directed(exact_dot_wide<DT>(iq, row * Di, ik, (start + sub) * Di, Di), scale);
+    seen = v == v;
+    if (seen) best = v;
+  }
+  const double own = best;
+#pragma unroll
+  for (int o = 8; o > 0; o >>= 1) best = fmax(best, __shfl_xor(best, o, 16));
+  const uint32_t at = static_cast<uint32_t>(__ballot(seen && own == best) >> (threadIdx.x & 48)) & 0xffffu;
+  if (sub == 0) {
+    const int count = __popc(at);
+    scores[row * NB] = public_score(best, static_cast<float>(fabs(scale)));
+    if (tie) tie[row * NB] = count == 1 ? __builtin_ctz(at) + 1 : -count;
+  }
 }
 
 // Monotone map of a double that is not NaN onto uint64 (+0 and -0 collapse; never 0), and back.
@@ -1177,20 +1219,26 @@ static int launch(const void* iq, const void* ik, const int32_t* cu, int nseq, i
   auto* amb = reinterpret_cast<uint32_t*>(wsb + ws_bitmap_offset(T));
   const int64_t words = bitmap_words(rows, NB);
   const int64_t rows_pad = rows_padded(rows);
+  // Short sequences apart where they can be a large part of the pack (a mean length below 32; the
+  // kernel's pass over all rows takes 4 to 6 us where there are none). They are one block each: B >= 64.
+  const int shortest = B >= 64 && T < 32 * static_cast<int64_t>(nseq) && rows < (int64_t{1} << 28) ? kShortSeq : 0;
+  if (shortest)
+    hipLaunchKernelGGL(score_fwd_short<DT>, dim3(grid_1d(rows, 16)), dim3(256), 0, st, iq, ik, cu, nseq, rows, G, Di, NB,
+                       scale, scores, tie);
   if (B >= 64) {
     const unsigned ng = grid_1d(T, 64), wg = grid_1d(words, 256);
-    hipLaunchKernelGGL(score_block_norms<DT>, dim3(ng > wg ? ng : wg), dim3(256), 0, st, ik, cu, nseq, T, Di, B, bnorm, amb, words);
+    hipLaunchKernelGGL(score_block_norms<DT>, dim3(ng > wg ? ng : wg), dim3(256), 0, st, ik, cu, nseq, T, Di, B, shortest, bnorm, amb, words);
   } else {
     hipLaunchKernelGGL(score_key_norms<DT>, dim3(grid_1d(T > words ? T : words, 256)), dim3(256), 0, st, ik, T, Di, knorm2, amb, words);
     hipLaunchKernelGGL(score_small_block_norms, dim3(grid_1d(T, 256)), dim3(256), 0, st, knorm2, cu, nseq, T, B, bnorm);
   }
   const int nk = Di <= 32 ? 1 : (Di <= 64 ? 2 : 4);
   if constexpr (DT == kF32) {
-#define MSA_SCORE_F32(NKV) hipLaunchKernelGGL(score_fwd_f32_kernel<NKV>, grid, block, 0, st, static_cast<const float*>(iq), static_cast<const float*>(ik), cu, nseq, rows, G, Di, NB, B, scale, bnorm, amb, rows_pad, scores, tie)
+#define MSA_SCORE_F32(NKV) hipLaunchKernelGGL((shortest ? score_fwd_f32_kernel<NKV, kShortSeq> : score_fwd_f32_kernel<NKV, 0>), grid, block, 0, st, static_cast<const float*>(iq), static_cast<const float*>(ik), cu, nseq, rows, G, Di, NB, B, scale, bnorm, amb, rows_pad, scores, tie)
     if (nk == 1) MSA_SCORE_F32(1); else if (nk == 2) MSA_SCORE_F32(2); else MSA_SCORE_F32(4);
 #undef MSA_SCORE_F32
   } else {
-#define MSA_SCORE_MFMA(NKV, FD) hipLaunchKernelGGL((score_fwd_mfma_kernel<DT, NKV, FD>), grid, block, 0, st, static_cast<const uint16_t*>(iq), static_cast<const uint16_t*>(ik), cu, nseq, rows, G, Di, NB, B, scale, bnorm, amb, rows_pad, scores, tie)
+#define MSA_SCORE_MFMA(NKV, FD) hipLaunchKernelGGL((shortest ? score_fwd_mfma_kernel<DT, NKV, FD, kShortSeq> : score_fwd_mfma_kernel<DT, NKV, FD, 0>), grid, block, 0, st, static_cast<const uint16_t*>(iq), static_cast<const uint16_t*>(ik), cu, nseq, rows, G, Di, NB, B, scale, bnorm, amb, rows_pad, scores, tie)
     const bool fd = Di == 32 * nk;
     if (nk == 1) { if (fd) MSA_SCORE_MFMA(1, true); else MSA_SCORE_MFMA(1, false); }
     else if (nk == 2) { if (fd) MSA_SCORE_MFMA(2, true); else MSA_SCORE_MFMA(2, false); }

@@ -301,13 +301,14 @@ def test_score_index_dims_beyond_512(dim, dtype, device):
     _run(q_cpu, k_cpu, lengths, max(lengths), block, 1.0, upstream, device)
 
 
-def _forward_on_both_paths(q_cpu, k_cpu, lengths, block, scale, device):
+def _forward_on_both_paths(q_cpu, k_cpu, lengths, block, scale, device, exact_dtype=None):
     """(scores, tie codes) of the MFMA path and of the exact kernel, which takes the same
-    values when their rows do not start on 16-byte boundaries."""
+    values (or, for bf16, those values in fp32) when their rows do not start on 16-byte boundaries."""
     from msa_triton_amd.index_score import _score_forward
     from msa_triton_amd.layout import sequence_meta
 
     def shifted(x):  # the same values, one element past a 16-byte boundary
+        x = x if exact_dtype is None else x.to(exact_dtype)
         flat = torch.empty(x.numel() + 1, dtype=x.dtype, device=device)
         flat[1:] = x.to(device).flatten()
         y = flat[1:].view(x.shape)
@@ -359,6 +360,31 @@ def test_score_mfma_path_equals_the_exact_kernel(values, lengths, groups, dim, b
                                           max(lengths) + 3 * block, block_size=block, scale=scale)
         np.testing.assert_array_equal(mfma[0], exp32)
         np.testing.assert_array_equal(mfma[1], exp_tie)
+
+
+_SHORT = [1, 2, 0, 16, 17, 3, 15, 1, 1, 5, 8, 9, 12, 1, 4, 16, 200, 1, 1, 7, 2, 6]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("groups,dim,block,scale,lengths", [
+    (2, 128, 128, 1.0, _SHORT), (1, 40, 64, -0.75, _SHORT), (5, 32, 100, 0.5, _SHORT), (3, 64, 128, 1.0, [1] * 90),
+    (2, 128, 128, -1.0, [16] * 9), (2, 64, 63, 1.0, _SHORT),  # blocks below 64 keys: no path of its own
+])
+@pytest.mark.parametrize("values", ["normal", "integer", "nan"])
+def test_score_short_sequences_equal_the_exact_kernel(values, groups, dim, block, scale, lengths, dtype, device):
+    """Packs of mostly short sequences (up to 16 tokens: a kernel of their own) beside longer ones:
+    scores and winners bit for bit those of the exact kernel, for distinct values, exact ties,
+    and infinities and NaN in some keys."""
+    gen = torch.Generator().manual_seed(dim + block)
+    total = sum(lengths)
+    q, k = torch.randn(total, groups, dim, generator=gen), torch.randn(total, 1, dim, generator=gen)
+    if values == "integer":
+        q, k = q.round(), k.round()
+    if values == "nan":
+        k[::5, 0, 3], k[2::7, 0, 1], q[4::11, 0, 0] = float("nan"), float("inf"), float("nan")
+    mfma, exact = _forward_on_both_paths(q.to(dtype), k.to(dtype), lengths, block, scale, device, torch.float32)
+    np.testing.assert_array_equal(mfma[0], exact[0])
+    np.testing.assert_array_equal(mfma[1], exact[1])
 
 
 @pytest.mark.parametrize("dtype,dim", [(torch.bfloat16, 128), (torch.float32, 40)])
