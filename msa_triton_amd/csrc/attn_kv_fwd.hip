@@ -82,9 +82,9 @@ struct FwdSmem {
 //     (row tails) are the last to start, so the workgroups of a launch finish closer
 //     together. Items of equal size take their slots in no fixed order (integer atomics); no
 //     result depends on it, as each item writes only its own outputs, indexed by item.
-// Bound by launches and latency: as three kernels per plan (bounds, prefix, order), the plans
-// of a forward and backward took 8 launches (63 us at 32 768 tokens and 16 slots, 45 at 8192, 33 at 1280), as
-// one kernel each 2 (77, 26 and 14 us).
+// Bound by launches and latency: as three kernels per plan (bounds, prefix, order), the plans of a forward
+// and a backward took 8 launches (45 us at 8192 tokens, 33 at 1280), as one kernel each 2 (26 and 14 us); calls of
+// more than one chunk and kPlanSearchRows rows take a launch more per pass.
 constexpr int kOrderBuckets = 1024;
 constexpr int kMaxPlans = 2;
 struct PlanOut {
@@ -96,9 +96,32 @@ struct PlanOut {
 struct PlanOuts {
   PlanOut p[kMaxPlans];
 };
+
+// The bounds alone, one thread per (row, chunk boundary), for all plans: ahead of the plan kernel where
+// its one workgroup per chunk would search many rows, 1024 at a time and each twice above that.
+// Measured, us for the plans of a forward and a backward, three kernels per plan / one that searches / this
+// launch and one that reads: 1024 rows in 3 and 2 chunks 50 / 65 / 40, 4096 76 / 255 / 76, 16 384 134 / 744 / 125;
+// 512 rows 48 / 43 (one that searches). A single chunk has nothing to search (8192 rows: 81 / 65).
+constexpr int64_t kPlanSearchRows = 512;
+__global__ __launch_bounds__(256) void kv_plan_bounds(const int32_t* __restrict__ row_ptr,
+                                                      const int32_t* __restrict__ qidx, int64_t rows, int64_t tc,
+                                                      int nch, int plans, PlanOuts outs) {
+  const int64_t r = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (r >= rows) return;
+  const int c = blockIdx.y;
+  int32_t lo = row_ptr[c == nch ? r + 1 : r], hi = row_ptr[r + 1];
+  if (c > 0)
+    while (lo < hi) {
+      const int32_t m = lo + ((hi - lo) >> 1);  // (lo + hi may exceed INT32_MAX)
+      if (qidx[m] < c * tc) lo = m + 1; else hi = m;
+    }
+  for (int y = 0; y < plans; ++y) outs.p[y].bounds[c * rows + r] = lo;
+}
+
 __global__ __launch_bounds__(1024) void kv_plan_kernel(const int32_t* __restrict__ row_ptr,
                                                        const int32_t* __restrict__ qidx, int64_t rows, int64_t T,
-                                                       int64_t tc, int nch, PlanOuts outs, int row_order) {
+                                                       int64_t tc, int nch, PlanOuts outs, int searched,
+                                                       int row_order) {
   __shared__ int32_t wsum[16];
   __shared__ int32_t cnt[kOrderBuckets];
   const PlanOut po = outs.p[blockIdx.y];
@@ -130,6 +153,7 @@ __global__ __launch_bounds__(1024) void kv_plan_kernel(const int32_t* __restrict
   };
   // the row's edges of this chunk, [x, y): both ends searched side by side (their loads overlap)
   auto edges_of = [&](int64_t r) {
+    if (searched) return make_int2(po.bounds[c * rows + r], po.bounds[(c + 1) * rows + r]);  // kv_plan_bounds
     const int32_t a = row_ptr[r], b = row_ptr[r + 1];
     const int64_t t0 = c * tc, t1 = (c + 1) * tc;
     int32_t lo0 = a, hi0 = c == 0 ? a : b, lo1 = c == nch - 1 ? b : a, hi1 = b;
@@ -154,7 +178,7 @@ __global__ __launch_bounds__(1024) void kv_plan_kernel(const int32_t* __restrict
     const int64_t r = base + tid;
     mine = r < rows ? edges_of(r) : make_int2(0, 0);
     const int32_t lo = mine.x, hi = mine.y;
-    if (r < rows) {
+    if (r < rows && !searched) {
       po.bounds[c * rows + r] = lo;
       if (c == nch - 1) po.bounds[nch * rows + r] = hi;
     }
@@ -614,8 +638,13 @@ void kv_plan_launch(std::initializer_list<KvPlanAt> plans, const int32_t* row_pt
                           x.ordered ? reinterpret_cast<int32_t*>(b + x.plan.order) : nullptr,
                           reinterpret_cast<int2*>(b + x.plan.items)};
   }
+  // (one chunk: its bounds are the rows' ends, nothing to search)
+  const int searched = p0.nch > 1 && p0.rows > kPlanSearchRows;
+  if (searched)
+    hipLaunchKernelGGL(kv_plan_bounds, dim3(grid_1d(p0.rows, 256), static_cast<unsigned>(p0.nch + 1)), dim3(256), 0, st,
+                       row_ptr, qidx, p0.rows, p0.tc, static_cast<int>(p0.nch), static_cast<int>(n), outs);
   hipLaunchKernelGGL(kv_plan_kernel, dim3(static_cast<unsigned>(p0.nch), n), dim3(1024), 0, st, row_ptr, qidx, p0.rows, T,
-                     p0.tc, static_cast<int>(p0.nch), outs, g_item_order.load(std::memory_order_relaxed) ? 0 : 1);
+                     p0.tc, static_cast<int>(p0.nch), outs, searched, g_item_order.load(std::memory_order_relaxed) ? 0 : 1);
 }
 
 struct FwdLayout {

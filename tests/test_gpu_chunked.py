@@ -94,6 +94,28 @@ def test_attention_through_many_chunks(with_f32, device):
     _within_one_ulp(dv, dv1, "chunked vs single-chunk dv")
 
 
+@pytest.mark.parametrize("lengths,groups,block", [
+    ([512], 2, 2),          # 512 rows: the plan kernel searches the chunk bounds itself
+    ([500, 13], 1, 1),      # 513: they come from a launch of their own
+    ([1025], 1, 1),         # more rows than threads in the plan kernel
+    ([900, 130], 4, 2),     # 2060
+])
+def test_plans_of_many_rows_and_chunks(lengths, groups, block, device):
+    ratio, dim, topk = 4, 32, 6
+    q, k, v, grad, ids, cu = _attn_case(lengths, groups, ratio, dim, block, topk, 61)
+    out_r, _, dq_r, dk_r, dv_r = O.sparse_attention(np64(q), np64(k), np64(v), ids.numpy(), cu.numpy(),
+                                                    block_size=block, dout=np64(grad))
+    meta = sequence_meta(cu.tolist(), block)
+    qd, kd, vd, gd, idd, cud = (x.to(device) for x in (q, k, v, grad, ids, cu))
+    with _lib.chunk_budgets(fwd=1, bwd=1):  # 64-token chunks in both passes
+        out, _, rs, o32, csr = _attn_forward(qd, kd, vd, idd, cud, meta, block, dim ** -0.5, None, save_f32=True)
+        grads = _attn_backward(qd, kd, vd, idd, cud, out, rs, gd, meta, block, dim ** -0.5, None, True, True, True,
+                               csr, o32)
+    torch.cuda.synchronize()
+    for got, ref, what in zip((out, *grads), (out_r, dq_r, dk_r, dv_r), ("out", "dq", "dk", "dv")):
+        check_bf16_stated(got, ref, f"rows {meta.total_blocks * groups} {what}")
+
+
 @pytest.mark.parametrize("need", [(True, False, False), (False, True, False), (False, False, True)])
 def test_attention_gradient_subsets_through_many_chunks(need, device):
     lengths, groups, ratio, dim, block, topk = [450, 190], 1, 8, 128, 64, 4
