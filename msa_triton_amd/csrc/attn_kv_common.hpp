@@ -109,8 +109,11 @@ struct KvPlan {
 // pass 114 / 34 / 22 / 16 us, KL main pass 86 / 26 / 17 / 13, the sums over the items' dK, dV
 // and d_ik partials 6 / 16 / 24 / 39. Above that, smaller items cost more than they balance:
 // 8192 tokens, 2 groups, 16 heads of 256 dims, 512 / 256 / 128 edges: step 3610 / 3700 / 3736 us.
-inline int64_t kv_item_edges(int64_t tc, int64_t G, int64_t K, int64_t most, int64_t least) {
-  const int64_t e = tc * G * K / 512 / 16 * 16;
+// The KL's main pass runs one workgroup per CU and is given 256 items: with 512 the call of 4
+// sequences of 2048 tokens, 2 groups, 8 slots took 260 us for 247 with 512 edges (with 256 items:
+// 243), one of 4096 in 4 groups 275 for 262 (257), one of 2048 144 for 205 (116).
+inline int64_t kv_item_edges(int64_t tc, int64_t G, int64_t K, int64_t most, int64_t least, int64_t items = 512) {
+  const int64_t e = tc * G * K / items / 16 * 16;
   return e > most ? most : (e > least ? e : (least < most ? least : most));
 }
 

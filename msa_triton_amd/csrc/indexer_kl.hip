@@ -745,7 +745,7 @@ KlLayout kl_layout(int64_t T, int64_t Hq, int64_t G, int64_t Di, int64_t K, int6
   // per (token, slot): teacher (m, l) per head, student (m, l), KL and d_iq per group
   const int64_t rec = Hq * 8 + G * (8 + 4 + 4 * Di);
   const int64_t tc = kv_chunk_tokens(T, 1, K, rec, kv_chunk_budget(kPassKl, int64_t(1) << 30));
-  L.plan = kv_plan_layout(T, rows, G, K, tc, kv_item_edges(tc, G, K, kKlEdges, 64));
+  L.plan = kv_plan_layout(T, rows, G, K, tc, kv_item_edges(tc, G, K, kKlEdges, 64, 256));
   int64_t off = align256(L.plan.bytes);
   L.tpart = off;   off += align256(tc * Hq * K * 8);
   L.spart = off;   off += align256(tc * G * K * 8);
