@@ -85,7 +85,8 @@ int topk_launch(const float* scores, const int32_t* cu_seqlens, int nseq, int64_
   if (NB <= 16) MSA_TOPK_LAUNCH(1);
   else if (NB <= 32) MSA_TOPK_LAUNCH(2);
   else if (NB <= 64) MSA_TOPK_LAUNCH(4);
-  else if (K <= kSelectMostSlots && NB <= 1024 && K > (NB <= 128 ? kArgmaxSlots128 : NB <= 256 ? kArgmaxSlots256 : 0)) {
+  else if (K <= kSelectMostSlots && NB <= 1024 && K > (NB <= 128 ? kArgmaxSlots128 : NB <= 256 ? kArgmaxSlots256 : 0) &&
+           rows < (int64_t{1} << 32) / kWave) {  // (a launch holds fewer than 2^32 threads: up to a wave per row here)
     if (NB <= 128) { MSA_TOPK_SELECT(2); }
     else if (NB <= 256) { MSA_TOPK_SELECT(4); }
     else if (NB <= 512) { MSA_TOPK_SELECT(8); }

@@ -11,6 +11,9 @@ of those sequences alone (every token of a sequence sees only its own sequence).
 Selections (current block plus one random earlier block per token and group) are
 drawn on the device.
 
+Calls whose wide kernels would need 2^32 threads or more in one launch (the top-k by sort) take the
+forms that need fewer: the last test.
+
 The capacity limit of the KV-major kernels is the CSR's T * G * K < 2^31 edges
 (triton/k2q.py:65-69), so a pack may hold T * Hq * K >= 2^31 (token, head, slot)
 triples -- the index space of the per-slot partial records of the attention and of
@@ -150,3 +153,23 @@ def test_token_head_slot_triples_past_int32(device):
         bound = 2.0 ** -8 * np.abs(want) + 2.0 ** -10 * np.abs(want).max()
         print(f"seq 1 {what}: worst err/bound {float((err / bound).max()):.3f}", flush=True)
         assert np.all(err <= bound), f"seq 1 {what}: max err/bound {float((err / bound).max()):.3f}"
+
+
+def test_topk_rows_past_one_launch_of_the_sort(device):
+    """2^26 rows of 65 blocks: a wave per row would be 2^32 threads; the argmax form takes them."""
+    from msa_triton_amd import _lib
+
+    tail, block, nb, topk = 130, 2, 65, 25
+    total = (1 << 26) + tail
+    scores = torch.full((total, 1, nb), -1.0, device=device)
+    last = torch.randn(tail, 1, nb, generator=torch.Generator().manual_seed(1))
+    scores[-tail:] = last.to(device)
+    cu = torch.tensor([0, total - tail, total], dtype=torch.int32, device=device)
+    got = torch.full((total, 1, topk), -7, dtype=torch.int32, device=device)
+    status = _lib.lib().msa_topk(scores.data_ptr(), cu.data_ptr(), 2, total, 1, nb, block, topk, 1, got.data_ptr(),
+                                 _lib.stream_of(device))
+    assert status == 0
+    ref = O.topk(last.numpy(), [0, tail], block_size=block, topk_blocks=topk, local_blocks=1)
+    np.testing.assert_array_equal(got[-tail:].cpu().numpy(), ref)
+    # equal scores: ascending blocks, and past the first sequence's 65 blocks of 2 tokens all of them
+    assert bool((got[nb * block:-tail] == torch.arange(topk, dtype=torch.int32, device=device)).all())
