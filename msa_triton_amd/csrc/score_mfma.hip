@@ -1039,8 +1039,9 @@ __global__ __launch_bounds__(64) void score_fwd_resolve(const void* __restrict__
   __shared__ uint64_t best[kResolveGroup];
   __shared__ int count[kResolveGroup], first[kResolveGroup];
   const int lane = threadIdx.x, c = lane & 15, q4 = lane >> 4;
-  const int b = blockIdx.x;
-  const int64_t c0 = static_cast<int64_t>(blockIdx.y) * kResolveRows;
+  // blockIdx.x: chunk * NB + block; blockIdx.y: share
+  const int b = static_cast<int>(blockIdx.x % static_cast<uint32_t>(NB));
+  const int64_t c0 = static_cast<int64_t>(blockIdx.x / static_cast<uint32_t>(NB)) * kResolveRows;
   static_assert(kResolveRows == 64 * 64, "one 64-bit bitmap word per lane");
   const uint32_t* words = amb + (static_cast<int64_t>(b) * rows_pad + c0) / 32 + 2 * lane;
   uint64_t mine = (static_cast<uint64_t>(words[1]) << 32) | words[0];
@@ -1060,10 +1061,10 @@ __global__ __launch_bounds__(64) void score_fwd_resolve(const void* __restrict__
   }
   __syncthreads();
   // (the lists are in order, so a share's groups are those of its rows: each row once)
-  const int marked = __builtin_amdgcn_readfirstlane(count[0]), shares = gridDim.z;
-  const int n = marked * (static_cast<int>(blockIdx.z) + 1) / shares;
+  const int marked = __builtin_amdgcn_readfirstlane(count[0]), shares = gridDim.y;
+  const int n = marked * (static_cast<int>(blockIdx.y) + 1) / shares;
   const bool neg = scale < 0.0;
-  for (int i = marked * static_cast<int>(blockIdx.z) / shares; i < n;) {
+  for (int i = marked * static_cast<int>(blockIdx.y) / shares; i < n;) {
     const int64_t row0 = c0 + __builtin_amdgcn_readfirstlane(list[i]);
     const int s = find_seq(cu, nseq, row0 / G);
     const int64_t start = cu[s], end = cu[s + 1];
@@ -1225,7 +1226,7 @@ static int launch(const void* iq, const void* ik, const int32_t* cu, int nseq, i
   if (shortest)
     hipLaunchKernelGGL(score_fwd_short<DT>, dim3(grid_1d(rows, 16)), dim3(256), 0, st, iq, ik, cu, nseq, rows, G, Di, NB,
                        scale, scores, tie);
-  if (B >= 64) {
+  if (B >= 64 && T < (int64_t{1} << 30)) {  // (four threads per token: a launch holds fewer than 2^32)
     const unsigned ng = grid_1d(T, 64), wg = grid_1d(words, 256);
     hipLaunchKernelGGL(score_block_norms<DT>, dim3(ng > wg ? ng : wg), dim3(256), 0, st, ik, cu, nseq, T, Di, B, shortest, bnorm, amb, words);
   } else {
@@ -1247,7 +1248,7 @@ static int launch(const void* iq, const void* ik, const int32_t* cu, int nseq, i
   }
   const int64_t chunks = rows_pad / kResolveRows;
   const int64_t shares = std::max<int64_t>(1, std::min<int64_t>(kResolveShares, kResolveWaves / (NB * chunks)));
-  hipLaunchKernelGGL(score_fwd_resolve<DT>, dim3(NB, static_cast<unsigned>(chunks), static_cast<unsigned>(shares)), dim3(64), 0,
+  hipLaunchKernelGGL(score_fwd_resolve<DT>, dim3(static_cast<unsigned>(NB * chunks), static_cast<unsigned>(shares)), dim3(64), 0,
                      st, iq, ik, cu, nseq, rows_pad, G, Di, NB, B, scale, bnorm, amb, scores, tie);
   return status_from(hipGetLastError());
 }

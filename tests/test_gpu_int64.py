@@ -11,8 +11,9 @@ of those sequences alone (every token of a sequence sees only its own sequence).
 Selections (current block plus one random earlier block per token and group) are
 drawn on the device.
 
-Calls whose wide kernels would need 2^32 threads or more in one launch (the top-k by sort) take the
-forms that need fewer: the last test.
+Calls whose wide kernels would need 2^32 threads or more in one launch (the top-k by sort), or more
+workgroups than a dimension holds (the score's settling pass), take the forms that need fewer or number
+their workgroups in one dimension: the last two tests.
 
 The capacity limit of the KV-major kernels is the CSR's T * G * K < 2^31 edges
 (triton/k2q.py:65-69), so a pack may hold T * Hq * K >= 2^31 (token, head, slot)
@@ -173,3 +174,21 @@ def test_topk_rows_past_one_launch_of_the_sort(device):
     np.testing.assert_array_equal(got[-tail:].cpu().numpy(), ref)
     # equal scores: ascending blocks, and past the first sequence's 65 blocks of 2 tokens all of them
     assert bool((got[nb * block:-tail] == torch.arange(topk, dtype=torch.int32, device=device)).all())
+
+
+def test_score_rows_past_65535_settling_chunks(device):
+    """65 537 chunks of 4096 rows, sequences of one token: every score is the row's own dot."""
+    groups, dim = 2048, 8
+    total = (65536 * 4096 + 4096) // groups
+    gen = torch.Generator(device=device).manual_seed(2)
+    q = torch.randn(total, groups, dim, generator=gen, device=device).bfloat16()
+    k = torch.randn(total, 1, dim, generator=gen, device=device).bfloat16()
+    q[-1, -1, 0] = float("inf")  # settled by the last chunk (not certified by the matrix pass)
+    cu = torch.arange(total + 1, dtype=torch.int32, device=device)
+    with torch.no_grad():
+        scores = msa.m3_index_score(q, k, cu, 1, block_size=128)
+    assert bool(torch.isinf(scores[-1, -1, 0]))
+    for part in (slice(0, 64), slice(total - 64, total)):
+        dots = (q[part].double() * k[part].double()).sum(2).float()
+        keep = torch.isfinite(dots)
+        assert torch.equal(scores[part, :, 0][keep], dots[keep])
