@@ -541,6 +541,9 @@ static int dkdv_splits(int64_t T, int64_t G) {
   return static_cast<int>(s > 8 ? 8 : s);
 }
 
+// Threads of a launch: fewer than 2^32. (The vector kernels have fewer threads per head or key.)
+constexpr int64_t kMostThreads = int64_t{1} << 32;
+
 // Head dims of 32, 64, 96 or 128 with rows that start on 16-byte boundaries; the query passes
 // also need 3 to 8 heads per group (see above).
 bool attn_f64_dims_fit(int D, std::initializer_list<const void*> rows) {
@@ -548,7 +551,9 @@ bool attn_f64_dims_fit(int D, std::initializer_list<const void*> rows) {
   for (const void* p : rows) bits |= reinterpret_cast<uintptr_t>(p);
   return D % 32 == 0 && D <= 128 && (bits & 15) == 0;
 }
-bool attn_f64_heads_fit(int R) { return R >= 3 && R <= kMostHeads; }
+bool attn_f64_heads_fit(int64_t T, int64_t G, int R) {
+  return R >= 3 && R <= kMostHeads && T * G < kMostThreads / (64 * kQueryWaves);
+}
 
 #define MSA_F64_DIMS(LAUNCH)  \
   switch (D) {                \
@@ -581,6 +586,24 @@ int64_t attn_f64_dkdv_workspace_bytes(int64_t T, int64_t G, int64_t D) {
   return n > 1 ? int64_t{16} * n * T * G * D : 0;
 }
 
+// One workgroup per tile of every block, a block's tiles side by side (they gather the same rows; with
+// one block's tiles far apart 4 sequences of 2048 tokens took 8790 us for the backward, so 6257), or,
+// where whole blocks would give more than two numbers per tile (short sequences, blocks far longer
+// than they), numbered by tile: 8 sequences of 1024 tokens in blocks of 2^19 keys 8815 -> 5538 us.
+// blocks: at least as many as there are; numbers without a tile come last, as far as possible
+// (spread evenly between the others they leave shader engines idle: 8 x 1024, 8668 us).
+struct KeyGrid {
+  int64_t compact, numbers;  // numbers per group
+};
+static KeyGrid key_grid(int64_t T, int64_t nseq, int64_t B) {
+  const int64_t blocks = T / B + nseq < T ? T / B + nseq : T, tiles = T / 16 + blocks, per_block = (B + 15) / 16;
+  const int64_t compact = per_block * blocks > 2 * tiles ? (tiles + 1) / 2 : 0;
+  return KeyGrid{compact, compact ? 2 * compact : blocks * per_block};
+}
+bool attn_f64_dkdv_fits(int64_t T, int64_t nseq, int64_t G, int64_t B) {
+  return key_grid(T, nseq, B).numbers * G < kMostThreads / (64 * kKeyWaves);
+}
+
 F64Tile attn_f64_mean_tile(int64_t T, int nseq, int R, int K, int B) {
   const double blocks = static_cast<double>(T / B + nseq < T ? T / B + nseq : T), keys = T / blocks;
   const double slots = std::min<double>(K, (std::max(1.0, blocks / nseq) + 1) / 2);  // that exist
@@ -598,17 +621,9 @@ int attn_f64_dkdv_launch(const float* q, const float* k, const float* v, const f
   const double most = attn_f64_mean_tile(T, nseq, Hq / G, K, B).rows / 32;
   const int splits = split ? std::max(1, static_cast<int>(std::min<double>(dkdv_splits(T, G), most))) : 1;
   double* part = splits > 1 ? static_cast<double*>(ws) : nullptr;
-  // One workgroup per tile of every block, a block's tiles side by side (they gather the same rows; with
-  // one block's tiles far apart 4 sequences of 2048 tokens took 8790 us for the backward, so 6257), or,
-  // where whole blocks would give more than two numbers per tile (short sequences, blocks far longer
-  // than they), numbered by tile: 8 sequences of 1024 tokens in blocks of 2^19 keys 8815 -> 5538 us.
-  // blocks: at least as many as there are; numbers without a tile come last, as far as possible
-  // (spread evenly between the others they leave shader engines idle: 8 x 1024, 8668 us).
-  const int64_t blocks = T / B + nseq < T ? T / B + nseq : T, tiles = T / 16 + blocks;
-  const int64_t per_block = (static_cast<int64_t>(B) + 15) / 16;
-  const int64_t compact = per_block * blocks > 2 * tiles ? (tiles + 1) / 2 : 0;
-  const dim3 grid(static_cast<unsigned>((compact ? 2 * compact : blocks * per_block) * G), 1, splits);
-#define MSA_F64_DKDV(DV) hipLaunchKernelGGL(attn_f64_dkdv<DV>, grid, dim3(64 * kKeyWaves), 0, st, q, k, v, dout, rs, cu, cu_blocks, row_ptr, qidx, nseq, T, Hq, G, B, compact, fewest, scale, dk, dv, part)
+  const KeyGrid kg = key_grid(T, nseq, B);
+  const dim3 grid(static_cast<unsigned>(kg.numbers * G), 1, splits);
+#define MSA_F64_DKDV(DV) hipLaunchKernelGGL(attn_f64_dkdv<DV>, grid, dim3(64 * kKeyWaves), 0, st, q, k, v, dout, rs, cu, cu_blocks, row_ptr, qidx, nseq, T, Hq, G, B, kg.compact, fewest, scale, dk, dv, part)
   MSA_F64_DIMS(MSA_F64_DKDV)
 #undef MSA_F64_DKDV
   if (splits > 1)

@@ -7,9 +7,11 @@
 namespace msa {
 
 // What the kernels take: every pass needs fitting dims and 16-byte aligned rows, the query
-// passes (forward, dQ) also fitting heads per group.
+// passes (forward, dQ) also fitting heads per group, and each a number of workgroups that one
+// launch holds.
 bool attn_f64_dims_fit(int D, std::initializer_list<const void*> rows);
-bool attn_f64_heads_fit(int R);
+bool attn_f64_heads_fit(int64_t T, int64_t G, int R);
+bool attn_f64_dkdv_fits(int64_t T, int64_t nseq, int64_t G, int64_t B);
 
 int attn_f64_fwd_launch(const float* q, const float* k, const float* v, const int32_t* idx, const int32_t* cu, int nseq,
                         int64_t T, int Hq, int G, int D, int K, int B, double scale, float* out, float* lse, double* rs,

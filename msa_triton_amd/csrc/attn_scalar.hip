@@ -704,7 +704,7 @@ int attn_valu_launch_fwd(const void* q, const void* k, const void* v, const int3
                          int nseq, int64_t T, int Hq, int G, int D, int K, int B, double scale, void* out,
                          float* lse, double* rs, float* o32, hipStream_t st) {
   if constexpr (DT == kF32) {
-    if (attn_f64_dims_fit(D, {q, k, v}) && attn_f64_heads_fit(Hq / G))
+    if (attn_f64_dims_fit(D, {q, k, v}) && attn_f64_heads_fit(T, G, Hq / G))
       return attn_f64_fwd_launch(static_cast<const float*>(q), static_cast<const float*>(k), static_cast<const float*>(v),
                                  idx, cu, nseq, T, Hq, G, D, K, B, scale, static_cast<float*>(out), lse, rs, o32, st);
   }
@@ -725,7 +725,7 @@ int attn_valu_launch_dq(const void* q, const void* k, const void* v, const void*
                         const int32_t* idx, const int32_t* cu, int nseq, int64_t T, int Hq, int G, int D, int K,
                         int B, double scale, void* dq, hipStream_t st) {
   if constexpr (DT == kF32) {
-    if (attn_f64_dims_fit(D, {q, k, v, out, dout}) && attn_f64_heads_fit(Hq / G))
+    if (attn_f64_dims_fit(D, {q, k, v, out, dout}) && attn_f64_heads_fit(T, G, Hq / G))
       return attn_f64_dq_launch(static_cast<const float*>(q), static_cast<const float*>(k), static_cast<const float*>(v),
                                 static_cast<const float*>(out), static_cast<const float*>(dout), rs, idx, cu, nseq, T, Hq,
                                 G, D, K, B, scale, static_cast<float*>(dq), st);
@@ -749,7 +749,7 @@ int attn_valu_launch_dkdv(const void* q, const void* k, const void* v, const voi
                           void* dk, void* dv, void* ws, int64_t ws_bytes, hipStream_t st) {
   int few_only = 0;
   if constexpr (DT == kF32) {
-    if (attn_f64_dims_fit(D, {q, k, v, dout, rs})) {
+    if (attn_f64_dims_fit(D, {q, k, v, dout, rs}) && attn_f64_dkdv_fits(T, nseq, G, B)) {
       // The tiles with few pairs are looked for where the mean tile has at most four times as few:
       // elsewhere there can be some, but the launch costs more than they do.
       const F64Tile mean = attn_f64_mean_tile(T, nseq, Hq / G, K, B);

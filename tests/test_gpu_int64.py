@@ -11,9 +11,9 @@ of those sequences alone (every token of a sequence sees only its own sequence).
 Selections (current block plus one random earlier block per token and group) are
 drawn on the device.
 
-Calls whose wide kernels would need 2^32 threads or more in one launch (the top-k by sort), or more
-workgroups than a dimension holds (the score's settling pass), take the forms that need fewer or number
-their workgroups in one dimension: the last two tests.
+Calls whose wide kernels would need 2^32 threads or more in one launch (the top-k by sort, the
+score's settling pass, the fp32 attention on matrix products) take the forms that need fewer,
+or number their workgroups in one dimension: the last three tests.
 
 The capacity limit of the KV-major kernels is the CSR's T * G * K < 2^31 edges
 (triton/k2q.py:65-69), so a pack may hold T * Hq * K >= 2^31 (token, head, slot)
@@ -192,3 +192,23 @@ def test_score_rows_past_65535_settling_chunks(device):
         dots = (q[part].double() * k[part].double()).sum(2).float()
         keep = torch.isfinite(dots)
         assert torch.equal(scores[part, :, 0][keep], dots[keep])
+
+
+@pytest.mark.parametrize("groups,ratio", [(128, 3), (64, 1)])
+def test_f32_attention_past_one_launch_of_the_matrix_kernels(groups, ratio, device):
+    """131 072 sequences of one token in blocks of one key: 2^24 (token, group) pairs, or 2^23
+    (block, group) pairs, would be 2^32 threads. out = v, dv = the sum of dO over the heads, dq = dk = 0."""
+    total, dim = 131072, 32
+    gen = torch.Generator(device=device).manual_seed(3)
+    q = torch.randn(total, groups * ratio, dim, generator=gen, device=device).requires_grad_()
+    k, v = (torch.randn(total, groups, dim, generator=gen, device=device).requires_grad_() for _ in range(2))
+    ids = torch.zeros(total, groups, 1, dtype=torch.int32, device=device)
+    cu = torch.arange(total + 1, dtype=torch.int32, device=device)
+    out = msa.m3_sparse_attention(q, k, v, ids, cu, 1, block_size=1)
+    assert torch.equal(out.view(total, groups, ratio, dim), v[:, :, None].expand(-1, -1, ratio, -1))
+    dout = torch.randn(out.shape, generator=gen, device=device)
+    dq, dk, dv = torch.autograd.grad(out, (q, k, v), dout)
+    # FP64 sums: dP - dO . O is below 2^-53 times their 32 terms, |terms| < 50
+    assert float(dq.abs().max()) < 1e-11 and float(dk.abs().max()) < 1e-11
+    want = dout.view(total, groups, ratio, dim).double().sum(2)
+    assert bool(((dv.double() - want).abs() <= 2.0 ** -23 * want.abs() + 1e-12).all())
