@@ -1222,7 +1222,8 @@ static int launch(const void* iq, const void* ik, const int32_t* cu, int nseq, i
   const int64_t rows_pad = rows_padded(rows);
   // Short sequences apart where they can be a large part of the pack (a mean length below 32; the
   // kernel's pass over all rows takes 4 to 6 us where there are none). They are one block each: B >= 64.
-  const int shortest = B >= 64 && T < 32 * static_cast<int64_t>(nseq) && rows < (int64_t{1} << 28) ? kShortSeq : 0;
+  const bool may_be_short = T < 32 * static_cast<int64_t>(nseq) && (nseq > 1 || T <= kShortSeq);
+  const int shortest = B >= 64 && may_be_short && rows < (int64_t{1} << 28) ? kShortSeq : 0;
   if (shortest)
     hipLaunchKernelGGL(score_fwd_short<DT>, dim3(grid_1d(rows, 16)), dim3(256), 0, st, iq, ik, cu, nseq, rows, G, Di, NB,
                        scale, scores, tie);
@@ -1247,7 +1248,8 @@ static int launch(const void* iq, const void* ik, const int32_t* cu, int nseq, i
 #undef MSA_SCORE_MFMA
   }
   const int64_t chunks = rows_pad / kResolveRows;
-  const int64_t shares = std::max<int64_t>(1, std::min<int64_t>(kResolveShares, kResolveWaves / (NB * chunks)));
+  const int64_t most = std::min<int64_t>(kResolveShares, std::min<int64_t>(rows, kResolveRows) / 64);  // (of 64 rows)
+  const int64_t shares = std::max<int64_t>(1, std::min(most, kResolveWaves / (NB * chunks)));
   hipLaunchKernelGGL(score_fwd_resolve<DT>, dim3(static_cast<unsigned>(NB * chunks), static_cast<unsigned>(shares)), dim3(64), 0,
                      st, iq, ik, cu, nseq, rows_pad, G, Di, NB, B, scale, bnorm, amb, scores, tie);
   return status_from(hipGetLastError());

@@ -25,6 +25,31 @@ from . import _lib
 from .layout import PackedSequences, prepared_for, sequence_meta
 
 
+def _exact_is_faster(q, meta):
+    """fp16 and fp32 calls of so few causal (row, key) pairs that the exact kernel's one launch takes less
+    than the matrix pass's three (bf16 has only that pass): about 16 us (32 where blocks have more than 64
+    keys of 128 dims, two per lane) and 0.24 us per 1000 pairs of 128 dims, against 17 to 31 us in fp16 and 25
+    to 59 in fp32. Measured, exact / matrix pass, us, one sequence in blocks of 128 keys, 128 dims: fp16
+    32 tokens x 8 groups 14 / 26, 64 x 8 18 / 26, 128 x 4 32 / 27; fp32 64 x 4 18 / 38, 128 x 1 32 / 29, 128 x 4
+    32 / 38, 256 x 2 33 / 48, 384 x 1 38 / 58, 384 x 2 56 / 59."""
+    total, groups, dim = q.shape
+    if q.dtype == torch.bfloat16 or total > 2048 or meta.num_seqs > 32:
+        return False
+    work = groups * dim * sum(n * (n + 1) // 2 for n in meta.lengths)
+    short_chain = -(-min(meta.block_size, max(meta.lengths)) // 64) * dim <= 128  # a lane's products
+    if q.dtype == torch.float16:
+        return short_chain and work <= 4.3e6
+    return (short_chain or total * groups > 128) and work <= 12.6e6
+
+
+def _score_workspace(q, blocks, meta):
+    """The matrix pass's workspace, or None for the exact kernel."""
+    if _exact_is_faster(q, meta):
+        return None
+    return torch.empty(_lib.lib().msa_score_fwd_workspace_bytes(q.shape[0], q.shape[1], blocks), dtype=torch.uint8,
+                       device=q.device)
+
+
 def _score_forward(q, k, cu, meta, max_seqlen, block_size, scale, save_state):
     """Forward launch on contiguous inputs: (scores, tie codes or None)."""
     total, groups, dim = q.shape
@@ -33,12 +58,12 @@ def _score_forward(q, k, cu, meta, max_seqlen, block_size, scale, save_state):
     tie = torch.empty((total, groups, blocks), dtype=torch.int32, device=q.device) if save_state else None
     if total:
         lib = _lib.lib()
-        workspace = torch.empty(lib.msa_score_fwd_workspace_bytes(total, groups, blocks), dtype=torch.uint8, device=q.device)
+        workspace = _score_workspace(q, blocks, meta)
         with _lib.on_device(q.device):
             status = lib.msa_score_fwd(
                 q.data_ptr(), k.data_ptr(), _lib.DTYPE_CODE[q.dtype], cu.data_ptr(), meta.num_seqs,
                 total, groups, dim, blocks, block_size, scale, scores.data_ptr(),
-                None if tie is None else tie.data_ptr(), workspace.data_ptr(), _lib.stream_of(q.device),
+                _lib.ptr(tie), _lib.ptr(workspace), _lib.stream_of(q.device),
             )
         _lib.check(status, "msa_score_fwd")
     return scores, tie
@@ -173,12 +198,12 @@ class _IndexScoreTopk(torch.autograd.Function):
         indices = torch.empty((total, groups, topk_blocks), dtype=torch.int32, device=q.device)
         if total:
             lib = _lib.lib()
-            workspace = torch.empty(lib.msa_score_fwd_workspace_bytes(total, groups, blocks), dtype=torch.uint8, device=q.device)
+            workspace = _score_workspace(q, blocks, meta)
             with _lib.on_device(q.device):
                 status = lib.msa_index_score_topk(
                     q.data_ptr(), k.data_ptr(), _lib.DTYPE_CODE[q.dtype], cu.data_ptr(), meta.num_seqs,
                     total, groups, dim, blocks, block_size, scale, topk_blocks, local_blocks, scores.data_ptr(),
-                    None if tie is None else tie.data_ptr(), indices.data_ptr(), workspace.data_ptr(),
+                    _lib.ptr(tie), indices.data_ptr(), _lib.ptr(workspace),
                     _lib.stream_of(q.device),
                 )
             _lib.check(status, "msa_index_score_topk")

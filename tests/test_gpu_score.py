@@ -301,6 +301,32 @@ def test_score_index_dims_beyond_512(dim, dtype, device):
     _run(q_cpu, k_cpu, lengths, max(lengths), block, 1.0, upstream, device)
 
 
+@pytest.fixture
+def matrix_pass(monkeypatch):
+    """Calls of any size take the matrix pass (small ones in fp16 and fp32 take the exact kernel)."""
+    from msa_triton_amd import index_score
+
+    monkeypatch.setattr(index_score, "_exact_is_faster", lambda q, meta: False)
+
+
+@pytest.mark.parametrize("dtype,lengths,groups,exact", [
+    (torch.float32, [64], 4, True), (torch.float32, [384], 1, True), (torch.float32, [500], 2, False),
+    (torch.float32, [1] * 40, 2, False), (torch.float16, [64, 0, 30], 8, True), (torch.float16, [65], 1, False),
+])
+def test_score_of_small_calls_is_the_matrix_pass_of_them(dtype, lengths, groups, exact, device, monkeypatch):
+    from msa_triton_amd import index_score
+    from msa_triton_amd.layout import sequence_meta
+
+    gen = torch.Generator().manual_seed(5)
+    q, k = (torch.randn(sum(lengths), n, 128, generator=gen).to(dtype).to(device) for n in (groups, 1))
+    assert index_score._exact_is_faster(q, sequence_meta(cu_list(lengths), 128)) == exact
+    cu, longest = cu_tensor(lengths, device), max(lengths)
+    got = msa.m3_index_score_topk(q, k, cu, longest, topk_blocks=2)
+    monkeypatch.setattr(index_score, "_exact_is_faster", lambda q, meta: not exact)
+    for a, b in zip(got, msa.m3_index_score_topk(q, k, cu, longest, topk_blocks=2)):
+        assert torch.equal(a, b)
+
+
 def _forward_on_both_paths(q_cpu, k_cpu, lengths, block, scale, device, exact_dtype=None):
     """(scores, tie codes) of the MFMA path and of the exact kernel, which takes the same
     values (or, for bf16, those values in fp32) when their rows do not start on 16-byte boundaries."""
@@ -331,7 +357,7 @@ def _forward_on_both_paths(q_cpu, k_cpu, lengths, block, scale, device, exact_dt
     ([513, 90], 4, 32, 33, 2.0),
 ])
 @pytest.mark.parametrize("values", ["normal", "integer", "range"])
-def test_score_mfma_path_equals_the_exact_kernel(values, lengths, groups, dim, block, scale, dtype, device):
+def test_score_mfma_path_equals_the_exact_kernel(values, lengths, groups, dim, block, scale, dtype, device, matrix_pass):
     """fp16 and fp32 on the MFMA path against the exact kernel, bit for bit (scores and tie
     codes): random values, small integers (exact ties) and magnitudes over the whole range of
     the type (fp16 subnormals; fp32 elements beyond the range whose products the bf16 terms
@@ -371,7 +397,8 @@ _SHORT = [1, 2, 0, 16, 17, 3, 15, 1, 1, 5, 8, 9, 12, 1, 4, 16, 200, 1, 1, 7, 2, 
     (2, 128, 128, -1.0, [16] * 9), (2, 64, 63, 1.0, _SHORT),  # blocks below 64 keys: no path of its own
 ])
 @pytest.mark.parametrize("values", ["normal", "integer", "nan"])
-def test_score_short_sequences_equal_the_exact_kernel(values, groups, dim, block, scale, lengths, dtype, device):
+def test_score_short_sequences_equal_the_exact_kernel(values, groups, dim, block, scale, lengths, dtype, device,
+                                                      matrix_pass):
     """Packs of mostly short sequences (up to 16 tokens: a kernel of their own) beside longer ones:
     scores and winners bit for bit those of the exact kernel, for distinct values, exact ties,
     and infinities and NaN in some keys."""
