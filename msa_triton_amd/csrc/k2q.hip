@@ -19,7 +19,8 @@
 //   4. k2q_scatter_par : per (tile, group), a stable counting sort of the tile's
 //                    edges on their block id places each edge at row_ptr[row] +
 //                    tile offset + its rank among the tile's edges of that row.
-//                    Entries at or beyond row_ptr[rows] become -1.
+//                    Entries at or beyond row_ptr[rows] become -1 (k2q_tail where the
+//                    blocks are few).
 #include <algorithm>
 #include <mutex>
 
@@ -188,8 +189,8 @@ __global__ __launch_bounds__(256) void k2q_scatter_par(const int32_t* __restrict
                                                        int32_t* __restrict__ counters,
                                                        int32_t* __restrict__ query_idx,
                                                        int32_t* __restrict__ slot_idx) {
-  // entries at or beyond row_ptr[rows] become -1: the grid's workgroups share them (a launch
-  // of its own took 3 to 5 us)
+  // entries at or beyond row_ptr[rows] become -1: the grid's workgroups share them (a launch of its own
+  // takes 3 to 5 us), unless that would be many each (then the host passes a capacity of 0)
   for (int64_t i = row_ptr[rows] + (static_cast<int64_t>(blockIdx.y) * gridDim.x + blockIdx.x) * 256 + threadIdx.x;
        i < capacity; i += static_cast<int64_t>(gridDim.x) * gridDim.y * 256) {
     query_idx[i] = -1;
@@ -273,6 +274,17 @@ __global__ __launch_bounds__(256) void k2q_scatter_par(const int32_t* __restrict
   }
 }
 
+// The same in a launch of its own.
+constexpr int64_t kTailPerWorkgroup = 16384;
+__global__ __launch_bounds__(256) void k2q_tail(const int32_t* __restrict__ row_ptr, int64_t rows, int64_t capacity,
+                                                int32_t* __restrict__ query_idx, int32_t* __restrict__ slot_idx) {
+  for (int64_t i = row_ptr[rows] + static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < capacity;
+       i += static_cast<int64_t>(gridDim.x) * 256) {
+    query_idx[i] = -1;
+    slot_idx[i] = -1;
+  }
+}
+
 __global__ __launch_bounds__(256) void fill_i32(int32_t* __restrict__ dst, int64_t n, int32_t value) {
   for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
        i += static_cast<int64_t>(gridDim.x) * blockDim.x)
@@ -303,7 +315,7 @@ namespace msa {
 
 namespace {
 
-// The four launches of the build over a caller-provided int32 workspace of
+// The four (or five) launches of the build over a caller-provided int32 workspace of
 // counter_elems + total_blocks * groups entries (the tile histograms are cleared by
 // k2q_count itself and the row totals are written before they are read, so the
 // workspace may hold anything on entry).
@@ -327,9 +339,15 @@ int k2q_build_launch(const int32_t* indices, const int32_t* cu_seqlens, const in
   hipLaunchKernelGGL(k2q_rowscan, dim3(grid_1d(rows, 4)), dim3(256), 0, st, cu_block_lens, tri_prefix,
                      nseq, G, rows, counters, totals);
   hipLaunchKernelGGL(k2q_ptrscan, dim3(1), dim3(1024), 0, st, totals, rows, row_ptr);
+  // Few blocks and much capacity: the tail apart (65 536 tokens, 16 slots, one group, in one block: 5226 us with
+  // the tail apart, 5523 with it in the one workgroup; 8 blocks 602 / 624).
+  const bool tail_apart = capacity > rows * kTailPerWorkgroup;
   hipLaunchKernelGGL(k2q_scatter_par, dim3(static_cast<unsigned>(total_blocks), static_cast<unsigned>(G)),
                      dim3(256), 0, st, indices, cu_seqlens, cu_block_lens, tri_prefix, nseq, G, K, B, row_ptr, rows,
-                     capacity, counters, query_indices, slot_indices);
+                     tail_apart ? 0 : capacity, counters, query_indices, slot_indices);
+  if (tail_apart)
+    hipLaunchKernelGGL(k2q_tail, dim3(capped_grid(capacity)), dim3(256), 0, st, row_ptr, rows, capacity, query_indices,
+                       slot_indices);
   return status_from(hipGetLastError());
 }
 

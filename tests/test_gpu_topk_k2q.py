@@ -127,6 +127,15 @@ def test_k2q_matches_oracle(lengths, groups, slots, block_size, device):
     _check_csr(ids, lengths, block_size, device)
 
 
+@pytest.mark.parametrize("tokens,slots,block", [(2048, 8, 2048), (2049, 8, 4096), (3000, 16, 1500)])
+def test_k2q_unused_tail_of_few_blocks(tokens, slots, block, device):
+    """Exactly 16 384 entries per (block, group) row (filled with -1 by the scatter), one token more
+    and several times as many (by a launch of their own)."""
+    ids = torch.full((tokens, 1, slots), -1, dtype=torch.int32)
+    ids[::3, 0, 2] = 0
+    _check_csr(ids, [tokens], block, device)
+
+
 def test_k2q_duplicates_and_block_reset(device):
     ids = torch.tensor(
         [[[0, 0, 1], [1, 0, -1]], [[0, -1, 8], [0, 0, 1]], [[1, 0, 1], [0, 1, -2]], [[0, 0, 1], [0, -1, 9]],
