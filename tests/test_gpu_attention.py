@@ -58,7 +58,10 @@ REFERENCE_SHAPES = [
 ]
 
 
-@pytest.mark.parametrize("lengths,groups,ratio,dimension,block_size,topk,scale", REFERENCE_SHAPES)
+@pytest.mark.parametrize("lengths,groups,ratio,dimension,block_size,topk,scale", [
+    *REFERENCE_SHAPES,
+    ([40] + [0] * 30 + [1] * 20 + [50], 1, 2, 32, 16, 2, None),  # lanes of a wave whose sequences are far apart
+])
 def test_forward_backward_against_fp64(lengths, groups, ratio, dimension, block_size, topk, scale, device):
     cpu, indices, cu = attention_inputs(lengths, groups, ratio, dimension, block_size, topk)
     tensors, indices_d, cu_d = _to(device, cpu, indices, cu)

@@ -40,6 +40,7 @@ def _run(q_cpu, k_cpu, lengths, max_seqlen, block_size, scale, upstream, device)
 
 
 @pytest.mark.parametrize("lengths,groups,dim,block_size,scale", [
+    ([40] + [0] * 30 + [1] * 20 + [50], 2, 64, 64, 1.0),  # lanes of a wave whose sequences are far apart
     ([1], 1, 1, 4, 1.0), ([0, 0], 2, 7, 4, 1.0), ([0, 3, 0, 2, 0], 2, 7, 4, 1.0), ([3, 7], 2, 7, 4, 1.0),
     ([7, 11], 4, 16, 8, 0.5), ([9], 2, 64, 4, 1.0), ([5], 4, 128, 128, 1.0),
     # scales that are not powers of two: exact path (Di 16) and MFMA path (Di 64, 128)
