@@ -7,8 +7,8 @@
   same way. Here the budgets are shrunk with the ``msa_set_chunk_budgets`` testing
   hook so that small packs, checked against the dense FP64 oracle, run through 4 to
   20 chunks: every early key then receives its gradient from several chunks.
-* The score backward forms dk per (key block, 8192-row segment) and adds the
-  segments in order; a pack with T * G > 3 * 8192 rows runs through 4 segments.
+* The score backward forms dk per (key block, segment of 2048 or 8192 rows) and adds the
+  segments in order; a pack with T * G = 26800 rows runs through 14 segments of 2048.
 
 Tolerance: the stated bf16 tolerance of the large-output tests
 (tests.helpers.check_bf16_stated); the KL uses its own stated bounds
@@ -162,7 +162,7 @@ def test_indexer_kl_through_many_chunks(device):
 
 
 def test_score_backward_through_several_row_segments(device):
-    """T * G = 26800 rows: the dk pass works on 4 segments of 8192 rows per key block."""
+    """T * G = 26800 rows: the dk pass works on up to 6 segments of 2048 rows per key block, 14 in all."""
     lengths, groups, dim, block = [3000, 2500, 1200], 4, 64, 128
     gen = torch.Generator().manual_seed(53)
     total = sum(lengths)
@@ -183,7 +183,7 @@ def test_score_backward_through_several_row_segments(device):
 
 @pytest.mark.parametrize("chunked", [False, True])
 def test_dispatch_order_leaves_results_bitwise_equal(chunked, device):
-    """The KV-major passes launch their work items largest first (``kv_item_order``);
+    """The KV-major passes launch their work items largest first (``kv_plan_kernel``'s order);
     every item writes only its own records and partial slot, so row-order dispatch (the
     ``msa_set_item_order`` testing hook) must give the same bits in every output."""
     lengths, groups, ratio, dim, block, topk = [2100, 1500, 37], 2, 8, 128, 64, 8

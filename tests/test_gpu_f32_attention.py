@@ -56,8 +56,8 @@ def test_f32_forward_backward_against_fp64(lengths, groups, ratio, block, topk, 
 
 
 def test_f32_rows_off_16_byte_boundaries_equal_aligned_ones(device):
-    """The same values one element past a 16-byte boundary take the vector kernels: both within
-    one fp32 rounding of the same FP64 result."""
+    """The same values one element past a 16-byte boundary take the vector kernels, forward and
+    backward: both within one fp32 rounding of the same FP64 result."""
     gen = torch.Generator().manual_seed(3)
     lengths, groups, ratio, dimension, block, topk = [150, 37], 2, 4, 64, 32, 3
     total = sum(lengths)
@@ -70,9 +70,14 @@ def test_f32_rows_off_16_byte_boundaries_equal_aligned_ones(device):
         flat[1:] = x.to(device).flatten()
         return flat[1:].view(x.shape)
 
-    a = msa.m3_sparse_attention(*(x.to(device) for x in values), ids, cu, max(lengths), block_size=block)
-    b = msa.m3_sparse_attention(*(shifted(x) for x in values), ids, cu, max(lengths), block_size=block)
-    assert bool(((a - b).abs() <= 2.0 ** -22 * b.abs()).all())
+    dout = torch.randn(values[0].shape, generator=gen)
+    results = []
+    for place in (lambda x: x.to(device), shifted):
+        leaves = [place(x).requires_grad_() for x in values]
+        out = msa.m3_sparse_attention(*leaves, ids, cu, max(lengths), block_size=block)
+        results.append([out.detach(), *torch.autograd.grad(out, leaves, place(dout))])
+    for a, b in zip(*results):  # (1e-11: the FP64 sums' own rounding, as above)
+        assert bool(((a - b).abs() <= 2.0 ** -22 * b.abs() + 1e-11).all())
 
 
 @pytest.mark.parametrize("dimension", [32, 64, 96, 128])

@@ -2,11 +2,15 @@
 attn_bwd_dkdv_rows: head dims 8, 16, 32, 64, 128 with 16-byte aligned rows) on fp16 and
 fp32 inputs, forward and backward against the FP64 oracle: fp32 within the reference's
 gate, fp16 within its stated analogue (every element within one fp16 ulp of the FP64
-value, at most 0.1 % outside the gate). Head ratio 3 makes a KV-pass step span edges
-(3 heads per edge against 4 to 16 rows per step); ragged lengths and blocks of 16 leave
-partly visible blocks, and the blocks of 128 keys fill the forward's 64-key steps.
+value, at most 0.1 % outside the gate). Ragged lengths and blocks of 16 leave partly
+visible blocks, and the blocks of 128 keys fill the forward's 64-key steps.
 fp16 takes these kernels only for shapes outside the MFMA kernels: its cases use blocks
-of 131 and 257 keys (primes above 128, so no sub-block split applies)."""
+of 131 and 257 keys (primes above 128, so no sub-block split applies) and 3 heads per
+group, which makes a KV-pass step span edges (3 heads per edge against 4 to 16 rows per
+step). fp32 with 3 to 8 heads takes the matrix products in the query passes, so its cases
+use 12 heads as well; its KV pass is the row-parallel one at dims 8 and 16 (12 heads
+against 32 and 64 rows per step) and, at 32, 64 and 128, only for tiles of few pairs, which
+are tested with the matrix kernel that leaves them (test_gpu_f32_attention.py)."""
 
 from __future__ import annotations
 
@@ -24,12 +28,13 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("block_index", [0, 1], ids=["short", "long"])
 @pytest.mark.parametrize("dim", [8, 16, 32, 64, 128])
-@pytest.mark.parametrize("dtype", [torch.float16, torch.float32], ids=["fp16", "fp32"])
-def test_row_parallel_fp64_kernels_against_oracle(dtype, dim, block_index, device):
+@pytest.mark.parametrize("dtype,ratio", [(torch.float16, 3), (torch.float32, 3), (torch.float32, 12)],
+                         ids=["fp16", "fp32", "fp32-12-heads"])
+def test_row_parallel_fp64_kernels_against_oracle(dtype, ratio, dim, block_index, device):
     from msa_triton_amd import _lib
 
     block = ([131, 257] if dtype == torch.float16 else [16, 128])[block_index]
-    lengths, groups, ratio, topk = [150, 61], 2, 3, 4
+    lengths, groups, topk = [150, 61], 2, 4
     total = sum(lengths)
     nblocks = sum((n + block - 1) // block for n in lengths)
     assert _lib.lib().msa_attn_fwd_workspace_bytes(_lib.DTYPE_CODE[dtype], total, groups * ratio, groups, dim, topk,
