@@ -182,10 +182,12 @@ int64_t msa_attn_bwd_split_bytes(int32_t dtype, int64_t total_tokens, int64_t kv
  * dS, one extra pass over every (row, slot). With out_f32 (the forward's, for the
  * same row_state) the bf16 path takes delta = out_f32 . dO in fp64 and the
  * forward's exact mass instead, and skips that pass; other paths ignore it.
- * The bf16 path is KV-major and needs the k2q CSR (cu_block_lens, row_ptr,
- * query_indices, slot_indices) and msa_attn_bwd_workspace_bytes(...) bytes of
- * workspace for every gradient set; the VALU path needs the CSR only when
- * grad_k or grad_v is requested. row_state slots 1..3 are (re)written.
+ * The bf16 and fp16 path is KV-major and needs the k2q CSR (cu_block_lens, row_ptr,
+ * query_indices, slot_indices, with total_blocks = cu_block_lens[num_seqs]) and
+ * msa_attn_bwd_workspace_bytes(...) bytes of workspace for every gradient set; the FP64
+ * path needs the CSR only when grad_k or grad_v is requested, does not read total_blocks
+ * or slot_indices, and can use msa_attn_bwd_split_bytes(...) bytes of workspace.
+ * row_state slots 1..3 are (re)written.
  * Deterministic: no floating-point atomics. */
 int msa_attn_bwd(const void* q, const void* k, const void* v, int32_t dtype, const void* out,
                  const void* grad_out, double* row_state, const float* out_f32, const int32_t* indices,
@@ -249,7 +251,7 @@ int msa_set_item_order(int enabled);
  * call's stream (at most 16384 launches). msa_profile_end waits for those events and
  * writes, for each kernel kind k < kinds, the summed duration in ms (ms[k]) and the
  * number of launches (launches[k]); either array may be NULL. Kinds, in order:
- * 0 forward work plan (kv_chunk_bounds + kv_item_scan), 1 attn_fwd_partial_kernel,
+ * 0 forward work plan (kv_plan_kernel, with kv_plan_bounds for many rows), 1 attn_fwd_partial_kernel,
  * 2 attn_fwd_combine, 3 backward work plans, 4 kv_bwd_center, 5 kv_bwd_stats_kernel,
  * 6 kv_bwd_stats_combine, 7 kv_bwd_main_kernel, 8 kv_bwd_accumulate,
  * 9 kv_bwd_dq_combine. Returns the number of kinds the library defines (10), or -1

@@ -19,11 +19,14 @@
 //    the last 32 dims.
 //
 // Query passes: one workgroup per (token, group), its R heads (3 to 8) the columns of the
-// logits (16: the rest is idle; below 3 the VALU kernels waste less), its key tiles of 16
+// logits (16: the rest is idle; below 3 the VALU kernels waste less; above 8 the dQ pass's two key
+// sums no longer fit the 16 rows of one product, nor the waves' sums the 64 KiB of LDS that two
+// workgroups per CU leave: 9 to 16 heads stay on the VALU kernels, untried here), its key tiles of 16
 // dealt to 4 waves; their sums are added in wave order. The query pass forms its two key sums
 // (of u = p (dp - c) and of p) in one product: rows 0-7 of the A operand are u, 8-15 p.
 // KV pass: one workgroup per 16 keys and group, the rows (edge, head) of the block's CSR row
-// 16 at a time, dealt to 8 waves; the waves' sums are added in wave order.
+// 16 at a time, dealt to 8 waves; the waves' sums are added in wave order. Tiles of few rows and keys
+// are the VALU kernel's (kF64FewestPairs).
 #include <algorithm>
 
 #include "attn_f64_mfma.hpp"

@@ -6,7 +6,8 @@
 // with head dims up to 256 and up to 512 heads per group take the KV-major MFMA kernels
 // (attn_kv_fwd.hip, attn_kv_bwd.hip; blocks above 128 keys as sub-blocks), fp32 inputs with
 // head dims 32, 64, 96 and 128 those on FP64 matrix products (attn_f64_mfma.hip; the query
-// passes with 3 to 8 heads per group); this file serves the other shapes. Measured at 2048
+// passes with 3 to 8 heads per group, the KV pass for tiles of enough rows and keys); this file
+// serves the rest. Measured at 2048
 // tokens, 2 groups, 128 dims, forward here and there: 520 us with 2 heads per group (here),
 // 694 -> 552 with 3, 888 -> 562 with 4.
 //

@@ -9,10 +9,12 @@
 // ascending block order; this is the canonical order documented for the
 // drop-in (torch.topk leaves it unspecified).
 //
-// Sixteen lanes own one (token, group) row and hold the row's causal prefix in
-// registers (VPL values per lane). Selection is an iterated argmax on a 64-bit
-// key (ordered float bits << 32 | ~block) so that the comparison itself
-// implements "larger value, then smaller block id".
+// Three forms (topk_row.hpp; topk_launch says which rows take which): sixteen lanes per
+// (token, group) row with its causal prefix in registers (VPL values per lane) and an iterated
+// argmax on a 64-bit key (ordered float bits << 32 | ~block), so that the comparison itself
+// implements "larger value, then smaller block id"; a wavefront per one or two rows that
+// finds a threshold and sorts the keys above it; a wavefront per row for long rows, with the
+// row in registers or streamed.
 #include "topk_row.hpp"
 
 namespace msa {
