@@ -110,9 +110,11 @@ __device__ __forceinline__ int find_seq(const int32_t* __restrict__ cu, int nseq
 // (tokens must not decrease with the lane), or search as well where that is more than a few
 // sequences (a run of empty ones: with 200 000 between two tokens the score took 63 ms, so 48).
 __device__ __forceinline__ int find_seq_near(const int32_t* __restrict__ cu, int nseq, int32_t t) {
-  int s = find_seq(cu, nseq, __builtin_amdgcn_readfirstlane(t));
-  for (int i = 0; i < 8 && s + 1 < nseq && cu[s + 1] <= t; ++i) ++s;
-  return s + 1 < nseq && cu[s + 1] <= t ? find_seq(cu, nseq, t) : s;
+  const int s0 = find_seq(cu, nseq, __builtin_amdgcn_readfirstlane(t));
+  int s = s0;
+  while (s + 1 < nseq && cu[s + 1] <= t)
+    if (++s - s0 > 8) return find_seq(cu, nseq, t);
+  return s;
 }
 
 // Largest index i in [0, n) with a[i] <= x, for nondecreasing a with a[0] <= x.
